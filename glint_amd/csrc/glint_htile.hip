@@ -17,14 +17,15 @@
  *   over 8 waves for M >= 256; k_tile_ss: 64 x 64 / 128 x 64 over 4 waves below, with the
  *   weights loaded a whole 128-B line per 8 lanes. Both are shared with the INT8-pin
  *   W8A16 GEMM.
- * k_htile_generic — every other shape (any M, K, bs, alignment): 64x32 output tiles,
- *   weights decoded to f32 in LDS per 32-wide K step, f32 FMAs in k order.
+ * k_htile_any (htile_any.h) — every other shape (any M, K, bs, alignment): unaligned rows
+ *   read from their own byte address, exact f32 weights as three BF16 planes on MFMA.
  */
 #include <algorithm>
 #include <type_traits>
 
 #include "glint_common.h"
 #include "glint_htile.h"
+#include "htile_any.h"
 #include "tile_mfma.h"
 
 /* ------------------------------------------------ GEMV with x in registers */
@@ -862,73 +863,6 @@ static int htile_launch_gemv_mr(const uint8_t *hole, const uint8_t *plug, const 
         return -3;
     kern<<<grid, threads, lds, st>>>(hole, plug, absmax, (const uint16_t *)x, y, M, N, K, G, (int)rows_per_wg);
     return hipGetLastError() == hipSuccess ? 0 : -3;
-}
-
-/* ------------------------------------------------------------ generic f32 tiles */
-#define GT_N 64
-#define GT_M 32
-#define GT_K 32
-
-__device__ __forceinline__ uint32_t glint_nibble(const uint8_t *pk, int64_t i) {
-    return (pk[i >> 1] >> ((uint32_t)(i & 1) * 4)) & 15u;
-}
-
-template <bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_htile_generic(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
-                                                       const float *__restrict__ absmax, const uint16_t *__restrict__ x,
-                                                       void *__restrict__ y, int M, int N, int K, int bs) {
-    __shared__ float ws[GT_K][GT_N + 1];
-    __shared__ float xsh[GT_K][GT_M + 1];
-    const int n0 = blockIdx.x * GT_N, m0 = blockIdx.y * GT_M;
-    const int tid = threadIdx.x;
-    const int tn = tid & 15, tm = tid >> 4; /* outputs n = n0 + tn + 16*i (i<4), m = m0 + tm + 16*j (j<2) */
-    float acc[4][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
-    for (int k0 = 0; k0 < K; k0 += GT_K) {
-        for (int e = tid; e < GT_N * GT_K; e += 256) {
-            const int r = e / GT_K, c = e % GT_K;
-            const int n = n0 + r, k = k0 + c;
-            float wv = 0.0f;
-            if (n < N && k < K) {
-                const int64_t i = (int64_t)n * K + k;
-                wv = kCells[glint_nibble(hole, i)][glint_nibble(plug, i)] * absmax[i / bs];
-            }
-            ws[c][r] = wv;
-        }
-        for (int e = tid; e < GT_M * GT_K; e += 256) {
-            const int r = e / GT_K, c = e % GT_K;
-            const int m = m0 + r, k = k0 + c;
-            xsh[c][r] = (m < M && k < K) ? __uint_as_float((uint32_t)x[(int64_t)m * K + k] << 16) : 0.0f;
-        }
-        __syncthreads();
-        const int kend = min(GT_K, K - k0);
-        for (int c = 0; c < kend; ++c) {
-            float wv[4], xv[2];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                wv[i] = ws[c][tn + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                xv[j] = xsh[c][tm + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = fmaf(wv[i], xv[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + tn + 16 * i, m = m0 + tm + 16 * j;
-            if (n < N && m < M) {
-                if (OUT_BF16)
-                    ((uint16_t *)y)[(int64_t)m * N + n] = glint_f32_to_bf16(acc[i][j]);
-                else
-                    ((float *)y)[(int64_t)m * N + n] = acc[i][j];
-            }
-        }
 }
 
 /* ---------------------------------------------------- prefill GEMM on BF16 MFMA */
@@ -1791,8 +1725,8 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
         if (!planned)
             return -5;
     } else {
-        dim3 grid((N + GT_N - 1) / GT_N, (M + GT_M - 1) / GT_M);
-        k_htile_generic<OUT_BF16><<<grid, 256, 0, st>>>(hole, plug, absmax, (const uint16_t *)x, y, M, N, K, bs);
+        return htile_any_launch<typename std::conditional<OUT_BF16, TileOutBF16, TileOutF32>::type>(
+            hole, plug, absmax, x, y, M, N, K, bs, st);
     }
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }

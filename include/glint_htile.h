@@ -17,7 +17,7 @@ struct ihipStream_t;
  * At M > 1 with blocksize 64, K % 64 == 0 and aligned pointers the products run on BF16
  * MFMA with each f32 weight split exactly into three BF16 planes (the sum differs from a
  * sequential f32 sum only in order); M = 1 is the f32 GEMV (K <= 32768; larger K takes
- * the MFMA route), other shapes a generic kernel. Enqueued on `stream`; y is overwritten
+ * the MFMA route), other shapes the same three planes from unaligned rows. Enqueued on `stream`; y is overwritten
  * (with zeros when K <= 0: the empty sum, as in the reference). Returns 0, -1 for a null
  * pointer, -2 for blocksize <= 0, -3 for a launch error; M <= 0 or N <= 0 launches nothing
  * and returns 0. The MFMA route uses the stream's split-K workspace as
