@@ -985,7 +985,7 @@ ENCODE_PIECE_CHUNKS = 1 << 17  # the library's most 512-element chunks per encod
 
 
 def encode_launches(n: int) -> int:
-    """k_encode_bf16_b64 dispatches of one BF16 bs-64 encode of n elements (n % 512 == 0):
+    """k_encode_blocks dispatches of one BF16 bs-64 encode of n elements (n % 512 == 0):
     the library launches tensors above ENCODE_PIECE_CHUNKS chunks in equal pieces."""
     return max(1, -(-(n // 512) // ENCODE_PIECE_CHUNKS))
 
@@ -1009,7 +1009,7 @@ def counter_workload(torch, H, manifest_path):
         log(f"counter workload: {name} ({count} dispatches)")
 
     def encode_pin(w):
-        launched["k_encode_bf16_b64"] = launched.get("k_encode_bf16_b64", 0) + 1
+        launched["k_encode_blocks"] = launched.get("k_encode_blocks", 0) + 1
         return H.encode_bf16(w, 64)
 
     g = torch.Generator(device="cuda").manual_seed(7001)
@@ -1024,7 +1024,7 @@ def counter_workload(torch, H, manifest_path):
     ws = [(torch.randn(N * K, device="cuda", generator=g) * 0.02).to(torch.bfloat16) for _ in range(6)]
     outs = [(torch.empty(N * K // 2, dtype=torch.uint8, device="cuda"), torch.empty(N * K // 2, dtype=torch.uint8, device="cuda"),
              torch.empty(N * K // 64, dtype=torch.float32, device="cuda")) for _ in range(6)]
-    phase("encode_14336x4096", "k_encode_bf16_b64", 6,
+    phase("encode_14336x4096", "k_encode_blocks", 6,
           lambda: [bound(lib.glint_encode_bf16_device, w, N * K, 64, *o, st)() for w, o in zip(ws, outs)],
           nbytes=6 * 3.0625 * N * K, elements=6 * N * K)
     del ws, outs
@@ -1036,7 +1036,7 @@ def counter_workload(torch, H, manifest_path):
     outs = [(torch.empty(w.numel() // 2, dtype=torch.uint8, device="cuda"),
              torch.empty(w.numel() // 2, dtype=torch.uint8, device="cuda"),
              torch.empty(w.numel() // 64, dtype=torch.float32, device="cuda")) for w in ws]
-    phase("encode_model_set", "k_encode_bf16_b64", sum(encode_launches(a * b) for a, b in shapes),
+    phase("encode_model_set", "k_encode_blocks", sum(encode_launches(a * b) for a, b in shapes),
           lambda: [bound(lib.glint_encode_bf16_device, w, w.numel(), 64, *o, st)() for w, o in zip(ws, outs)],
           nbytes=3.0625 * total, elements=total, note="226 Llama-3-8B tensors, 8.03e9 weights")
     del ws, outs

@@ -15,7 +15,13 @@
  * subtract. Other blocks (zero, tiny, huge, inf or NaN present) take the NaN-skipping
  * absmax and the IEEE divide. The nearest-code search is one LDS bucket lookup and one
  * compare (glint_codebook.h, verified against the scan for every float in [-1, 1]).
- * Everything else (any bs, F32 input, tails, unaligned pointers) runs the generic pair.
+ * Blocks of 32 and 128 and F32 input (always the IEEE divide) run the same kernel; the last
+ * partial chunk of a tensor is one more workgroup of the launch. Against the generic pair,
+ * which reads the weights twice with a wave per block and an element pair per thread:
+ * F32 14336 x 4096 251 -> 59 us (5.0 TB/s, the rate of a device copy), 1283 x 3001 19.7 -> 7.4;
+ * BF16 in blocks of 32 4096 x 4096 94 -> 12.5, of 128 63 -> 12.0; a partial last chunk as two
+ * more launches 4097 x 4099 17.0 -> 12.4. Other block sizes, unaligned pointers and tensors
+ * below one chunk run the generic pair.
  */
 #include "glint_common.h"
 #include "glint_codebook.h"
@@ -25,6 +31,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <type_traits>
 
 __constant__ GlintCodeEntry kCodeTable[GLINT_CODE_BUCKETS] = {
 #include "glint_code_table.inc"
@@ -128,28 +135,108 @@ __device__ __forceinline__ uint32_t glint_mag_max(const glint_u32x4 d) {
     return max((uint32_t)m.x, (uint32_t)m.y);
 }
 
-/* Block absmax bits with NaN skipped (glint_mag_key), reduced over the 8 lanes. */
+/* Max over the 2^LOGL lanes (4, 8 or 16) that share a block, in each of them: DPP moves inside
+ * an aligned group. */
+template <int LOGL>
+__device__ __forceinline__ int glint_block_max(int v) {
+    static_assert(LOGL >= 2 && LOGL <= 4, "a block is 4, 8 or 16 lanes");
+    v = glint_max_dpp<GLINT_DPP_QUAD_1032>(v);
+    v = glint_max_dpp<GLINT_DPP_QUAD_2301>(v);
+    if constexpr (LOGL >= 3)
+        v = glint_max_dpp<GLINT_DPP_ROW_HALF_MIRROR>(v);
+    if constexpr (LOGL >= 4)
+        v = glint_max_dpp<GLINT_DPP_ROW_MIRROR>(v);
+    return v;
+}
+
+/* Block absmax bits with NaN skipped (glint_mag_key), reduced over the block's lanes. */
+template <int LOGL>
 __device__ __forceinline__ uint32_t glint_absmax_skip_nan(const glint_u32x4 d) {
     glint_i16x2 k = __builtin_elementwise_max(glint_mag_key(d.x), glint_mag_key(d.y));
     k = __builtin_elementwise_max(k, __builtin_elementwise_max(glint_mag_key(d.z), glint_mag_key(d.w)));
-    int m16 = max(max((int)k.x, (int)k.y), 0x7F) - 0x7F;
-    m16 = glint_max_dpp<GLINT_DPP_QUAD_1032>(m16);
-    m16 = glint_max_dpp<GLINT_DPP_QUAD_2301>(m16);
-    m16 = glint_max_dpp<GLINT_DPP_ROW_HALF_MIRROR>(m16);
-    return (uint32_t)m16 << 16;
+    return (uint32_t)glint_block_max<LOGL>(max(max((int)k.x, (int)k.y), 0x7F) - 0x7F) << 16;
 }
 
-__device__ __forceinline__ void glint_encode_chunk(const glint_u32x4 d, const glint_u32x4 *tab, uint32_t lane_k,
+/* A lane's 8 f32 values against its block's absmax `sbits` by the IEEE divide: acc[h] folds
+ * elements 4 h .. 4 h + 3, hole nibble at bit 4 i and plug nibble at 16 + 4 i. */
+__device__ __forceinline__ void glint_encode_div(const float (&w)[8], uint32_t sbits, const glint_u32x4 *tab,
+                                                 uint32_t lane_k, uint32_t (&acc)[2]) {
+    const float s = __uint_as_float(sbits);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t a = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a |= glint_spread_of((s == 0.0f) ? 0.0f : w[4 * h + i] / s, tab, lane_k) << (4 * i);
+            if (i & 1)
+                __builtin_amdgcn_sched_barrier(0); /* two divides at a time: the F32 kernel has 64 registers */
+        }
+        acc[h] = a;
+    }
+}
+
+/* Largest magnitude bits of a lane's 8 f32 values, NaN skipped. */
+__device__ __forceinline__ int glint_mag_max_f32(const float (&w)[8]) {
+    int m = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int a = (int)(__float_as_uint(w[i]) & 0x7FFFFFFFu);
+        m = max(m, a > 0x7F800000 ? 0 : a);
+    }
+    return m;
+}
+
+/* What a lane holds of a 512-element chunk: elements [8 lane, 8 lane + 8). */
+template <typename T>
+struct EncLane;
+template <>
+struct EncLane<uint16_t> {
+    glint_u32x4 d;
+    __device__ __forceinline__ void load(const uint16_t *w, int64_t chunk, int lane) {
+        d = __builtin_nontemporal_load((const glint_u32x4 *)w + chunk * 64 + lane);
+    }
+};
+template <>
+struct EncLane<float> {
+    glint_f32x4 d[2];
+    __device__ __forceinline__ void load(const float *w, int64_t chunk, int lane) {
+        const glint_f32x4 *p = (const glint_f32x4 *)w + (chunk * 64 + lane) * 2;
+        d[0] = p[0]; /* default policy: the two loads share the lane pair's lines */
+        d[1] = p[1];
+    }
+};
+
+template <int LOGL>
+__device__ __forceinline__ void glint_encode_store(const uint32_t (&acc)[2], uint32_t sbits, int64_t chunk, int lane,
+                                                   uint32_t *__restrict__ hole, uint32_t *__restrict__ plug,
+                                                   float *__restrict__ absmax) {
+    hole[chunk * 64 + lane] = __builtin_amdgcn_perm(acc[1], acc[0], 0x05040100u);
+    plug[chunk * 64 + lane] = __builtin_amdgcn_perm(acc[1], acc[0], 0x07060302u);
+    if ((lane & ((1 << LOGL) - 1)) == 0)
+        absmax[chunk * (64 >> LOGL) + (lane >> LOGL)] = __uint_as_float(sbits);
+}
+
+/* F32 input: an f32 quotient pair has no short exact form as the BF16 ones do, and with 5
+ * bytes an element the divide hides behind the stream. */
+template <int LOGL>
+__device__ __forceinline__ void glint_encode_chunk(const EncLane<float> &d, const glint_u32x4 *tab, uint32_t lane_k,
+                                                   uint32_t, int64_t chunk, int lane, uint32_t *__restrict__ hole,
+                                                   uint32_t *__restrict__ plug, float *__restrict__ absmax) {
+    const float w[8] = {d.d[0].x, d.d[0].y, d.d[0].z, d.d[0].w, d.d[1].x, d.d[1].y, d.d[1].z, d.d[1].w};
+    const uint32_t sbits = (uint32_t)glint_block_max<LOGL>(glint_mag_max_f32(w));
+    uint32_t acc[2];
+    glint_encode_div(w, sbits, tab, lane_k, acc);
+    glint_encode_store<LOGL>(acc, sbits, chunk, lane, hole, plug, absmax);
+}
+
+template <int LOGL>
+__device__ __forceinline__ void glint_encode_chunk(const EncLane<uint16_t> &dl, const glint_u32x4 *tab, uint32_t lane_k,
                                                    uint32_t lane_r, int64_t chunk, int lane,
                                                    uint32_t *__restrict__ hole, uint32_t *__restrict__ plug,
                                                    float *__restrict__ absmax) {
-    /* magnitude max of this lane's 8 values, then of the 8 lanes that share the block (the
-     * DPP moves stay inside each aligned group of 8 lanes) */
-    int m16 = (int)glint_mag_max(d);
-    m16 = glint_max_dpp<GLINT_DPP_QUAD_1032>(m16);
-    m16 = glint_max_dpp<GLINT_DPP_QUAD_2301>(m16);
-    m16 = glint_max_dpp<GLINT_DPP_ROW_HALF_MIRROR>(m16);
-    uint32_t sbits = (uint32_t)m16 << 16;
+    const glint_u32x4 d = dl.d;
+    /* magnitude max of this lane's 8 values, then of the lanes that share the block */
+    uint32_t sbits = (uint32_t)glint_block_max<LOGL>((int)glint_mag_max(d)) << 16;
 
     const uint32_t dw[4] = {d.x, d.y, d.z, d.w};
     float w[8];
@@ -174,32 +261,65 @@ __device__ __forceinline__ void glint_encode_chunk(const glint_u32x4 d, const gl
             acc[h] = a;
         }
     } else {
-        sbits = glint_absmax_skip_nan(d);
-        const float s = __uint_as_float(sbits);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t a = 0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                a |= glint_spread_of((s == 0.0f) ? 0.0f : w[4 * h + i] / s, tab, lane_k) << (4 * i);
-            acc[h] = a;
-        }
+        sbits = glint_absmax_skip_nan<LOGL>(d);
+        glint_encode_div(w, sbits, tab, lane_k, acc);
     }
-    hole[chunk * 64 + lane] = __builtin_amdgcn_perm(acc[1], acc[0], 0x05040100u);
-    plug[chunk * 64 + lane] = __builtin_amdgcn_perm(acc[1], acc[0], 0x07060302u);
-    if ((lane & 7) == 0)
-        absmax[chunk * 8 + (lane >> 3)] = __uint_as_float(sbits);
+    glint_encode_store<LOGL>(acc, sbits, chunk, lane, hole, plug, absmax);
+}
+
+__device__ __forceinline__ float glint_load_w(const uint16_t *w, int64_t i) { return __uint_as_float((uint32_t)w[i] << 16); }
+__device__ __forceinline__ float glint_load_w(const float *w, int64_t i) { return w[i]; }
+
+/* The rem < 512 elements behind the last whole chunk, by one wave: element loads and byte
+ * stores only of what exists, the IEEE divide, a pad nibble of 0. */
+template <typename T, int LOGL>
+__device__ __forceinline__ void glint_encode_tail(const T *__restrict__ w, int rem, const glint_u32x4 *tab,
+                                                  uint32_t lane_k, int64_t chunk, int lane, uint8_t *__restrict__ hole,
+                                                  uint8_t *__restrict__ plug, float *__restrict__ absmax) {
+    const int mine = min(max(rem - 8 * lane, 0), 8);
+    const T *wl = w + chunk * 512 + 8 * lane;
+    int m = 0;
+#pragma unroll 1
+    for (int i = 0; i < mine; ++i) {
+        const int a = (int)(__float_as_uint(glint_load_w(wl, i)) & 0x7FFFFFFFu);
+        m = max(m, a > 0x7F800000 ? 0 : a);
+    }
+    const uint32_t sbits = (uint32_t)glint_block_max<LOGL>(m);
+    const float s = __uint_as_float(sbits);
+    uint32_t acc[2] = {0u, 0u};
+#pragma unroll 1
+    for (int i = 0; i < mine; ++i) {
+        const uint32_t c = glint_spread_of((s == 0.0f) ? 0.0f : glint_load_w(wl, i) / s, tab, lane_k) << (4 * (i & 3));
+        acc[0] |= i < 4 ? c : 0u;
+        acc[1] |= i < 4 ? 0u : c;
+    }
+    const uint32_t keep = mine == 8 ? 0xFFFFFFFFu : (1u << (4 * mine)) - 1u; /* nibbles that exist */
+    const uint32_t h = __builtin_amdgcn_perm(acc[1], acc[0], 0x05040100u) & keep;
+    const uint32_t p = __builtin_amdgcn_perm(acc[1], acc[0], 0x07060302u) & keep;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (2 * i < mine) {
+            hole[chunk * 256 + lane * 4 + i] = (uint8_t)(h >> (8 * i));
+            plug[chunk * 256 + lane * 4 + i] = (uint8_t)(p >> (8 * i));
+        }
+    if ((lane & ((1 << LOGL) - 1)) == 0 && mine > 0)
+        absmax[chunk * (64 >> LOGL) + (lane >> LOGL)] = __uint_as_float(sbits);
 }
 
 /* One wave handles groups of ENC_UNROLL consecutive chunks: groups wave, wave + nwaves, ...
  * two groups in flight (register double buffer, unconditional clamped loads, full rounds
  * so the wait counter can count them); the table fill's loads go out first and its LDS
  * writes after the first two groups' loads. Chunks past the last full group are spread
- * one per wave at the end. */
-__global__ __launch_bounds__(ENC_THREADS, ENC_WPE) void k_encode_bf16_b64(const glint_u32x4 *__restrict__ w,
-                                                                 uint32_t *__restrict__ hole,
-                                                                 uint32_t *__restrict__ plug,
-                                                                 float *__restrict__ absmax, int64_t nchunks) {
+ * one per wave at the end.
+ * LOGL: log2 of the lanes per block (32, 64 or 128 elements: 2, 3 or 4). TAIL: one more
+ * workgroup, for the rem elements behind the last chunk (as one more chunk of a wave they took
+ * registers from the loop: 1024 x 4096 BF16 6.08 -> 6.16 us, the F32 kernel spilled). */
+template <typename T, int LOGL, bool TAIL>
+__global__ __launch_bounds__(ENC_THREADS, sizeof(T) == 4 ? 8 : ENC_WPE) void k_encode_blocks(const T *__restrict__ w,
+                                                                        uint32_t *__restrict__ hole,
+                                                                        uint32_t *__restrict__ plug,
+                                                                        float *__restrict__ absmax, int64_t nchunks,
+                                                                        int rem) {
     __shared__ __attribute__((aligned(16))) glint_u32x4 tab[GLINT_CODE_BUCKETS * ENC_COPIES];
     const int lane = threadIdx.x & 63;
     /* bucket * ENC_COPIES * 16 + lane_k == byte offset of entry (bucket, lane % ENC_COPIES):
@@ -210,7 +330,7 @@ __global__ __launch_bounds__(ENC_THREADS, ENC_WPE) void k_encode_bf16_b64(const 
     const uint32_t lane_r = (uint32_t)(lane % ENC_COPIES) * 16u + 12u; /* word 3 of this lane's copy */
     /* wave-uniform, so group arithmetic stays in scalar registers */
     const int wave = (int)blockIdx.x * (ENC_THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nwaves = (int)gridDim.x * (ENC_THREADS / 64);
+    const int nwaves = ((int)gridDim.x - (TAIL ? 1 : 0)) * (ENC_THREADS / 64);
     const int ngroups = (int)(nchunks / ENC_UNROLL);
     const int my = wave < ngroups ? (ngroups - wave + nwaves - 1) / nwaves : 0; /* groups wave + i nwaves */
     const int last = max(ngroups - 1, 0);
@@ -227,15 +347,15 @@ __global__ __launch_bounds__(ENC_THREADS, ENC_WPE) void k_encode_bf16_b64(const 
     /* unconditional loads (a branch here would make every later wait count the worst
      * path); chunk indices are clamped to the last chunk for the case of no full group */
     const int64_t lastc = nchunks - 1;
-    glint_u32x4 da[ENC_UNROLL], db[ENC_UNROLL];
+    EncLane<T> da[ENC_UNROLL], db[ENC_UNROLL];
     {
         const int64_t ga = (int64_t)min(wave, last) * ENC_UNROLL, gb = (int64_t)min(wave + nwaves, last) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            da[u] = __builtin_nontemporal_load(&w[min(ga + u, lastc) * 64 + lane]);
+            da[u].load(w, min(ga + u, lastc), lane);
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            db[u] = __builtin_nontemporal_load(&w[min(gb + u, lastc) * 64 + lane]);
+            db[u].load(w, min(gb + u, lastc), lane);
     }
 #pragma unroll
     for (int k = 0; k < kFill; ++k) /* clamped indices rewrite the last entry with its own value */
@@ -243,48 +363,52 @@ __global__ __launch_bounds__(ENC_THREADS, ENC_WPE) void k_encode_bf16_b64(const 
     for (int e = threadIdx.x + kFill * blockDim.x; e < kEntries; e += blockDim.x) /* blockDim < 1024 only */
         tab[e] = glint_code_lds_entry(kCodeTable[e / ENC_COPIES], e / ENC_COPIES);
     __syncthreads();
+    if (TAIL && blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < 64)
+            glint_encode_tail<T, LOGL>(w, rem, tab, lane_k, nchunks, lane, (uint8_t *)hole, (uint8_t *)plug, absmax);
+        return;
+    }
 
     int i = 0;
     for (; i + 2 <= my; i += 2) {
         const int64_t c0 = (int64_t)(wave + i * nwaves) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            glint_encode_chunk(da[u], tab, lane_k, lane_r, c0 + u, lane, hole, plug, absmax);
+            glint_encode_chunk<LOGL>(da[u], tab, lane_k, lane_r, c0 + u, lane, hole, plug, absmax);
         const int64_t ga = (int64_t)min(wave + (i + 2) * nwaves, last) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            da[u] = __builtin_nontemporal_load(&w[(ga + u) * 64 + lane]);
+            da[u].load(w, ga + u, lane);
         const int64_t c1 = (int64_t)(wave + (i + 1) * nwaves) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            glint_encode_chunk(db[u], tab, lane_k, lane_r, c1 + u, lane, hole, plug, absmax);
+            glint_encode_chunk<LOGL>(db[u], tab, lane_k, lane_r, c1 + u, lane, hole, plug, absmax);
         const int64_t gb = (int64_t)min(wave + (i + 3) * nwaves, last) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            db[u] = __builtin_nontemporal_load(&w[(gb + u) * 64 + lane]);
+            db[u].load(w, gb + u, lane);
     }
     if (i < my) {
         const int64_t c0 = (int64_t)(wave + i * nwaves) * ENC_UNROLL;
 #pragma unroll
         for (int u = 0; u < ENC_UNROLL; ++u)
-            glint_encode_chunk(da[u], tab, lane_k, lane_r, c0 + u, lane, hole, plug, absmax);
+            glint_encode_chunk<LOGL>(da[u], tab, lane_k, lane_r, c0 + u, lane, hole, plug, absmax);
     }
     const int64_t c = (int64_t)ngroups * ENC_UNROLL + wave; /* at most ENC_UNROLL - 1 leftover chunks */
-    if (c < nchunks)
-        glint_encode_chunk(w[c * 64 + lane], tab, lane_k, lane_r, c, lane, hole, plug, absmax);
+    if (c < nchunks) {
+        da[0].load(w, c, lane);
+        glint_encode_chunk<LOGL>(da[0], tab, lane_k, lane_r, c, lane, hole, plug, absmax);
+    }
 }
 
 /* ---------------------------------------------------------------- generic encode */
-__device__ __forceinline__ float glint_load_w(const uint16_t *w, int64_t i) { return __uint_as_float((uint32_t)w[i] << 16); }
-__device__ __forceinline__ float glint_load_w(const float *w, int64_t i) { return w[i]; }
-
-/* absmax of blocks [b0, b1): one wave per block, NaN skipped (fabsf(NaN) > m is false). */
+/* absmax of the nb blocks: one wave per block, NaN skipped (fabsf(NaN) > m is false). */
 template <typename T>
-__global__ __launch_bounds__(256) void k_absmax_generic(const T *__restrict__ w, int64_t n, int bs, int64_t b0,
-                                                        int64_t b1, float *__restrict__ absmax) {
+__global__ __launch_bounds__(256) void k_absmax_generic(const T *__restrict__ w, int64_t n, int bs, int64_t nb,
+                                                        float *__restrict__ absmax) {
     const int lane = threadIdx.x & 63;
     const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
-    for (int64_t b = b0 + (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); b < b1; b += nwaves) {
+    for (int64_t b = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); b < nb; b += nwaves) {
         const int64_t i0 = b * bs;
         const int64_t i1 = min(i0 + bs, n);
         float m = 0.0f;
@@ -299,13 +423,13 @@ __global__ __launch_bounds__(256) void k_absmax_generic(const T *__restrict__ w,
     }
 }
 
-/* packed bytes [e0, e1): v = (s == 0) ? 0 : w / s (IEEE divide), code lookup, pack. */
+/* the npk packed bytes: v = (s == 0) ? 0 : w / s (IEEE divide), code lookup, pack. */
 template <typename T>
 __global__ __launch_bounds__(256) void k_encode_generic(const T *__restrict__ w, const float *__restrict__ absmax,
-                                                        int64_t n, int bs, int64_t e0, int64_t e1,
+                                                        int64_t n, int bs, int64_t npk,
                                                         uint8_t *__restrict__ hole, uint8_t *__restrict__ plug) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t e = e0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < e1; e += stride) {
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < npk; e += stride) {
         uint32_t c[2] = {0u, 0u};
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -352,35 +476,37 @@ static int encode_device(const T *d_w, int64_t n, int bs, uint8_t *d_hole, uint8
     if (!d_w || !d_hole || !d_plug || !d_am)
         return -1;
     const int cus = glint_num_cus();
-    int64_t n_fast = 0;
-    if (sizeof(T) == 2 && bs == 64 && glint_aligned(d_w, 16) && glint_aligned(d_hole, 4) && glint_aligned(d_plug, 4) &&
-        glint_aligned(d_am, 4))
-        n_fast = (n / 512) * 512;
-    if (n_fast) {
-        const int64_t nchunks = n_fast / 512;
+    if ((bs == 32 || bs == 64 || bs == 128) && n >= 512 && glint_aligned(d_w, 16) && glint_aligned(d_hole, 4) &&
+        glint_aligned(d_plug, 4) && glint_aligned(d_am, 4)) {
+        auto pick = [&](auto tail) {
+            constexpr bool R = decltype(tail)::value;
+            return bs == 64 ? k_encode_blocks<T, 3, R> : (bs == 32 ? k_encode_blocks<T, 2, R> : k_encode_blocks<T, 4, R>);
+        };
+        const auto whole = pick(std::false_type{}), tail = pick(std::true_type{});
+        const int64_t nchunks = n / 512;
         /* Tensors above ENC_PIECE_CHUNKS chunks go as equal consecutive pieces, one launch
          * each on the stream (the bytes are the same): one launch over the 525 M-element
          * embedding ran at 57-59% of HBM, eight pieces of 66 M elements at 62-64% (16 pieces
          * 59%); the Llama-3-8B set on 4 streams 62.0 -> 63.5%. */
         const int64_t pieces = (nchunks + ENC_PIECE_CHUNKS - 1) / ENC_PIECE_CHUNKS;
         const int64_t per = (nchunks + pieces - 1) / pieces;
-        const int resident = (int)glint_resident_grid((const void *)k_encode_bf16_b64, ENC_THREADS, 0);
+        const int resident = (int)glint_resident_grid((const void *)whole, ENC_THREADS, 0);
         for (int64_t c0 = 0; c0 < nchunks; c0 += per) {
             const int64_t nc = std::min(per, nchunks - c0);
-            /* a group per wave while there are enough groups, at most the resident blocks;
-             * the leftover chunks (< ENC_UNROLL) need fewer waves than one block has */
-            const unsigned grid = glint_grid(nc, (ENC_THREADS / 64) * ENC_UNROLL, resident);
-            k_encode_bf16_b64<<<grid, ENC_THREADS, 0, st>>>((const glint_u32x4 *)d_w + c0 * 64,
-                                                            (uint32_t *)d_hole + c0 * 64, (uint32_t *)d_plug + c0 * 64,
-                                                            d_am + c0 * 8, nc);
+            const int rem = c0 + nc == nchunks ? (int)(n % 512) : 0;
+            /* a group per wave while there are enough groups, at most the resident blocks (the
+             * tail's workgroup among them: as one more generation it cost 0.8 us); the leftover
+             * chunks (< ENC_UNROLL) need fewer waves than one block has */
+            const unsigned grid =
+                glint_grid(nc, (ENC_THREADS / 64) * ENC_UNROLL, std::max(1, rem ? resident - 1 : resident));
+            (rem ? tail : whole)<<<grid + (rem ? 1 : 0), ENC_THREADS, 0, st>>>(d_w + c0 * 512, (uint32_t *)d_hole + c0 * 64,
+                                                               (uint32_t *)d_plug + c0 * 64, d_am + c0 * (512 / bs), nc,
+                                                               rem);
         }
-    }
-    if (n_fast < n) {
-        const int64_t b0 = n_fast / bs, b1 = (n + bs - 1) / bs;
-        k_absmax_generic<T><<<glint_grid(b1 - b0, 4, cus * 16), 256, 0, st>>>(d_w, n, bs, b0, b1, d_am);
-        const int64_t e0 = n_fast / 2, e1 = (n + 1) / 2;
-        k_encode_generic<T><<<glint_grid(e1 - e0, 256, cus * 16), 256, 0, st>>>(d_w, d_am, n, bs, e0, e1, d_hole,
-                                                                                 d_plug);
+    } else {
+        const int64_t nb = (n + bs - 1) / bs, npk = (n + 1) / 2;
+        k_absmax_generic<T><<<glint_grid(nb, 4, cus * 16), 256, 0, st>>>(d_w, n, bs, nb, d_am);
+        k_encode_generic<T><<<glint_grid(npk, 256, cus * 16), 256, 0, st>>>(d_w, d_am, n, bs, npk, d_hole, d_plug);
     }
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
@@ -497,7 +623,7 @@ __global__ __launch_bounds__(256) void k_expand_generic(const uint8_t *__restric
     }
 }
 
-/* Run-mapped expand (power-of-two bs >= 8, n % 2048 == 0 part): a wave chunk is 256 runs of
+/* Run-mapped expand (power-of-two bs >= 8, n >= 2048): a wave chunk is 256 runs of
  * 8 elements; lane l owns runs 64 s + l (s < 4), i.e. one dword of each plane per run, so
  * every plane load of a wave reads 256 B contiguous and every BF16 store writes 1 KiB
  * contiguous (f32: two 16-B stores, 2 KiB). Chunks are double-buffered in registers with
@@ -512,23 +638,27 @@ __global__ __launch_bounds__(256) void k_expand_generic(const uint8_t *__restric
 #define EXPANDR_HWCVT 1 /* BF16 by v_cvt_pk_bf16_f32 (RNE); NaN absmax takes the scalar rule */
 #endif
 
+template <bool BF16>
 struct ExpandChunk {
-    uint32_t h[4], p[4];
-    float a[4];
+    static constexpr int S = BF16 ? 4 : 8; /* steps of 64 runs of 8 (BF16) or of 64 half runs of 4 (f32) */
+    uint32_t h[S], p[S];
+    float a[S];
 };
 
 /* Loads of wave chunk c: runs c*256 + 64 s + lane. `abase` = c * (2048 >> shift) is the
  * chunk's first absmax index (bs <= 2048, so a chunk starts on a block boundary). */
+template <bool BF16>
 __device__ __forceinline__ void expand_load_chunk(const uint32_t *__restrict__ hole, const uint32_t *__restrict__ plug,
                                                   const float *__restrict__ absmax, int64_t c, int lane, int shift,
-                                                  ExpandChunk &ck) {
+                                                  ExpandChunk<BF16> &ck) {
     const uint32_t *h = hole + c * 256, *p = plug + c * 256;
     const float *a = absmax + (c << (11 - shift));
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        ck.h[s] = __builtin_nontemporal_load(h + s * 64 + lane);
-        ck.p[s] = __builtin_nontemporal_load(p + s * 64 + lane);
-        ck.a[s] = a[(uint32_t)(s * 512 + lane * 8) >> shift];
+    for (int s = 0; s < ExpandChunk<BF16>::S; ++s) {
+        const int run = BF16 ? s * 64 + lane : s * 32 + (lane >> 1);
+        ck.h[s] = __builtin_nontemporal_load(h + run);
+        ck.p[s] = __builtin_nontemporal_load(p + run);
+        ck.a[s] = a[(uint32_t)(run * 8) >> shift];
     }
 }
 
@@ -542,9 +672,8 @@ __device__ __forceinline__ uint32_t expand_pack2(float lo, float hi) {
 #endif
 }
 
-template <bool BF16>
-__device__ __forceinline__ void expand_chunk(const float *ltab, uint32_t lane4, const ExpandChunk &ck, void *__restrict__ out,
-                                             int64_t c, int lane) {
+__device__ __forceinline__ void expand_chunk(const float *ltab, uint32_t lane4, const ExpandChunk<true> &ck,
+                                             void *__restrict__ out, int64_t c, int lane) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const uint32_t E = glint_codes_even(ck.h[s], ck.p[s]);
@@ -559,24 +688,35 @@ __device__ __forceinline__ void expand_chunk(const float *ltab, uint32_t lane4, 
         r[5] = glint_lds_f32(ltab, glint_cell_addr<2>(O, lane4)) * a;
         r[6] = glint_lds_f32(ltab, glint_cell_addr<3>(E, lane4)) * a;
         r[7] = glint_lds_f32(ltab, glint_cell_addr<3>(O, lane4)) * a;
-        const int64_t run = c * 256 + s * 64 + lane;
-        if (BF16) {
-            glint_u32x4 v;
-            if (a == a) {
-                v = glint_u32x4{expand_pack2(r[0], r[1]), expand_pack2(r[2], r[3]), expand_pack2(r[4], r[5]),
-                                expand_pack2(r[6], r[7])};
-            } else { /* NaN absmax: the reference NaN rule for every element */
-                v = glint_u32x4{(uint32_t)glint_f32_to_bf16(r[0]) | (uint32_t)glint_f32_to_bf16(r[1]) << 16,
-                                (uint32_t)glint_f32_to_bf16(r[2]) | (uint32_t)glint_f32_to_bf16(r[3]) << 16,
-                                (uint32_t)glint_f32_to_bf16(r[4]) | (uint32_t)glint_f32_to_bf16(r[5]) << 16,
-                                (uint32_t)glint_f32_to_bf16(r[6]) | (uint32_t)glint_f32_to_bf16(r[7]) << 16};
-            }
-            ((glint_u32x4 *)out)[run] = v;
-        } else {
-            ((glint_f32x4 *)out)[2 * run] = glint_f32x4{r[0], r[1], r[2], r[3]};
-            ((glint_f32x4 *)out)[2 * run + 1] = glint_f32x4{r[4], r[5], r[6], r[7]};
+        glint_u32x4 v;
+        if (a == a) {
+            v = glint_u32x4{expand_pack2(r[0], r[1]), expand_pack2(r[2], r[3]), expand_pack2(r[4], r[5]),
+                            expand_pack2(r[6], r[7])};
+        } else { /* NaN absmax: the reference NaN rule for every element */
+            v = glint_u32x4{(uint32_t)glint_f32_to_bf16(r[0]) | (uint32_t)glint_f32_to_bf16(r[1]) << 16,
+                            (uint32_t)glint_f32_to_bf16(r[2]) | (uint32_t)glint_f32_to_bf16(r[3]) << 16,
+                            (uint32_t)glint_f32_to_bf16(r[4]) | (uint32_t)glint_f32_to_bf16(r[5]) << 16,
+                            (uint32_t)glint_f32_to_bf16(r[6]) | (uint32_t)glint_f32_to_bf16(r[7]) << 16};
         }
+        ((glint_u32x4 *)out)[c * 256 + s * 64 + lane] = v;
         __builtin_amdgcn_sched_barrier(0);
+    }
+}
+/* f32 out: lanes 2 j and 2 j + 1 load the same run and take its lower and upper 4 elements, so
+ * a store instruction writes 1 KiB of consecutive bytes, as the BF16 form's do. */
+__device__ __forceinline__ void expand_chunk(const float *ltab, uint32_t lane4, const ExpandChunk<false> &ck,
+                                             void *__restrict__ out, int64_t c, int lane) {
+    const uint32_t half = (uint32_t)(lane & 1) * 16u;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const uint32_t H = ck.h[s] >> half, P = ck.p[s] >> half;
+        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+        const float a = ck.a[s];
+        ((glint_f32x4 *)out)[c * 512 + s * 64 + lane] =
+            glint_f32x4{glint_lds_f32(ltab, glint_cell_addr<0>(E, lane4)) * a, glint_lds_f32(ltab, glint_cell_addr<0>(O, lane4)) * a,
+                        glint_lds_f32(ltab, glint_cell_addr<1>(E, lane4)) * a, glint_lds_f32(ltab, glint_cell_addr<1>(O, lane4)) * a};
+        if (s & 1)
+            __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -584,7 +724,8 @@ template <bool BF16>
 __global__ __launch_bounds__(EXPANDR_THREADS) void k_expand_runs(const uint32_t *__restrict__ hole,
                                                                  const uint32_t *__restrict__ plug,
                                                                  const float *__restrict__ absmax,
-                                                                 void *__restrict__ out, int64_t nchunks, int shift) {
+                                                                 void *__restrict__ out, int64_t nchunks, int shift,
+                                                                 int rem) {
     __shared__ __attribute__((aligned(16))) float ltab[GLINT_LDS_CELLS64_WORDS];
     const int lane = threadIdx.x & 63;
     const uint32_t lane4 = (uint32_t)lane * 4u;
@@ -596,20 +737,32 @@ __global__ __launch_bounds__(EXPANDR_THREADS) void k_expand_runs(const uint32_t 
     const int last = nch - 1;
     GlintCellFill fill;
     glint_cells_fill_load(fill);
-    ExpandChunk ca, cb;
-    expand_load_chunk(hole, plug, absmax, min(wave, last), lane, shift, ca);
-    expand_load_chunk(hole, plug, absmax, min(wave + nwaves, last), lane, shift, cb);
+    ExpandChunk<BF16> ca, cb;
+    expand_load_chunk<BF16>(hole, plug, absmax, min(wave, last), lane, shift, ca);
+    expand_load_chunk<BF16>(hole, plug, absmax, min(wave + nwaves, last), lane, shift, cb);
     glint_cells_fill_store(ltab, fill);
     __syncthreads();
     int i = 0;
     for (; i + 2 <= my; i += 2) {
-        expand_chunk<BF16>(ltab, lane4, ca, out, wave + i * nwaves, lane);
-        expand_load_chunk(hole, plug, absmax, min(wave + (i + 2) * nwaves, last), lane, shift, ca);
-        expand_chunk<BF16>(ltab, lane4, cb, out, wave + (i + 1) * nwaves, lane);
-        expand_load_chunk(hole, plug, absmax, min(wave + (i + 3) * nwaves, last), lane, shift, cb);
+        expand_chunk(ltab, lane4, ca, out, wave + i * nwaves, lane);
+        expand_load_chunk<BF16>(hole, plug, absmax, min(wave + (i + 2) * nwaves, last), lane, shift, ca);
+        expand_chunk(ltab, lane4, cb, out, wave + (i + 1) * nwaves, lane);
+        expand_load_chunk<BF16>(hole, plug, absmax, min(wave + (i + 3) * nwaves, last), lane, shift, cb);
     }
     if (i < my)
-        expand_chunk<BF16>(ltab, lane4, ca, out, (int64_t)wave + (int64_t)i * nwaves, lane);
+        expand_chunk(ltab, lane4, ca, out, (int64_t)wave + (int64_t)i * nwaves, lane);
+    /* the rem < 2048 elements behind the last chunk, one at a time by the last workgroup */
+    if (rem > 0 && blockIdx.x == gridDim.x - 1)
+        for (int t = threadIdx.x; t < rem; t += EXPANDR_THREADS) {
+            const int64_t e = nchunks * 2048 + t;
+            const uint32_t sh = (uint32_t)(e & 1) * 4u;
+            const uint32_t h = (((const uint8_t *)hole)[e >> 1] >> sh) & 15u, p = (((const uint8_t *)plug)[e >> 1] >> sh) & 15u;
+            const float r = ltab[((h << 4 | p) << 6) | (uint32_t)lane] * absmax[e >> shift];
+            if (BF16)
+                ((uint16_t *)out)[e] = glint_f32_to_bf16(r);
+            else
+                ((float *)out)[e] = r;
+        }
 }
 
 template <bool BF16>
@@ -624,15 +777,15 @@ static int expand_device(const uint8_t *d_hole, const uint8_t *d_plug, const flo
     const bool aligned = glint_aligned(d_hole, 16) && glint_aligned(d_plug, 16) && glint_aligned(d_am, 4) &&
                          glint_aligned(d_out, 16);
     if (aligned && bs >= 8 && bs <= 2048 && (bs & (bs - 1)) == 0 && n >= 2048 && n / 2048 < (1LL << 30)) {
-        n_fast = (n / 2048) * 2048;
-        const int64_t nchunks = n_fast / 2048;
+        const int64_t nchunks = n / 2048;
         const int64_t resident = std::max<int64_t>(1, glint_resident_grid((const void *)k_expand_runs<BF16>, EXPANDR_THREADS, 0) / EXPANDR_GRID_DIV);
         const int64_t wanted = (nchunks + EXPANDR_THREADS / 64 - 1) / (EXPANDR_THREADS / 64);
         const unsigned grid = (unsigned)(wanted < resident ? wanted : resident);
         /* one launch: split into pieces as the encode is, the 525 M-element embedding
          * expanded at 59% of HBM against 62% whole */
         k_expand_runs<BF16><<<grid, EXPANDR_THREADS, 0, st>>>((const uint32_t *)d_hole, (const uint32_t *)d_plug, d_am,
-                                                               d_out, nchunks, __builtin_ctz((unsigned)bs));
+                                                               d_out, nchunks, __builtin_ctz((unsigned)bs), (int)(n % 2048));
+        n_fast = n;
     } else if (aligned && bs % 32 == 0 && n >= 32) { /* ngroups >= 1: the kernel clamps to ngroups - 1 */
         n_fast = (n / 32) * 32;
         const int64_t ngroups = n_fast / 32;
