@@ -83,7 +83,7 @@ static_assert(ENC_COPIES >= 1 && ENC_COPIES <= 64 && (ENC_COPIES & (ENC_COPIES -
 #define ENC_WPE 4
 #endif
 #ifndef ENC_PIECE_CHUNKS
-#define ENC_PIECE_CHUNKS (1 << 17) /* most 512-element chunks per k_encode_bf16_b64 launch (67 M elements) */
+#define ENC_PIECE_CHUNKS (1 << 17) /* most 512-element chunks per k_encode_blocks launch (67 M elements) */
 #endif
 
 __device__ __forceinline__ uint32_t glint_spread_code(uint32_t c) { return (c >> 4) | ((c & 15u) << 16); }

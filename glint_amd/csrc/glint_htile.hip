@@ -761,7 +761,12 @@ __global__ __launch_bounds__(MAXT) void k_htile_gemv_mr(const void *__restrict__
 #define GEMV_MR_RL 4 /* BF16 out: above this many rows k_htile_rl goes first where it takes the shape */
 #endif
 #ifndef GEMV_MR_RL_F32
-#define GEMV_MR_RL_F32 6 /* f32 out: above this many rows k_htile_rl goes first where it takes the shape */
+#define GEMV_MR_RL_F32 4 /* f32 out: above this many rows k_htile_rl3 goes first where it takes the shape */
+#endif
+#ifndef GEMV_MR_RL_F32_WEIGHTS
+/* f32 out, M = 5 and 6: fewer weights than this take the two small-M launches (1024 x 4096 M = 5
+ * 8.8 us against 9.2; 4096 x 4096 12.9 against 10.1). M = 7 and 8 always took k_htile_rl's form. */
+#define GEMV_MR_RL_F32_WEIGHTS (1 << 23)
 #endif
 #ifndef GEMV_MR_MAX_F32
 #define GEMV_MR_MAX_F32 4 /* largest M of the f32-out small-M GEMV (x as f32: MR x 32 registers) */
@@ -1248,17 +1253,10 @@ __global__ __launch_bounds__(64 * RD_STRIPS * KW, 1) void k_htile_rd(const uint8
 #define RL_STAGES 4 /* k_htile_rl: W line register stages (6: M = 64 gate 29.5 -> 30.2 us, 8: 31.1; the
                      * prologue's longer first load burst costs more than the deeper lead gains) */
 #endif
-#ifndef RD_FL_F32
-#define RD_FL_F32 1 /* f32 out at M <= 64: k_htile_rl's three-plane form (0: the f32 tiles) */
-#endif
-/* F32: f32 out (the reference ABI) with the weights w = CELLS * absmax split into three exact
- * BF16 planes (GlintTileProducer::finish_split's rule), each multiplied by x in the MFMA: the
- * products are exact and only the f32 sums differ from a scalar loop's. A step dequantizes
- * and multiplies one MFMA step at a time (3 B operands, 3 MB MFMAs). */
-template <int MB, bool F32 = false>
+template <int MB>
 __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
                                                      const float *__restrict__ absmax, const uint16_t *__restrict__ x,
-                                                     typename std::conditional<F32, float, uint16_t>::type *__restrict__ y,
+                                                     uint16_t *__restrict__ y,
                                                      int M, int N, int K, int R, int cps, float *__restrict__ part,
                                                      unsigned *ctr) {
     constexpr int KW = 2, T = 512, STRIPS = 4;
@@ -1389,60 +1387,6 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
                 acc[mb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[s & 1][mb], bq[s], acc[mb][0], 0, 0, 0);
         }
     };
-    /* F32: MFMA step s's 8 weights of this lane as three BF16 planes (hi, mid, lo: w == hi + mid
-     * + lo exactly; an infinite w keeps mid = lo = 0, a NaN w stays NaN in hi) */
-    auto split3 = [&](const WLine &s, float a, int q, glint_bf16x8 (&bp)[3]) {
-        const uint32_t E = glint_codes_even(s.h[q], s.p[q]), O = glint_codes_odd(s.h[q], s.p[q]);
-        float v[8];
-        v[0] = glint_lds_f32(ltab, glint_cell_addr<0>(E, lane4));
-        v[1] = glint_lds_f32(ltab, glint_cell_addr<0>(O, lane4));
-        v[2] = glint_lds_f32(ltab, glint_cell_addr<1>(E, lane4));
-        v[3] = glint_lds_f32(ltab, glint_cell_addr<1>(O, lane4));
-        v[4] = glint_lds_f32(ltab, glint_cell_addr<2>(E, lane4));
-        v[5] = glint_lds_f32(ltab, glint_cell_addr<2>(O, lane4));
-        v[6] = glint_lds_f32(ltab, glint_cell_addr<3>(E, lane4));
-        v[7] = glint_lds_f32(ltab, glint_cell_addr<3>(O, lane4));
-        const bool big = !(__builtin_fabsf(a) < 0x1p126f); /* only there can w be infinite */
-        uint32_t hi[8], mid[8], lo[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float w = v[i] * a;
-            const float h = __uint_as_float(__float_as_uint(w) & 0xFFFF0000u);
-            float r1 = w - h;
-            if (big)
-                r1 = __builtin_isinf(w) ? 0.0f : r1;
-            const float md = __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
-            hi[i] = __float_as_uint(h);
-            mid[i] = __float_as_uint(md);
-            lo[i] = __float_as_uint(r1 - md);
-        }
-        uint32_t ph[4], pm[4], pl[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            ph[j] = __builtin_amdgcn_perm(hi[2 * j + 1], hi[2 * j], 0x07060302u);
-            pm[j] = __builtin_amdgcn_perm(mid[2 * j + 1], mid[2 * j], 0x07060302u);
-            pl[j] = __builtin_amdgcn_perm(lo[2 * j + 1], lo[2 * j], 0x07060302u);
-        }
-        bp[0] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{ph[0], ph[1], ph[2], ph[3]});
-        bp[1] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pm[0], pm[1], pm[2], pm[3]});
-        bp[2] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pl[0], pl[1], pl[2], pl[3]});
-    };
-    auto mma3 = [&](const uint8_t *xs, const WLine &s, float a) {
-        glint_bf16x8 af[2][MB];
-        aread(xs, 0, af[0]);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            glint_bf16x8 bp[3];
-            split3(s, a, st, bp);
-            if (st + 1 < 4)
-                aread(xs, st + 1, af[(st + 1) & 1]);
-#pragma unroll
-            for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-                    acc[mb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[st & 1][mb], bp[pl], acc[mb][0], 0, 0, 0);
-        }
-    };
     /* step X (u = X % U): x chunk X + 1 into LDS, x chunk X + 3 and the absmax of X + 3
      * issued, line X + 2 into LDS, line X + 1 out of LDS, line X dequantized and multiplied;
      * on even steps lines X + 4 and X + 5 go out into the stages lines X and X + 1 left */
@@ -1453,21 +1397,13 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
         aload(X + 3, am[(u + 3) % U]);
         wput(X + 2, wl[(u + 2) % U]);
         wget(X + 1, wb[(u + 1) & 1]);
-        if constexpr (F32) {
-            if ((u & 1) == 0) {
-                wline(X + U, wl[u]);
-                wline(X + U + 1, wl[u + 1]);
-            }
-            mma3((u & 1) ? xb1 : xb0, wb[u & 1], am[u]);
-        } else {
-            glint_bf16x8 bq[4];
-            dequant(wb[u & 1], am[u], bq);
-            if ((u & 1) == 0) {
-                wline(X + U, wl[u]);
-                wline(X + U + 1, wl[u + 1]);
-            }
-            mma((u & 1) ? xb1 : xb0, bq);
+        glint_bf16x8 bq[4];
+        dequant(wb[u & 1], am[u], bq);
+        if ((u & 1) == 0) {
+            wline(X + U, wl[u]);
+            wline(X + U + 1, wl[u + 1]);
         }
+        mma((u & 1) ? xb1 : xb0, bq);
     };
 
     GlintCellFillHN<(2048 + T - 1) / T> fill;
@@ -1531,17 +1467,370 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int m = 16 * mb + 4 * g + i;
-                if (m < M) {
-                    if constexpr (F32)
-                        y[(int64_t)m * N + n0 + nl] = acc[mb][0][i];
-                    else
-                        y[(int64_t)m * N + n0 + nl] = glint_f32_to_bf16(acc[mb][0][i]);
-                }
+                if (m < M)
+                    y[(int64_t)m * N + n0 + nl] = glint_f32_to_bf16(acc[mb][0][i]);
             }
 }
 
-/* k_htile_rl (k_htile_rd) over an M <= 64 prefill, BF16 out, or f32 out (F32: k_htile_rl
- * only). Returns 1 where the shape does not fit (K % 128 != 0, offsets beyond 31 bits; the
+/* k_htile_rl3: f32 out (the reference ABI) at M <= 64: k_htile_rl's loads and x path with exact
+ * f32 weights, and the block scale applied to block sums instead of to weights.
+ *   - The cell table holds the cells as three BF16 planes, hi + mid + lo == cell exactly (8-byte
+ *     entries, 32 copies: all 256 B of a row, so the W lines have LDS rows of their own). A
+ *     weight costs half a VALU op for its code byte, one v_perm for the address, one LDS read
+ *     and half a v_perm per plane; splitting w = cell * absmax per weight cost a multiply, the
+ *     split's four operations and the three half v_perms.
+ *   - A lane takes 8 B of each 64-block of its row (16 weights), so MFMA steps 2 b and 2 b + 1 of
+ *     a chunk hold block b alone. Their MFMAs start from zero, and D's column is the lane's own
+ *     W row, so a block's sums (4 per lane and 16 rows of x) take one FMA by the lane's scale.
+ *     x times a plane is exact; the f32 sums of a block, one rounded product with the scale and
+ *     one addition per block are all the roundings there are.
+ *   - A workgroup that met a scale that is infinite, NaN or at least 2^126 goes over its split
+ *     again with the products w = cell * absmax split as GlintTileProducer::finish_split does,
+ *     so infinities of both signs meet as they do in a sum of weights.
+ * Bound: a step's chain of LDS reads, lookups and MFMAs at two waves per SIMD, as k_htile_rl.
+ * Measured against the per-weight split (rotated pins):
+ * 14336 x 4096 M = 5 30.6 (as two small-M launches) -> 21.0 us, 8 30.0 -> 21.0, 32 33.9 -> 26.1,
+ * 64 41.9 -> 36.7; 4096 x 14336 M = 8 29.3 -> 21.5, 64 41.3 -> 35.4; relative error against
+ * 64 bits 5.0e-7 -> 1.3e-7. BF16 out in the same form (one plane, BF16(cell)) was slower than
+ * k_htile_rl (M = 8 18.0 -> 18.9 us), and so were the scaling FMAs put off to the next step
+ * (M = 32 23.8 -> 26.5) and a branch on special scales in the step (M = 32 25.7). */
+#ifndef RD_FL_F32
+#define RD_FL_F32 1 /* f32 out at M <= 64: k_htile_rl3 (0: the f32 tiles) */
+#endif
+/* the three BF16 planes of an f32 (upper halves of the words): hi + mid + lo == v exactly for
+ * finite v; an infinite v keeps mid = lo = 0 where v - hi would be NaN */
+__device__ __forceinline__ void rl_split3(float v, bool big, uint32_t (&o)[3]) {
+    const float h = __uint_as_float(__float_as_uint(v) & 0xFFFF0000u);
+    float r1 = v - h;
+    if (big)
+        r1 = __builtin_isinf(v) ? 0.0f : r1;
+    const float md = __uint_as_float(__float_as_uint(r1) & 0xFFFF0000u);
+    o[0] = __float_as_uint(h);
+    o[1] = __float_as_uint(md);
+    o[2] = __float_as_uint(r1 - md);
+}
+/* a cell's table entry for f32 out: hi | mid << 16, lo */
+__device__ __forceinline__ glint_u32x2 rl_entry(float cell) {
+    uint32_t o[3];
+    rl_split3(cell, false, o);
+    return glint_u32x2{(o[0] >> 16) | o[1], o[2] >> 16};
+}
+template <int MB>
+__global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
+                                                     const float *__restrict__ absmax, const uint16_t *__restrict__ x,
+                                                     float *__restrict__ y,
+                                                     int M, int N, int K, int R, int cps, float *__restrict__ part,
+                                                     unsigned *ctr) {
+    constexpr int KW = 2, T = 512, STRIPS = 4;
+    constexpr int NP = 3;               /* BF16 planes of a weight */
+    constexpr int XROW = 256 * KW;      /* bytes of one x row of an x chunk (one W line) */
+    constexpr int XCH = 16 * MB * XROW; /* bytes of one x chunk */
+    constexpr int NX = XCH / 16 / T;    /* 16-B pieces of an x chunk per thread */
+    constexpr int U = RL_STAGES;        /* W line register stages (x chunks per unrolled round) */
+    static_assert(U % 2 == 0 && U >= 4, "stages in pairs, lines loaded U - 2 steps ahead of their LDS write");
+    static_assert(NX >= 1 && NX * 16 * T == XCH, "x chunk split over the threads");
+    __shared__ __attribute__((aligned(16))) float ltab[GLINT_LDS_CELLS64_WORDS];
+    __shared__ __attribute__((aligned(16))) uint8_t xb0[XCH], xb1[XCH];
+    __shared__ __attribute__((aligned(16))) uint8_t wln[256 * 128];
+    uint8_t *const lt = (uint8_t *)ltab;
+    const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int strip = w % STRIPS, kw = w / STRIPS;
+    const uint32_t lane4 = (uint32_t)(lane & 31) * 8u; /* copy lane % 32 of an entry */
+    const int n0 = blockIdx.x * R;
+    const int nrows = min(R, N - n0); /* >= 1 */
+    const int c0 = blockIdx.z * cps;  /* even: the host keeps cps even */
+    const int nj = min(K >> 7, c0 + cps) - c0;
+    const int nxc = (nj + 1) >> 1; /* x chunks = W lines */
+    const uint32_t rowb = (uint32_t)K >> 1;
+
+    const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(hole + (int64_t)n0 * rowb), (short)0, (int)((uint32_t)nrows * rowb), GLINT_BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(plug + (int64_t)n0 * rowb), (short)0, (int)((uint32_t)nrows * rowb), GLINT_BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(absmax + (int64_t)n0 * (K >> 6)), (short)0, (int)((uint32_t)nrows * (rowb >> 3)), GLINT_BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)x, (short)0, (int)((uint32_t)M * (uint32_t)K * 2u), GLINT_BUF_DWORD3);
+    /* the lane's line piece: row lr of the strip, 16-B piece lane % 8 */
+    const int lr = 8 * kw + (lane >> 3);
+    const uint32_t lofs = (uint32_t)(16 * strip + lr) * rowb + (uint32_t)(lane & 7) * 16u;
+    /* the lane's two block scales: MFMA row 16 strip + m16 */
+    const uint32_t aofs = (uint32_t)(16 * strip + m16) * (uint32_t)(K >> 6) * 4u;
+    /* LDS slots: W row r of plane pl in buffer b of this strip is LDS row
+     * ((strip * 2 + b) * 2 + pl) * 16 + r; piece c sits at c ^ swz(r). 128-B rows: rows r and
+     * r + 8 share their banks, so the swizzle takes the row's upper bits */
+    auto swz = [](int r) -> int { return (r >> 1) & 7; };
+    const uint32_t put0 = (uint32_t)((strip * 2) * 2 * 16 + lr) * 128u + ((uint32_t)((lane & 7) ^ swz(lr)) << 4);
+    /* 8 B of block b: piece 4 kw + 2 b + g / 2, half g % 2 */
+    const uint32_t getr = (uint32_t)((strip * 2) * 2 * 16 + m16) * 128u + 8u * (uint32_t)(g & 1);
+    const uint32_t get0[2] = {getr + ((uint32_t)((4 * kw + (g >> 1)) ^ swz(m16)) << 4),
+                              getr + ((uint32_t)((4 * kw + 2 + (g >> 1)) ^ swz(m16)) << 4)};
+    constexpr uint32_t BUF = 2 * 16 * 128, PLANE = 16 * 128; /* byte steps of b and pl */
+    uint32_t xgo[NX], xlo[NX];
+    int xhalf[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+        const int sl = (int)threadIdx.x + T * i, r = sl / (16 * KW), pc = sl % (16 * KW);
+        xgo[i] = (uint32_t)r * (uint32_t)K * 2u + (uint32_t)(pc << 4);
+        xlo[i] = (uint32_t)(r * XROW + ((pc ^ (r & 15)) << 4));
+        xhalf[i] = pc >> 4; /* the W chunk of the line the piece belongs to */
+    }
+
+    struct WLine {
+        glint_u32x4 h, p;
+    };
+    struct WBlk {
+        glint_u32x2 h[2], p[2]; /* [block]: the words of MFMA steps 2 b and 2 b + 1 */
+    };
+    WLine wl[U];      /* lines in the load layout */
+    WBlk wb[2];       /* lines in the MFMA layout (this wave's chunk), from LDS */
+    glint_f32x2 am[U]; /* the wave's two block scales of x chunk X, stage X % U */
+    glint_u32x4 xr[2][NX];
+    auto wline = [&](int X, WLine &s) {
+        const uint32_t o = 2 * X < nj ? lofs + (uint32_t)(c0 + 2 * X) * 64u : RD_OOR;
+        s.h = __builtin_amdgcn_raw_buffer_load_b128(rh, o, 0, 0);
+        s.p = __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, 0);
+    };
+    auto aload = [&](int X, glint_f32x2 &a) {
+        const int j = 2 * X + kw;
+        a = __builtin_bit_cast(glint_f32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                                ra, j < nj ? aofs + (uint32_t)(c0 + j) * 8u : RD_OOR, 0, 0));
+    };
+    auto xload = [&](int X, glint_u32x4 (&xs)[NX]) {
+        const uint32_t c = (uint32_t)(c0 + KW * X);
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+            xs[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, 2 * X + xhalf[i] < nj ? xgo[i] + c * 256u : RD_OOR, 0, 0);
+    };
+    auto xstore = [&](uint8_t *buf, const glint_u32x4 (&xs)[NX]) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+            *(glint_u32x4 *)(buf + xlo[i]) = xs[i];
+    };
+    auto wput = [&](int X, const WLine &s) {
+        const uint32_t a = put0 + (uint32_t)(X & 1) * BUF;
+        *(glint_u32x4 *)(wln + a) = s.h;
+        *(glint_u32x4 *)(wln + a + PLANE) = s.p;
+    };
+    auto wget = [&](int X, WBlk &s) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const uint32_t a = get0[b] + (uint32_t)(X & 1) * BUF;
+            s.h[b] = *(const glint_u32x2 *)(wln + a);
+            s.p[b] = *(const glint_u32x2 *)(wln + a + PLANE);
+        }
+    };
+    /* the 8 weights of MFMA step st as planes of their cells */
+    auto planes = [&](const WBlk &s, int st, glint_bf16x8 (&bp)[NP]) {
+        const uint32_t H = s.h[st >> 1][st & 1], P = s.p[st >> 1][st & 1];
+        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+        const uint32_t ad[8] = {glint_cell_addr<0>(E, lane4), glint_cell_addr<0>(O, lane4), glint_cell_addr<1>(E, lane4),
+                                glint_cell_addr<1>(O, lane4), glint_cell_addr<2>(E, lane4), glint_cell_addr<2>(O, lane4),
+                                glint_cell_addr<3>(E, lane4), glint_cell_addr<3>(O, lane4)};
+        uint32_t pk[NP][4];
+        glint_u32x2 e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            e[i] = *(const glint_u32x2 *)(lt + ad[i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pk[0][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x05040100u);
+            pk[1][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x07060302u);
+            pk[2][j] = __builtin_amdgcn_perm(e[2 * j + 1].y, e[2 * j].y, 0x05040100u);
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+    };
+    /* the same with the weights of the lane's row multiplied by `a` */
+    auto planes_scaled = [&](const WBlk &s, int st, float a, glint_bf16x8 (&bp)[NP]) {
+        const uint32_t H = s.h[st >> 1][st & 1], P = s.p[st >> 1][st & 1];
+        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            v[i] = (&kCells[0][0])[((i & 1 ? O : E) >> (8 * (i >> 1))) & 255u] * a;
+        uint32_t pk[NP][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t l[3], h[3];
+            rl_split3(v[2 * j], true, l);
+            rl_split3(v[2 * j + 1], true, h);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                pk[i][j] = __builtin_amdgcn_perm(h[i], l[i], 0x07060302u);
+        }
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+    };
+    glint_f32x4 acc[MB][1];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+        acc[mb][0] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+    /* x of MFMA step st: elements 64 (st / 2) + 16 g + 8 (st % 2) of the wave's chunk */
+    auto aread = [&](const uint8_t *xs, int st, glint_bf16x8 (&af)[MB]) {
+        const int pc = 16 * kw + 8 * (st >> 1) + 2 * g + (st & 1);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            af[mb] = __builtin_bit_cast(glint_bf16x8,
+                                        *(const glint_u32x4 *)(xs + (16 * mb + m16) * XROW + ((pc ^ m16) << 4)));
+    };
+    /* the chunk's 4 MFMA steps, the two blocks by turns (their sums are independent); the
+     * smallest plane first */
+    auto mma = [&](const uint8_t *xs, const WBlk &s, glint_f32x2 a, bool scaled) {
+        glint_f32x4 t[2][MB];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int st = ((i & 1) << 1) | (i >> 1), b = i & 1;
+            glint_bf16x8 af[MB], bp[NP];
+            aread(xs, st, af);
+            if (scaled)
+                planes_scaled(s, st, b ? a.y : a.x, bp);
+            else
+                planes(s, st, bp);
+#pragma unroll
+            for (int pl = NP - 1; pl >= 0; --pl)
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    t[b][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        af[mb], bp[pl], i < 2 && pl == NP - 1 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb], 0, 0, 0);
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[mb][0][i] = scaled ? acc[mb][0][i] + t[b][mb][i] : fmaf(b ? a.y : a.x, t[b][mb][i], acc[mb][0][i]);
+    };
+    /* step X (u = X % U): x chunk X + 1 into LDS, x chunk X + 3 and the scales of X + 3
+     * issued, line X + 2 into LDS, line X + 1 out of LDS, line X multiplied; on even steps
+     * lines X + 4 and X + 5 go out into the stages lines X and X + 1 left */
+    uint32_t amax = 0; /* largest |scale| met */
+    auto step = [&](int X, int u) {
+        __syncthreads();
+        xstore((u & 1) ? xb0 : xb1, xr[(u + 1) & 1]);
+        xload(X + 3, xr[(u + 1) & 1]);
+        const glint_f32x2 a = am[u];
+        amax = max(amax, max(__float_as_uint(a.x) & 0x7FFFFFFFu, __float_as_uint(a.y) & 0x7FFFFFFFu));
+        aload(X + 3, am[(u + 3) % U]);
+        wput(X + 2, wl[(u + 2) % U]);
+        wget(X + 1, wb[(u + 1) & 1]);
+        if ((u & 1) == 0) {
+            wline(X + U, wl[u]);
+            wline(X + U + 1, wl[u + 1]);
+        }
+        mma((u & 1) ? xb1 : xb0, wb[u & 1], a, false);
+    };
+    /* the split once more, unpipelined, with every weight multiplied by its scale */
+    auto rerun = [&]() {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            acc[mb][0] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int X = 0; X < nxc; ++X) {
+            __syncthreads();
+            xload(X, xr[0]);
+            wline(X, wl[0]);
+            aload(X, am[0]);
+            xstore(xb0, xr[0]);
+            wput(0, wl[0]);
+            __syncthreads();
+            wget(0, wb[0]);
+            mma(xb0, wb[0], am[0], true);
+        }
+    };
+
+    /* 16-B runs of two copies; run r is cell r / 16 (a wave's 64 runs hold 4 cells: scalar
+     * loads), 4096 runs in 8 steps */
+    glint_f32x4 c4[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        c4[k] = *(const glint_f32x4 *)(&kCells[0][0] + ((64 * w + k * T) >> 4));
+    __builtin_amdgcn_sched_barrier(0);
+    xload(0, xr[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    xload(1, xr[1]);
+    aload(0, am[0]);
+    aload(1, am[1]);
+    aload(2, am[2]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < U; ++s)
+        wline(s, wl[s]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float lo = g & 1 ? c4[k].y : c4[k].x, hi = g & 1 ? c4[k].w : c4[k].z;
+        const glint_u32x2 e = rl_entry(g & 2 ? hi : lo);
+        ((glint_u32x4 *)lt)[threadIdx.x + k * T] = glint_u32x4{e.x, e.y, e.x, e.y};
+    }
+    xstore(xb0, xr[0]);
+    xload(2, xr[0]);
+    wput(0, wl[0]);
+    wput(1, wl[1]);
+    __syncthreads();
+    wget(0, wb[0]);
+    int X = 0;
+    for (; X + U <= nxc; X += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            step(X + u, u);
+    }
+#pragma unroll
+    for (int u = 0; u + 1 < U; ++u)
+        if (X + u < nxc)
+            step(X + u, u);
+    __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0); /* the trailing dropped loads */
+    /* the strip's two partials meet in xb0 (the x buffers are free); the waves' largest scales
+     * in xb1 tell whether the workgroup has to run again */
+    float *red = (float *)xb0;
+    uint32_t *wmax = (uint32_t *)xb1;
+    static_assert(STRIPS * 64 * MB * 4 * 4 <= XCH, "partials fit an x buffer");
+    auto meet = [&]() -> bool {
+        const bool big = __any(amax >= 0x7E800000u); /* 2^126, infinite or NaN */
+        __syncthreads();
+        if (lane == 0)
+            wmax[w] = big;
+        if (kw > 0)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    red[((strip * MB + mb) * 4 + i) * 64 + lane] = acc[mb][0][i];
+        __syncthreads();
+        const glint_u32x4 f0 = ((const glint_u32x4 *)wmax)[0], f1 = ((const glint_u32x4 *)wmax)[1];
+        return (f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) != 0u;
+    };
+    if (meet()) {
+        rerun();
+        meet();
+    }
+    if (kw == 0) /* added in kw order */
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[mb][0][i] += red[((strip * MB + mb) * 4 + i) * 64 + lane];
+    __syncthreads(); /* the split-K epilogue's flag word lives in xb0 */
+    if (gridDim.z > 1 && !tile_splitk_epilogue<MB, 1, 64 * STRIPS>(acc, part, ctr, *(unsigned *)xb1,
+                                                                    (int)threadIdx.x, kw == 0))
+        return;
+    const int nl = 16 * strip + m16;
+    if (kw == 0 && nl < nrows)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 16 * mb + 4 * g + i;
+                if (m < M)
+                    y[(int64_t)m * N + n0 + nl] = acc[mb][0][i];
+            }
+}
+
+/* k_htile_rl (k_htile_rd) over an M <= 64 prefill, BF16 out, or f32 out (F32: k_htile_rl3). Returns 1 where the shape does not fit (K % 128 != 0, offsets beyond 31 bits; the
  * caller takes the LDS tiles), -5 where a `fixed` workspace is too small for the split plan,
  * else 0 or -3. */
 template <int MB, bool F32>
@@ -1568,12 +1857,14 @@ static int htile_launch_rd_mb(const uint8_t *hole, const uint8_t *plug, const fl
         if (!fits) {
             if (fixed)
                 return -5;
+            if (F32 && M <= 2 * GEMV_MR_MAX_F32 - 2)
+                return 1; /* no workspace (a capture without one): the two small-M launches need none */
             ks = plan(1, cps, R, gx); /* no workspace (a capture without one): unsplit */
             ws = GlintSplitWs{nullptr, nullptr, 0, 0};
         }
     }
     if (F32)
-        k_htile_rl<MB, true><<<dim3(gx, 1, (unsigned)ks), 512, 0, st>>>(hole, plug, absmax, x, (float *)y, M, N, K, R,
+        k_htile_rl3<MB><<<dim3(gx, 1, (unsigned)ks), 512, 0, st>>>(hole, plug, absmax, x, (float *)y, M, N, K, R,
                                                                       cps, ws.part, ws.ctr);
     else if (RD_FL)
         k_htile_rl<MB><<<dim3(gx, 1, (unsigned)ks), 512, 0, st>>>(hole, plug, absmax, x, (uint16_t *)y, M, N, K, R, cps,
@@ -1650,11 +1941,11 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
     const bool rl_first = M > (OUT_BF16 ? GEMV_MR_RL : GEMV_MR_RL_F32);
     if (mfma_ok && GEMV_MR_ON && !rl_first && gemv_mr_takes(M, K, !OUT_BF16))
         return htile_launch_gemv_mr<!OUT_BF16>(hole, plug, absmax, x, y, M, N, K, st);
-    /* f32 out from GEMV_MR_RL_F32 + 1 rows: k_htile_rl's three-plane form (14336 x 4096 M = 8
-     * 31.3 -> 30.1 us, 16 49.7 -> 30.2, 32 49.9 -> 33.9, 64 50.3 -> 41.4; 4096 x 14336 M = 8
-     * 33.6 -> 29.2, 64 61.8 -> 39.8, against the two small-M launches and the f32 tiles; at
-     * M = 5 the two launches were faster, 30.6 against 31.5) */
-    if (!OUT_BF16 && mfma_ok && M > GEMV_MR_RL_F32 && M <= 64) {
+    /* f32 out from GEMV_MR_RL_F32 + 1 rows: k_htile_rl3 (14336 x 4096 M = 5 21.0 us against 30.6
+     * for the two small-M launches below, M = 64 36.7 against 50.3 for the f32 tiles; at M = 4
+     * the small-M GEMV takes 15.4) */
+    if (!OUT_BF16 && mfma_ok && M > GEMV_MR_RL_F32 && M <= 64 &&
+        (M > 2 * GEMV_MR_MAX_F32 - 2 || (int64_t)N * K >= GEMV_MR_RL_F32_WEIGHTS)) {
         const int rc = htile_launch_rd<true>(hole, plug, absmax, x, y, M, N, K, st, fixed);
         if (rc != 1)
             return rc;

@@ -1,0 +1,55 @@
+"""k_htile_rl3: f32 out at 5 <= M <= 64, K % 128 == 0 (cells as three BF16 planes, the block
+scale on block sums).
+
+Against the oracle's float64 sum within (K + 2) 2^-23 sum |w x| (each block's f32 sums, one
+rounded scaling and one addition per block stay below one rounding per weight). Shapes: one,
+two and four 16-row blocks of x, a single W chunk, odd chunk counts (the last line half used),
+strips partly filled, K split over workgroups."""
+import numpy as np
+import pytest
+
+from glint_amd import glint_hip as H
+from tests.gpu_util import bf16_bits, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(M, N, K):
+    rng = np.random.default_rng(M + 7 * N + K)
+    hole = rng.integers(0, 256, N * K // 2, dtype=np.uint8)
+    plug = rng.integers(0, 256, N * K // 2, dtype=np.uint8)
+    am = rng.uniform(0.01, 1.0, N * K // 64).astype(np.float32) * (rng.random(N * K // 64) > 0.1)
+    return hole, plug, am.astype(np.float32), bf16_bits(rng.normal(0, 1e-3, M * K).astype(np.float32))
+
+
+SHAPES = [(5, 13, 128), (6, 1000, 384), (8, 4097, 4096), (16, 56, 2048), (17, 777, 640), (32, 300, 14464), (33, 130, 256),
+          (64, 64, 14464), (64, 1000, 2304)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_vs_float64(oracle, M, N, K):
+    print(f"htile planes M={M} N={N} K={K}", flush=True)
+    ins = _inputs(M, N, K)
+    y = host(H.htile_f32(*[dev(a) for a in ins[:3]], dev(ins[3]).reshape(M, K), N, K, 64)).reshape(M, N)
+    ref, asum = (a.reshape(M, N) for a in oracle.htile_f64(*ins, M, N, K, 64))
+    assert (np.abs(y - ref) <= (K + 2) * 2.0 ** -23 * asum).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 13, 384), (20, 100, 1152), (64, 64, 14464)])
+def test_special_scales(oracle, M, N, K):
+    """Infinite, NaN and huge scales: NaN and infinities where the f32 restatement has them (a
+    workgroup that met one goes over its K range again with weights as products), finite
+    outputs, its own rows' and others', within the bound."""
+    print(f"htile planes special M={M} N={N} K={K}", flush=True)
+    hole, plug, am, x = _inputs(M, N, K)
+    nb = K // 64
+    am[nb * 3 + 1], am[nb * 5], am[nb * 7 + nb - 1] = np.inf, np.nan, -np.inf
+    am[nb * 9 + 2], am[nb * 11] = np.finfo(np.float32).max, np.float32(2.0 ** 126)
+    y = host(H.htile_f32(dev(hole), dev(plug), dev(am), dev(x).reshape(M, K), N, K, 64)).reshape(M, N)
+    with np.errstate(all="ignore"):
+        want = oracle.htile_f32(hole, plug, am, x, M, N, K, 64).reshape(M, N)
+        ref, asum = (a.reshape(M, N) for a in oracle.htile_f64(hole, plug, am, x, M, N, K, 64))
+    assert np.isnan(want).any()
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
+    fin = np.isfinite(want)
+    assert (np.abs(y - ref)[fin] <= ((K + 2) * 2.0 ** -23 * asum)[fin]).all()
