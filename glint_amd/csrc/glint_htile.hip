@@ -1495,7 +1495,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
  * k_htile_rl (M = 8 18.0 -> 18.9 us), and so were the scaling FMAs put off to the next step
  * (M = 32 23.8 -> 26.5) and a branch on special scales in the step (M = 32 25.7). */
 #ifndef RD_FL_F32
-#define RD_FL_F32 1 /* f32 out at M <= 64: k_htile_rl3 (0: the f32 tiles) */
+#define RD_FL_F32 1 /* f32 out at M <= 64: k_htile_rl3 (0: k_htile_f3) */
 #endif
 /* the three BF16 planes of an f32 (upper halves of the words): hi + mid + lo == v exactly for
  * finite v; an infinite v keeps mid = lo = 0 where v - hi would be NaN */
@@ -1830,6 +1830,281 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
             }
 }
 
+/* k_htile_f3: f32 out at M > 64 (the reference ABI's prefill), bs = 64, K % 128 == 0, aligned:
+ * k_htile_rl3's exact cell planes and block scaling on 16 MB x 128 output tiles.
+ *   - Wave w of 8 owns W rows [16 w, +16) of the tile and all its 16 MB rows of x, so the three
+ *     planes of a weight are made once per workgroup in the registers of the wave that multiplies
+ *     them, never pass through LDS, and every x fragment read from LDS feeds three MFMAs. (Tiles
+ *     that put the planes into LDS read 3 fragments of W for every 2 of x and wrote 24 KiB a
+ *     step.)
+ *   - A step is a 128-wide K chunk: 12 MB MFMAs per wave and one barrier. The lane's 8 B of each
+ *     64-block of its row come straight from memory one chunk ahead (the planes are cached: every
+ *     16 MB rows of x read them again), x through registers into a swizzled LDS double buffer.
+ *   - Block sums start from zero; a block's FMAs by its scale are issued among the next block's
+ *     MFMAs (two sets of sums).
+ *   - K is split over gridDim.z workgroups where the tiles alone leave CUs idle.
+ * Special scales as in k_htile_rl3.
+ * Bound: the matrix cores, three planes of every product (2048 x 14336 x 4096: 1.21 PFLOP/s of
+ * BF16 MFMA; a dense BF16 product of that shape by the vendor's library runs at 1.14). Measured
+ * against the three-plane LDS tiles (128 x 128; rotated pins): 2048 x 14336 x 4096 762 -> 597 us,
+ * 2047 x 8192 x 3072 333 -> 261, 512 x 14336 x 4096 215 -> 164, 512 x 4096 x 14336 196 -> 158,
+ * 128 x 14336 x 4096 64 -> 50, 96 x 4096 x 4096 28.8 -> 18.6; relative error against 64 bits
+ * 7.1e-7 -> 1.6e-7 at 2048 x 14336 x 4096. */
+template <int MB>
+__global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
+                                                     const float *__restrict__ absmax, const uint16_t *__restrict__ x,
+                                                     float *__restrict__ y, int M, int N, int K, int cps,
+                                                     float *__restrict__ part, unsigned *ctr) {
+    constexpr int T = 512, BN = 128, BM = 16 * MB;
+    constexpr int XCH = BM * 256;      /* bytes of an x chunk */
+    constexpr int NX = XCH / 16 / T;   /* its 16-B pieces per thread */
+    static_assert(NX >= 1 && NX * 16 * T == XCH, "x chunk split over the threads");
+    __shared__ __attribute__((aligned(16))) float ltab[GLINT_LDS_CELLS64_WORDS];
+    __shared__ __attribute__((aligned(16))) uint8_t xb0[XCH], xb1[XCH];
+    uint8_t *const lt = (uint8_t *)ltab;
+    const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane8 = (uint32_t)(lane & 31) * 8u; /* copy lane % 32 of an entry */
+    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+    const int nrows = min(BN, N - n0); /* >= 1 */
+    const int c0 = blockIdx.z * cps;
+    const int nj = min(K >> 7, c0 + cps) - c0; /* chunks of the split, >= 1 */
+    const uint32_t rowb = (uint32_t)K >> 1;
+    const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(hole + (int64_t)n0 * rowb), (short)0, (int)((uint32_t)nrows * rowb), GLINT_BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(plug + (int64_t)n0 * rowb), (short)0, (int)((uint32_t)nrows * rowb), GLINT_BUF_DWORD3);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(absmax + (int64_t)n0 * (K >> 6)), (short)0, (int)((uint32_t)nrows * (rowb >> 3)), GLINT_BUF_DWORD3);
+    const int mrows = min(BM, M - m0); /* >= 1 */
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(x + (int64_t)m0 * K), (short)0, (int)((uint32_t)mrows * (uint32_t)K * 2u), GLINT_BUF_DWORD3);
+    /* rows past N or M lie past their buffers: loads of them are dropped and give zeros */
+    const uint32_t wrow = (uint32_t)(16 * w + m16);
+    const uint32_t wofs = wrow * rowb + 8u * (uint32_t)g, aofs = wrow * (uint32_t)(K >> 6) * 4u;
+    uint32_t xgo[NX], xlo[NX];
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+        const int sl = (int)threadIdx.x + T * i, r = sl >> 4, pc = sl & 15;
+        xgo[i] = (uint32_t)r * (uint32_t)K * 2u + (uint32_t)(pc << 4);
+        xlo[i] = (uint32_t)(r * 256 + ((pc ^ (r & 15)) << 4));
+    }
+    struct WBlk {
+        glint_u32x2 h[2], p[2]; /* [block]: the words of MFMA steps 2 b and 2 b + 1 */
+        glint_f32x2 a;          /* the blocks' scales */
+    };
+    WBlk wb[2];
+    glint_u32x4 xr[NX];
+    auto wload = [&](int j, WBlk &s) {
+        const uint32_t c = (uint32_t)(c0 + j);
+        const uint32_t o = j < nj ? wofs + c * 64u : RD_OOR, oa = j < nj ? aofs + c * 8u : RD_OOR;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            s.h[b] = __builtin_bit_cast(glint_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rh, o + 32u * b, 0, 0));
+            s.p[b] = __builtin_bit_cast(glint_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rp, o + 32u * b, 0, 0));
+        }
+        s.a = __builtin_bit_cast(glint_f32x2, __builtin_amdgcn_raw_buffer_load_b64(ra, oa, 0, 0));
+    };
+    auto xload = [&](int j) {
+        const uint32_t c = (uint32_t)(c0 + j) * 256u;
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+            xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, j < nj ? xgo[i] + c : RD_OOR, 0, 0);
+    };
+    auto xstore = [&](uint8_t *buf) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+            *(glint_u32x4 *)(buf + xlo[i]) = xr[i];
+    };
+    auto planes = [&](uint32_t H, uint32_t P, glint_bf16x8 (&bp)[3]) {
+        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+        const uint32_t ad[8] = {glint_cell_addr<0>(E, lane8), glint_cell_addr<0>(O, lane8), glint_cell_addr<1>(E, lane8),
+                                glint_cell_addr<1>(O, lane8), glint_cell_addr<2>(E, lane8), glint_cell_addr<2>(O, lane8),
+                                glint_cell_addr<3>(E, lane8), glint_cell_addr<3>(O, lane8)};
+        glint_u32x2 e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            e[i] = *(const glint_u32x2 *)(lt + ad[i]);
+        uint32_t pk[3][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            pk[0][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x05040100u);
+            pk[1][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x07060302u);
+            pk[2][j] = __builtin_amdgcn_perm(e[2 * j + 1].y, e[2 * j].y, 0x05040100u);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+    };
+    auto planes_scaled = [&](uint32_t H, uint32_t P, float a, glint_bf16x8 (&bp)[3]) {
+        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+        uint32_t pk[3][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t l[3], h[3];
+            rl_split3((&kCells[0][0])[(E >> (8 * j)) & 255u] * a, true, l);
+            rl_split3((&kCells[0][0])[(O >> (8 * j)) & 255u] * a, true, h);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                pk[i][j] = __builtin_amdgcn_perm(h[i], l[i], 0x07060302u);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+    };
+    glint_f32x4 acc[MB][1], t[2][MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+        acc[mb][0] = t[1][mb] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+    /* block b's sums in t[b]: MFMA step st = 2 b + s takes x elements 64 b + 16 g + 8 s, +8 */
+    auto block = [&](const uint8_t *xs, const WBlk &k, int b, bool scaled) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            glint_bf16x8 bp[3];
+            if (scaled)
+                planes_scaled(k.h[b][s], k.p[b][s], b ? k.a.y : k.a.x, bp);
+            else
+                planes(k.h[b][s], k.p[b][s], bp);
+            const int pc = 8 * b + 2 * g + s;
+            glint_bf16x8 af[MB];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                af[mb] = __builtin_bit_cast(glint_bf16x8,
+                                            *(const glint_u32x4 *)(xs + (16 * mb + m16) * 256 + ((pc ^ m16) << 4)));
+#pragma unroll
+            for (int pl = 2; pl >= 0; --pl) /* the smallest plane first */
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    t[b][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        af[mb], bp[pl], s == 0 && pl == 2 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb], 0, 0, 0);
+        }
+    };
+    auto add = [&](int b, float a) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[mb][0][i] = fmaf(a, t[b][mb][i], acc[mb][0][i]);
+    };
+    uint32_t amax = 0; /* largest |scale| met */
+    float ap = 0.f;    /* scale of the sums in t[1] */
+    auto step = [&](int j, int u) {
+        __syncthreads();
+        xstore(u ? xb0 : xb1);
+        xload(j + 2);
+        wload(j + 1, wb[u ^ 1]);
+        const WBlk &k = wb[u];
+        amax = max(amax, max(__float_as_uint(k.a.x) & 0x7FFFFFFFu, __float_as_uint(k.a.y) & 0x7FFFFFFFu));
+        const uint8_t *xs = u ? xb1 : xb0;
+        block(xs, k, 0, false);
+        add(1, ap);
+        block(xs, k, 1, false);
+        add(0, k.a.x);
+        ap = k.a.y;
+    };
+
+    glint_f32x4 c4[8]; /* the table: as k_htile_rl3's */
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        c4[i] = *(const glint_f32x4 *)(&kCells[0][0] + ((64 * w + i * T) >> 4));
+    xload(0);
+    wload(0, wb[0]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float lo = g & 1 ? c4[i].y : c4[i].x, hi = g & 1 ? c4[i].w : c4[i].z;
+        const glint_u32x2 e = rl_entry(g & 2 ? hi : lo);
+        ((glint_u32x4 *)lt)[threadIdx.x + i * T] = glint_u32x4{e.x, e.y, e.x, e.y};
+    }
+    xstore(xb0);
+    xload(1);
+    int j = 0;
+    for (; j + 2 <= nj; j += 2) {
+        step(j, 0);
+        step(j + 1, 1);
+    }
+    if (j < nj)
+        step(j, 0);
+    add(1, ap);
+
+    /* a special scale anywhere in the workgroup: the split once more, unpipelined, with every
+     * weight multiplied by its scale */
+    const bool big = __any(amax >= 0x7E800000u); /* 2^126, infinite or NaN */
+    uint32_t *flag = (uint32_t *)xb0;
+    __syncthreads();
+    if (lane == 0)
+        flag[w] = big;
+    __syncthreads();
+    const glint_u32x4 f0 = ((const glint_u32x4 *)flag)[0], f1 = ((const glint_u32x4 *)flag)[1];
+    if ((f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) != 0u) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            acc[mb][0] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int i = 0; i < nj; ++i) {
+            xload(i);
+            wload(i, wb[0]);
+            __syncthreads();
+            xstore(xb1);
+            __syncthreads();
+            block(xb1, wb[0], 0, true);
+            add(0, 1.f);
+            block(xb1, wb[0], 1, true);
+            add(1, 1.f);
+        }
+    }
+    if (gridDim.z > 1) {
+        __syncthreads(); /* the flags have been read: their words are the epilogue's */
+        if (!tile_splitk_epilogue<MB, 1, T>(acc, part, ctr, *(unsigned *)xb0))
+            return;
+    }
+    const int n = n0 + 16 * w + m16;
+    if (n < N)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + 16 * mb + 4 * g + i;
+                if (m < M)
+                    y[(int64_t)m * N + n] = acc[mb][0][i];
+            }
+}
+#ifndef F3_MIN_CHUNKS
+#define F3_MIN_CHUNKS 2 /* fewest 128-wide chunks per K split (8: 65 x 1024 x 4096 17.2 -> 26.3 us on 128-row tiles) */
+#endif
+/* What a launch of 16 mb x 128 tiles takes, in hundredths of a microsecond beside its fixed
+ * cost: rounds of workgroups times chunks, at 2.66 us a chunk of 128 rows of x and 1.55 of 64,
+ * and the meeting of a K split, 6 and 4 us. Fitted on both tiles measured at 300 x 5000 x 1024
+ * (128 rows split twice 21.1 us, 64 rows unsplit 15.3), 512 x 2048 x 2048 (21.4, 20.1),
+ * 96 x 4096 x 4096 (27.3, 18.6), 256 x 4096 x 4096 (31.2, 31.7), 128 x 14336 x 4096 (49.6, 53.1)
+ * and 200 x 4096 x 14336 (79.2, 91.1): it picks the faster one at each. */
+static inline int64_t f3_cost(int mb, int M, int N, int K) {
+    const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 16 * mb - 1) / (16 * mb)), cus = glint_cu_count();
+    const int nc = K >> 7, cps = glint_split_kps(tiles, cus, nc, F3_MIN_CHUNKS);
+    const int64_t ks = (nc + cps - 1) / cps, rounds = (tiles * ks + cus - 1) / cus;
+    return rounds * cps * (mb == 8 ? 266 : 155) + (ks > 1 ? (mb == 8 ? 600 : 400) : 0);
+}
+/* Returns 1 where the shape does not fit (the caller takes the f32 LDS tiles), else 0 or -3. */
+#ifndef F3_ON
+#define F3_ON 1
+#endif
+template <int MB>
+static int htile_launch_f3(const uint8_t *hole, const uint8_t *plug, const float *absmax, const void *x, float *y, int M,
+                           int N, int K, hipStream_t st, const GlintSplitWs *fixed) {
+    constexpr int BM = 16 * MB;
+    if (!F3_ON || K % 128 != 0 || (int64_t)BM * K * 2 >= (int64_t)RD_OOR || (int64_t)128 * (K / 2) >= (int64_t)RD_OOR)
+        return 1;
+    const unsigned gx = (unsigned)((N + 127) / 128), gy = (unsigned)((M + BM - 1) / BM);
+    if (gy > 65535u)
+        return 1;
+    int cps, ks;
+    GlintSplitWs ws;
+    if (!tile_split_plan(st, gx, gy, K >> 7, (size_t)BM * 128, cps, ks, ws, 1, fixed, F3_MIN_CHUNKS))
+        return -5;
+    k_htile_f3<MB><<<dim3(gx, gy, (unsigned)ks), 512, 0, st>>>(hole, plug, absmax, (const uint16_t *)x, y, M, N, K, cps,
+                                                             ws.part, ws.ctr);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
 /* k_htile_rl (k_htile_rd) over an M <= 64 prefill, BF16 out, or f32 out (F32: k_htile_rl3). Returns 1 where the shape does not fit (K % 128 != 0, offsets beyond 31 bits; the
  * caller takes the LDS tiles), -5 where a `fixed` workspace is too small for the split plan,
  * else 0 or -3. */
@@ -1888,8 +2163,8 @@ static int htile_launch_rd(const uint8_t *hole, const uint8_t *plug, const float
     return htile_launch_rd_mb<4, F32>(hole, plug, absmax, xb, y, M, N, K, st, fixed);
 }
 
-/* f32 output at M > 1 (the reference ABI's prefill use): 3-plane k_tile_mfma, whose
- * products are exact and whose sums are f32. 128 x 128 tiles over 8 waves (2 x 4, wave tile
+/* f32 output at M > 1 where K % 128 == 64 (else k_htile_rl3 and k_htile_f3 take it): 3-plane
+ * k_tile_mfma, whose products are exact and whose sums are f32. 128 x 128 tiles over 8 waves (2 x 4, wave tile
  * 64 x 32) fill the 160 KiB of LDS: x 32 KiB, three W planes 96 KiB, cell table 32 KiB;
  * below 128 rows 64 x 128 tiles (8 waves in a row, wave tile 64 x 16), or 64 x 64 over 4
  * waves where those would leave CUs idle (4096 x 14336 at M = 64: 78.5 -> 61.6 us). */
@@ -1968,6 +2243,7 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
         const int rc = htile_launch_gemv_cu<OUT_BF16>(hole, plug, absmax, x, y, N, K, st);
         return rc != 1 ? rc : htile_launch_gemv_xreg<OUT_BF16>(hole, plug, absmax, x, y, N, K, st);
     }
+    int f3 = 1; /* f32 out above 64 rows: k_htile_f3's code, 1 where it does not take the shape */
     if (mfma_ok && OUT_BF16) {
         const GlintTileProducer p{(const glint_u32x2 *)hole, (const glint_u32x2 *)plug, absmax, N, K, nullptr};
         const uint16_t *xb = (const uint16_t *)x;
@@ -1999,6 +2275,11 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
                                                                                                        K, st, fixed);
         if (!planned)
             return -5;
+    } else if (mfma_ok && M > 64 &&
+               (f3 = f3_cost(8, M, N, K) <= f3_cost(4, M, N, K)
+                         ? htile_launch_f3<8>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)
+                         : htile_launch_f3<4>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)) != 1) {
+        return f3;
     } else if (mfma_ok) {
         const GlintTileProducer p{(const glint_u32x2 *)hole, (const glint_u32x2 *)plug, absmax, N, K, nullptr};
         const uint16_t *xb = (const uint16_t *)x;

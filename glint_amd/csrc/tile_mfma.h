@@ -1161,9 +1161,10 @@ static inline int glint_split_kps(int64_t tiles, int64_t slots, int nK, int min_
  * workspace that is too small the plan is refused instead (returns false), so the caller
  * can report it. */
 static inline bool tile_split_plan(hipStream_t st, unsigned gx, unsigned gy, int nS, size_t tile_floats, int &kps,
-                                   int &ks, GlintSplitWs &ws, int per_cu = 1, const GlintSplitWs *fixed = nullptr) {
+                                   int &ks, GlintSplitWs &ws, int per_cu = 1, const GlintSplitWs *fixed = nullptr,
+                                   int min_steps = TILE_SPLIT_MIN_STEPS) {
     const int64_t tiles = (int64_t)gx * gy;
-    kps = glint_split_kps(tiles, (int64_t)per_cu * glint_cu_count(), nS, TILE_SPLIT_MIN_STEPS);
+    kps = glint_split_kps(tiles, (int64_t)per_cu * glint_cu_count(), nS, min_steps);
     ks = (nS + kps - 1) / kps;
     ws = GlintSplitWs{nullptr, nullptr, 0, 0};
     if (ks <= 1)

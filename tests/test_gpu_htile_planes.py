@@ -1,10 +1,11 @@
-"""k_htile_rl3: f32 out at 5 <= M <= 64, K % 128 == 0 (cells as three BF16 planes, the block
-scale on block sums).
+"""k_htile_rl3 (f32 out at 5 <= M <= 64, K % 128 == 0) and k_htile_f3 (M > 64): cells as three
+BF16 planes, the block scale on block sums.
 
 Against the oracle's float64 sum within (K + 2) 2^-23 sum |w x| (each block's f32 sums, one
 rounded scaling and one addition per block stay below one rounding per weight). Shapes: one,
 two and four 16-row blocks of x, a single W chunk, odd chunk counts (the last line half used),
-strips partly filled, K split over workgroups."""
+strips partly filled, K split over workgroups; above 64 rows both tile heights (64 and 128 rows
+of x), one chunk, odd chunk counts, row and column tails, split and unsplit K."""
 import numpy as np
 import pytest
 
@@ -23,7 +24,9 @@ def _inputs(M, N, K):
 
 
 SHAPES = [(5, 13, 128), (6, 1000, 384), (8, 4097, 4096), (16, 56, 2048), (17, 777, 640), (32, 300, 14464), (33, 130, 256),
-          (64, 64, 14464), (64, 1000, 2304)]
+          (64, 64, 14464), (64, 1000, 2304),
+          (65, 13, 128), (66, 1000, 384), (96, 4096, 1152), (128, 130, 256), (129, 5000, 640), (200, 257, 14464),
+          (300, 5000, 1024), (513, 4100, 256), (700, 2049, 896)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -35,7 +38,8 @@ def test_vs_float64(oracle, M, N, K):
     assert (np.abs(y - ref) <= (K + 2) * 2.0 ** -23 * asum).all()
 
 
-@pytest.mark.parametrize("M,N,K", [(5, 13, 384), (20, 100, 1152), (64, 64, 14464)])
+@pytest.mark.parametrize("M,N,K", [(5, 13, 384), (20, 100, 1152), (64, 64, 14464), (70, 40, 384), (130, 64, 14464),
+                                   (300, 5000, 256)])
 def test_special_scales(oracle, M, N, K):
     """Infinite, NaN and huge scales: NaN and infinities where the f32 restatement has them (a
     workgroup that met one goes over its K range again with weights as products), finite
