@@ -18,6 +18,8 @@
  * [(l / 16) * 16, +16) of A (and the same for B's row = output column); the 4 int32
  * results of lane l are D[(l / 16) * 4 + i][l % 16], i = 0..3.
  */
+#include <type_traits>
+
 #include "glint_common.h"
 #include "int8_mma_gemm.h"
 
@@ -763,24 +765,43 @@ __global__ __launch_bounds__(512) void k_int8_gemm_dma5(const int8_t *__restrict
 
 /* The attach ABI's W8A8 GEMM on the same 256 x 256 DMA ring (int8_mma_gemm at the shapes
  * with at least 3/4 as many 256 x 256 tiles as CUs). Per 64-slice kb the wave's 32 MFMAs
- * run with zero C (ic = the slice's exact int32 dot products), and each A tile's 4 results
- * go straight into the f32 accumulators as acc = fma((float)ic * sx[m, kb], sw[n, kb], acc)
- * (kb ascending: bit-identical to the 64 x 64 kernel). A third ring carries the slice's
- * scales: 256 sx (rows of the tile) and 256 sw (columns), one 4-byte DMA per wave per step
- * (waves 0-3 rows, 4-7 columns). That epilogue is 3 VALU ops per output per slice (convert,
- * multiply, fused multiply-add) against one MFMA per 16 x 16 x 64, so the kernel is
- * VALU-bound: at 2048 x 8192 x 8192 about 164 us of VALU issue on 256 CUs.
+ * give ic, the slice's exact int32 dot products, and each result goes straight into its f32
+ * accumulator as acc = fma(RN((float)ic * sx[m, kb]), sw[n, kb], acc), kb ascending
+ * (bit-identical to the 64 x 64 kernel). A third ring carries the slice's scales, one 4-byte
+ * DMA per wave per step (waves 0-3 W rows, 4-7 x rows).
+ *
+ * Two VALU ops per output and slice, with no convert. The MFMAs start from C = 2^20, so the
+ * int32 result is ic + 2^20, in [0, 2^21] (|ic| <= 64 * 128 * 127 < 2^20): read as f32 bits it
+ * is the subnormal (ic + 2^20) 2^-149, exactly. With S = sx 2^120 and P = -2^20 2^-149 S (both
+ * exact), fma(that, S, P) rounds ic sx 2^-29 once: RN((float)ic * sx) times 2^-29. The
+ * accumulators carry the 2^-29 (undone at the store), and every step is the plain form's scaled
+ * by it, exactly, as long as nothing leaves the f32 range or loses bits to subnormals. That
+ * holds for sx in [2^-36, 2^7) and |sw| zero or in the same range: then S < 2^127; a nonzero
+ * ic sx 2^-29 is at least 2^-65; acc is a multiple of ulp(2^-36)^2 = 2^-118, so acc 2^-29 is a
+ * multiple of 2^-147, which f32 holds at any magnitude. A workgroup that met another scale goes
+ * over its tile again with the convert, the multiply and the fused multiply-add.
+ * W rows are the MFMA's rows and x rows its columns, so a lane's S and P are four pairs per
+ * slice (against 32 the other way around), its 4 results are consecutive outputs of one x row
+ * and leave in 16-byte stores.
+ * Bound: a slice's chain of barrier, fragment reads, MFMAs and FMAs at two waves per SIMD, on
+ * matrix and vector instructions that do not overlap there (per slice and SIMD 64 MFMAs and 512
+ * FMAs). Against the form with the convert (whole call, one box): 2048 x 8192 x 8192 269 -> 256 us,
+ * 4096 x 14336 x 4096 502 -> 475, 2047 x 8192 x 3072 109.6 -> 104.0. Two 256 x 128 workgroups of
+ * four waves per CU in place of one of eight were slower (288 us at 2048 x 8192 x 8192).
  * ACCUM stores y + acc (the second pass of the two-pass forms). Offsets are 32-bit:
  * M K, N K, M K / 16 and N K / 16 < 2^31 (the host checks). */
+#define Q_SC_LO 0x2D800000u /* f32 bits of 2^-36 */
+#define Q_SC_HI 0x43000000u /* 2^7 */
 template <bool ACCUM>
 __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
-                                                      const float *__restrict__ sx, const float *__restrict__ sw,
-                                                      float *__restrict__ y, int M, int N, int K) {
+                                                      const float *__restrict__ sw, const float *__restrict__ sx,
+                                                      float *__restrict__ y, int M, int N, int K, int vec) {
+    /* A: W [M, K] with scales sw; B: the quantized x [N, K] with scales sx; y [N, M] */
     __shared__ __attribute__((aligned(16))) int8_t sA0[G2_BM * G2_LDS_ROW], sA1[G2_BM * G2_LDS_ROW],
         sA2[G2_BM * G2_LDS_ROW], sA3[G2_BM * G2_LDS_ROW];
     __shared__ __attribute__((aligned(16))) int8_t sB0[G2_BN * G2_LDS_ROW], sB1[G2_BN * G2_LDS_ROW],
         sB2[G2_BN * G2_LDS_ROW], sB3[G2_BN * G2_LDS_ROW];
-    /* scales of a slice: [0, 256) sx of the tile's rows, [256, 512) sw of its columns */
+    /* scales of a slice: [0, 256) sw of the tile's W rows, [256, 512) sx of its x rows */
     __shared__ __attribute__((aligned(16))) float sS0[512], sS1[512], sS2[512], sS3[512];
     auto bufA = [&](int i) { return i == 0 ? sA0 : (i == 1 ? sA1 : (i == 2 ? sA2 : sA3)); };
     auto bufB = [&](int i) { return i == 0 ? sB0 : (i == 1 ? sB1 : (i == 2 ? sB2 : sB3)); };
@@ -788,23 +809,16 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
     constexpr int NW = 8, WNW = 4, TM = 8, TN = 4, RPW = 32, QN = 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WNW, wn = wave % WNW;
-    const int m0 = blockIdx.y * G2_BM, n0 = blockIdx.x * G2_BN;
+    const int m0 = blockIdx.x * G2_BM, n0 = blockIdx.y * G2_BN;
     const int nkb = K / 64;
     float acc[TM][TN][4];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[a][b][i] = 0.0f;
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void *)A, (short)0, (int)((uint32_t)M * (uint32_t)K), GLINT_BUF_DWORD3);
     const __amdgpu_buffer_rsrc_t rb =
         __builtin_amdgcn_make_buffer_rsrc((void *)B, (short)0, (int)((uint32_t)N * (uint32_t)K), GLINT_BUF_DWORD3);
     const __amdgpu_buffer_rsrc_t rs = wave < 4
-        ? __builtin_amdgcn_make_buffer_rsrc((void *)sx, (short)0, (int)((uint32_t)M * (uint32_t)nkb * 4u), GLINT_BUF_DWORD3)
-        : __builtin_amdgcn_make_buffer_rsrc((void *)sw, (short)0, (int)((uint32_t)N * (uint32_t)nkb * 4u), GLINT_BUF_DWORD3);
+        ? __builtin_amdgcn_make_buffer_rsrc((void *)sw, (short)0, (int)((uint32_t)M * (uint32_t)nkb * 4u), GLINT_BUF_DWORD3)
+        : __builtin_amdgcn_make_buffer_rsrc((void *)sx, (short)0, (int)((uint32_t)N * (uint32_t)nkb * 4u), GLINT_BUF_DWORD3);
     uint32_t avo[QN], bvo[QN];
 #pragma unroll
     for (int q = 0; q < QN; ++q) {
@@ -832,6 +846,9 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
                                                  4, svo, kc * 4u, 0, 0);
     };
     const int fr_ofs = g2_lds_ofs(lane & 15, lane >> 4);
+    glint_i32x4 c20 = glint_i32x4{1 << 20, 1 << 20, 1 << 20, 1 << 20};
+    asm volatile("" : "+v"(c20)); /* in registers once, not set again before every MFMA */
+    uint32_t far = 0; /* how far the scales met lie above 2^-36, in f32 bits */
     auto step = [&](int kb, int u) {
         /* own loads of step kb landed (later steps' 2 QN + 1 each remain), own reads of step
          * kb - 1 done; then the barrier with global-only fences (see k_int8_gemm_dma) */
@@ -844,39 +861,59 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
         const int8_t *ta = bufA(u), *tb = bufB(u);
         const float *ts = bufS(u);
         glint_i32x4 bf[TN];
-        float swv[TN];
+        float S[TN], P[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
             bf[b] = *(const glint_i32x4 *)(tb + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
-            swv[b] = ts[256 + wn * TN * 16 + b * 16 + (lane & 15)];
+            S[b] = ts[256 + wn * TN * 16 + b * 16 + (lane & 15)];
+        }
+        /* the wave's scales, each looked at once: 128 sw as pairs, 64 sx */
+        const glint_u32x2 cw = *(const glint_u32x2 *)(ts + wm * 128 + 2 * lane);
+        const uint32_t cx = __float_as_uint(ts[256 + wn * 64 + lane]);
+        const uint32_t c0 = cw.x & 0x7FFFFFFFu, c1 = cw.y & 0x7FFFFFFFu;
+        /* below 2^-36 the difference wraps to the top; a zero sw is taken as 2^-36 */
+        far = max(far, max(cx - Q_SC_LO, max((c0 ? c0 : Q_SC_LO) - Q_SC_LO, (c1 ? c1 : Q_SC_LO) - Q_SC_LO)));
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+            S[b] *= 0x1p120f;
+            P[b] = S[b] * -0x1p-129f;
         }
         /* A tile a's MFMAs go out before tile a - 2's epilogue, which then runs while they
-         * complete instead of waiting for its own results (2048 x 8192 x 8192: 334 -> 320 us
-         * one tile behind, 311 us two behind; three or four behind 385-392 us) */
+         * complete instead of waiting for its own results */
         constexpr int PD = 2;
         glint_i32x4 ic[PD + 1][TN];
-        glint_f32x4 sxv[PD + 1];
+        glint_f32x4 swv[PD + 1];
         auto epi = [&](int a, const glint_i32x4 (&c)[TN], const glint_f32x4 &sv) {
 #pragma unroll
             for (int b = 0; b < TN; ++b)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    acc[a][b][i] = __builtin_fmaf((float)c[b][i] * sv[i], swv[b], acc[a][b][i]);
+                for (int i = 0; i < 4; ++i) {
+                    const float t = __builtin_fmaf(__int_as_float(c[b][i]), S[b], P[b]);
+                    acc[a][b][i] = __builtin_fmaf(t, sv[i], acc[a][b][i]);
+                }
         };
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
             const glint_i32x4 af = *(const glint_i32x4 *)(ta + (wm * 128 + a * 16) * G2_LDS_ROW + fr_ofs);
-            sxv[a % (PD + 1)] = *(const glint_f32x4 *)(ts + wm * 128 + a * 16 + (lane >> 4) * 4);
+            swv[a % (PD + 1)] = *(const glint_f32x4 *)(ts + wm * 128 + a * 16 + (lane >> 4) * 4);
 #pragma unroll
             for (int b = 0; b < TN; ++b)
-                ic[a % (PD + 1)][b] = glint_mfma_i8(af, bf[b], glint_i32x4{0, 0, 0, 0});
+                ic[a % (PD + 1)][b] = glint_mfma_i8(af, bf[b], c20);
             if (a >= PD)
-                epi(a - PD, ic[(a - PD) % (PD + 1)], sxv[(a - PD) % (PD + 1)]);
+                epi(a - PD, ic[(a - PD) % (PD + 1)], swv[(a - PD) % (PD + 1)]);
+            __builtin_amdgcn_sched_barrier(0); /* without it the ring spilled, and a spill's reload waits for the DMAs */
         }
 #pragma unroll
         for (int a = TM - PD; a < TM; ++a)
-            epi(a, ic[a % (PD + 1)], sxv[a % (PD + 1)]);
+            epi(a, ic[a % (PD + 1)], swv[a % (PD + 1)]);
     };
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc[a][b][i] = 0.0f;
 #pragma unroll
     for (int i = 0; i < G3_NBUF - 1; ++i)
         dma(i, i);
@@ -890,20 +927,73 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
     for (int u = 0; u + 1 < G3_NBUF; ++u)
         if (kb + u < nkb)
             step(kb + u, u);
-    __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0); /* the ring's last (clamped) loads land first */
+    __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT_LGKM0(0)); /* the ring's last (clamped) loads land first */
+
+    /* the tile's 16-row block a: W rows r .. r + 3 of x row c */
+    auto store = [&](int a, const float (&o)[TN][4], float unscale) {
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+        for (int b = 0; b < TN; ++b) {
+            const int r = m0 + wm * 128 + a * 16 + (lane >> 4) * 4;
+            const int c = n0 + wn * TN * 16 + b * 16 + (lane & 15);
+            float *dst = y + (int64_t)c * M + r;
+            if (vec) { /* M % 4 == 0 and y 16-byte aligned */
+                if (r < M && c < N) {
+                    glint_f32x4 v = glint_f32x4{o[b][0] * unscale, o[b][1] * unscale, o[b][2] * unscale, o[b][3] * unscale};
+                    if (ACCUM)
+                        v += *(const glint_f32x4 *)dst;
+                    *(glint_f32x4 *)dst = v;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (r + i < M && c < N)
+                        dst[i] = ACCUM ? dst[i] + o[b][i] * unscale : o[b][i] * unscale;
+            }
+        }
+    };
+    uint32_t *flag = (uint32_t *)sS0;
+    __syncthreads();
+    const bool wbad = __any(far >= Q_SC_HI - Q_SC_LO);
+    if (lane == 0)
+        flag[wave] = wbad;
+    __syncthreads();
+    const glint_u32x4 f0 = ((const glint_u32x4 *)flag)[0], f1 = ((const glint_u32x4 *)flag)[1];
+    if (__builtin_expect((f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) == 0u, 1)) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+            store(a, acc[a], 0x1p29f);
+        return;
+    }
+    /* the tile once more with the convert, one 16-row block of W at a time (a second set of 128
+     * accumulators made the compiler spill in the ring) */
+#pragma unroll 1
+    for (int a = 0; a < TM; ++a) {
+        float ax[TN][4];
 #pragma unroll
         for (int b = 0; b < TN; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = m0 + wm * 128 + a * 16 + (lane >> 4) * 4 + i;
-                const int c = n0 + wn * TN * 16 + b * 16 + (lane & 15);
-                if (r < M && c < N) {
-                    float *dst = y + (int64_t)r * N + c;
-                    *dst = ACCUM ? *dst + acc[a][b][i] : acc[a][b][i];
-                }
+            for (int i = 0; i < 4; ++i)
+                ax[b][i] = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < nkb; ++k) {
+            __syncthreads(); /* the flags, then the last slice, have been read */
+            dma(k, 0);
+            __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0);
+            __syncthreads();
+            const glint_i32x4 af = *(const glint_i32x4 *)(sA0 + (wm * 128 + a * 16) * G2_LDS_ROW + fr_ofs);
+            const glint_f32x4 sv = *(const glint_f32x4 *)(sS0 + wm * 128 + a * 16 + (lane >> 4) * 4);
+#pragma unroll
+            for (int b = 0; b < TN; ++b) {
+                const glint_i32x4 bf = *(const glint_i32x4 *)(sB0 + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
+                const float S = sS0[256 + wn * TN * 16 + b * 16 + (lane & 15)];
+                const glint_i32x4 ic = glint_mfma_i8(af, bf, glint_i32x4{0, 0, 0, 0});
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    ax[b][i] = __builtin_fmaf((float)ic[i] * S, sv[i], ax[b][i]);
             }
+        }
+        store(a, ax, 1.0f);
+    }
 }
 
 /* The attach ABI's W8A8 GEMM for the shapes with few 256 x 256 tiles (small m: a decode or
@@ -1236,8 +1326,8 @@ template <bool PLUG, bool ACCUM>
 static void q_launch_gemm(const int8_t *xq, const float *sx, const int8_t *wq, const float *sw, float *y, int m,
                           int n, int k_in, const uint8_t *pq4, const float *psc, hipStream_t st) {
     if (!PLUG && g2_pays(m, n) && g3_fits(m, n, k_in)) {
-        k_int8_mma_dma<ACCUM><<<dim3((n + G2_BN - 1) / G2_BN, (m + G2_BM - 1) / G2_BM), 512, 0, st>>>(
-            xq, wq, sx, sw, y, m, n, k_in);
+        k_int8_mma_dma<ACCUM><<<dim3((n + G2_BM - 1) / G2_BM, (m + G2_BN - 1) / G2_BN), 512, 0, st>>>(
+            wq, xq, sw, sx, y, n, m, k_in, n % 4 == 0 && glint_aligned(y, 16));
         return;
     }
     if (!PLUG && g3_fits(m, n, k_in)) {
