@@ -171,15 +171,34 @@ def _check(rc: int, what: str) -> None:
 
 
 # ------------------------------------------------------------ tensor helpers (device)
+# A decode launch lasts 5 to 12 us on the device, so what a helper does before it counts: the
+# pointers go to ctypes as ints (argtypes convert them), the current stream's handle is read
+# without building a Stream object, and outputs come from new_empty / empty_like. Host time of
+# a call on one box: htile_bf16 10.3 -> 6.5 us, encode_f32 16.6 -> 8.5, seven
+# decode linears 76 -> 52, a K-major step 28 -> 17.
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
 def _stream(stream=None) -> ctypes.c_void_p:
     torch = _torch()
     s = torch.cuda.current_stream() if stream is None else stream
     return VP(s.cuda_stream)
+
+
+def _sh(stream) -> int:
+    """The stream's handle (of the current stream of the current device for None)."""
+    if stream is not None:
+        return stream.cuda_stream
+    torch = _TORCH or _torch()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _p(t) -> ctypes.c_void_p:
@@ -195,18 +214,28 @@ def _as_u16(t):
     raise TypeError(f"expected bf16 bits, got {t.dtype}")
 
 
+def _check_u16(t) -> None:
+    """t holds BF16 bits (_as_u16 without the view: only its data pointer is used)."""
+    torch = _TORCH or _torch()
+    d = t.dtype
+    if d is not torch.bfloat16 and d is not torch.int16 and d is not torch.uint16:
+        raise TypeError(f"expected bf16 bits, got {d}")
+
+
+def _pin_out(w, n: int, blocksize: int):
+    torch = _TORCH or _torch()
+    hole = w.new_empty((n + 1) // 2, dtype=torch.uint8)
+    return hole, torch.empty_like(hole), w.new_empty((n + blocksize - 1) // blocksize, dtype=torch.float32)
+
+
 def encode_bf16(w, blocksize: int = 64, out=None, stream=None):
     """GPU encode of a BF16 device tensor -> (hole u8, plug u8, absmax f32) device tensors."""
-    torch = _torch()
-    w = _as_u16(w).contiguous()
+    _check_u16(w)
+    w = w.contiguous()
     n = w.numel()
-    if out is None:
-        npk, nam = (n + 1) // 2, (n + blocksize - 1) // blocksize
-        out = (torch.empty(npk, dtype=torch.uint8, device=w.device), torch.empty(npk, dtype=torch.uint8, device=w.device),
-               torch.empty(nam, dtype=torch.float32, device=w.device))
-    hole, plug, am = out
-    _check(encode_lib().glint_encode_bf16_device(_p(w), n, blocksize, _p(hole), _p(plug), _p(am), _stream(stream)),
-           "glint_encode_bf16_device")
+    hole, plug, am = _pin_out(w, n, blocksize) if out is None else out
+    _check(encode_lib().glint_encode_bf16_device(w.data_ptr(), n, blocksize, hole.data_ptr(), plug.data_ptr(),
+                                                 am.data_ptr(), _sh(stream)), "glint_encode_bf16_device")
     return hole, plug, am
 
 
@@ -215,50 +244,47 @@ def encode_f32(w, blocksize: int = 64, stream=None):
     w = w.contiguous()
     assert w.dtype == torch.float32
     n = w.numel()
-    npk, nam = (n + 1) // 2, (n + blocksize - 1) // blocksize
-    hole = torch.empty(npk, dtype=torch.uint8, device=w.device)
-    plug = torch.empty(npk, dtype=torch.uint8, device=w.device)
-    am = torch.empty(nam, dtype=torch.float32, device=w.device)
-    _check(encode_lib().glint_encode_f32_device(_p(w), n, blocksize, _p(hole), _p(plug), _p(am), _stream(stream)),
-           "glint_encode_f32_device")
+    hole, plug, am = _pin_out(w, n, blocksize)
+    _check(encode_lib().glint_encode_f32_device(w.data_ptr(), n, blocksize, hole.data_ptr(), plug.data_ptr(),
+                                                am.data_ptr(), _sh(stream)), "glint_encode_f32_device")
     return hole, plug, am
 
 
 def expand_f32(hole, plug, absmax, n: int, blocksize: int = 64, out=None, stream=None):
-    torch = _torch()
-    out = torch.empty(n, dtype=torch.float32, device=hole.device) if out is None else out
-    _check(encode_lib().glint_expand_packed_to_f32_device(_p(hole), _p(plug), _p(absmax), n, blocksize, _p(out),
-                                                          _stream(stream)), "glint_expand_packed_to_f32_device")
+    out = hole.new_empty(n, dtype=_torch().float32) if out is None else out
+    _check(encode_lib().glint_expand_packed_to_f32_device(hole.data_ptr(), plug.data_ptr(), absmax.data_ptr(), n,
+                                                          blocksize, out.data_ptr(), _sh(stream)),
+           "glint_expand_packed_to_f32_device")
     return out
 
 
 def expand_bf16(hole, plug, absmax, n: int, blocksize: int = 64, out=None, stream=None):
-    torch = _torch()
-    out = torch.empty(n, dtype=torch.bfloat16, device=hole.device) if out is None else out
-    _check(encode_lib().glint_expand_packed_to_bf16_device(_p(hole), _p(plug), _p(absmax), n, blocksize, _p(out),
-                                                           _stream(stream)), "glint_expand_packed_to_bf16_device")
+    out = hole.new_empty(n, dtype=_torch().bfloat16) if out is None else out
+    _check(encode_lib().glint_expand_packed_to_bf16_device(hole.data_ptr(), plug.data_ptr(), absmax.data_ptr(), n,
+                                                           blocksize, out.data_ptr(), _sh(stream)),
+           "glint_expand_packed_to_bf16_device")
     return out
 
 
 def htile_f32(hole, plug, absmax, x, N: int, K: int, blocksize: int = 64, out=None, stream=None):
     """y[M, N] f32 = x[M, K] (bf16) @ W^T via launch_glint_htile_s3_f32_stream."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     M = x.numel() // K
-    y = torch.empty((M, N), dtype=torch.float32, device=x.device) if out is None else out
-    _check(encode_lib().launch_glint_htile_s3_f32_stream(_p(hole), _p(plug), _p(absmax), _p(x), _p(y), M, N, K,
-                                                         blocksize, _stream(stream)), "launch_glint_htile_s3_f32_stream")
+    y = x.new_empty((M, N), dtype=_TORCH.float32) if out is None else out
+    _check(encode_lib().launch_glint_htile_s3_f32_stream(hole.data_ptr(), plug.data_ptr(), absmax.data_ptr(),
+                                                         x.data_ptr(), y.data_ptr(), M, N, K, blocksize, _sh(stream)),
+           "launch_glint_htile_s3_f32_stream")
     return y
 
 
 def htile_bf16(hole, plug, absmax, x, N: int, K: int, blocksize: int = 64, out=None, stream=None):
     """y[M, N] bf16 (f32 accumulation) via launch_glint_htile_bf16_stream."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     M = x.numel() // K
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device) if out is None else out
-    _check(encode_lib().launch_glint_htile_bf16_stream(_p(hole), _p(plug), _p(absmax), _p(x), _p(y), M, N, K,
-                                                       blocksize, _stream(stream)), "launch_glint_htile_bf16_stream")
+    y = x.new_empty((M, N), dtype=_TORCH.bfloat16) if out is None else out
+    _check(encode_lib().launch_glint_htile_bf16_stream(hole.data_ptr(), plug.data_ptr(), absmax.data_ptr(),
+                                                       x.data_ptr(), y.data_ptr(), M, N, K, blocksize, _sh(stream)),
+           "launch_glint_htile_bf16_stream")
     return y
 
 
@@ -266,22 +292,22 @@ def htile_bf16(hole, plug, absmax, x, N: int, K: int, blocksize: int = 64, out=N
 def kmajor_pack(hole, plug, absmax, N: int, K: int, stream=None):
     """Row-major pin planes -> (hole_k, plug_k, scales_k) device tensors."""
     torch = _torch()
-    hk = torch.empty(K * N // 2, dtype=torch.uint8, device=hole.device)
-    pk = torch.empty(K * N // 2, dtype=torch.uint8, device=hole.device)
-    sk = torch.empty(N * K // 64, dtype=torch.float32, device=hole.device)
-    _check(encode_lib().glint_kmajor_pack(_p(hole), _p(plug), _p(absmax), N, K, _p(hk), _p(pk), _p(sk),
-                                          _stream(stream)), "glint_kmajor_pack")
+    hk = hole.new_empty(K * N // 2, dtype=torch.uint8)
+    pk = torch.empty_like(hk)
+    sk = hole.new_empty(N * K // 64, dtype=torch.float32)
+    _check(encode_lib().glint_kmajor_pack(hole.data_ptr(), plug.data_ptr(), absmax.data_ptr(), N, K, hk.data_ptr(),
+                                          pk.data_ptr(), sk.data_ptr(), _sh(stream)), "glint_kmajor_pack")
     return hk, pk, sk
 
 
 def gemv_km_fold(hole_k, scales_k, x, N: int, K: int, ksg: int = 1, y=None, part=None, stream=None):
     """Parent-only GEMV over the K-major hole: x bf16 [K] -> y f32 [N]."""
-    torch = _torch()
-    y = torch.empty(N, dtype=torch.float32, device=hole_k.device) if y is None else y
+    _check_u16(x)
+    y = hole_k.new_empty(N, dtype=_TORCH.float32) if y is None else y
     if ksg > 1 and part is None:
-        part = torch.empty(ksg * N, dtype=torch.float32, device=hole_k.device)
-    _check(encode_lib().glint_gemv_km_fold(_p(hole_k), _p(scales_k), _p(_as_u16(x)), _p(y), N, K, ksg,
-                                           _p(part) if part is not None else None, _stream(stream)),
+        part = hole_k.new_empty(ksg * N, dtype=_TORCH.float32)
+    _check(encode_lib().glint_gemv_km_fold(hole_k.data_ptr(), scales_k.data_ptr(), x.data_ptr(), y.data_ptr(), N, K,
+                                           ksg, part.data_ptr() if part is not None else None, _sh(stream)),
            "glint_gemv_km_fold")
     return y
 
@@ -290,95 +316,98 @@ def select_topk(x, nsel: int, idx=None, cnt=None, stream=None, tkey: int = 0, nf
                 slot: int = 0):
     """Kept channels of x (ascending) and their count, both on the device (the rank rule,
     and the price / relational / floor rules when tkey or nfloor is given)."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     K = x.numel()
-    idx = torch.empty(K, dtype=torch.int32, device=x.device) if idx is None else idx
-    cnt = torch.empty(1, dtype=torch.int32, device=x.device) if cnt is None else cnt
+    idx = x.new_empty(K, dtype=_TORCH.int32) if idx is None else idx
+    cnt = x.new_empty(1, dtype=_TORCH.int32) if cnt is None else cnt
     if tkey == 0 and nfloor == 0 and cnt_log is None:
-        _check(encode_lib().glint_select_topk(_p(x), K, nsel, _p(idx), _p(cnt), _stream(stream)), "glint_select_topk")
+        _check(encode_lib().glint_select_topk(x.data_ptr(), K, nsel, idx.data_ptr(), cnt.data_ptr(), _sh(stream)),
+               "glint_select_topk")
     else:
-        _check(encode_lib().glint_select_topk_ex(_p(x), K, nsel, tkey, nfloor, _p(idx), _p(cnt),
-                                                 _p(cnt_log) if cnt_log is not None else None, slot,
-                                                 _stream(stream)), "glint_select_topk_ex")
+        _check(encode_lib().glint_select_topk_ex(x.data_ptr(), K, nsel, tkey, nfloor, idx.data_ptr(), cnt.data_ptr(),
+                                                 cnt_log.data_ptr() if cnt_log is not None else None, slot,
+                                                 _sh(stream)), "glint_select_topk_ex")
     return idx, cnt
 
 
 def apply_corr_km(hole_k, plug_k, scales_k, x, idx, cnt, y, N: int, K: int, ks: int = 1, part=None, stream=None):
     """y += the plug correction over the selected channels (in place)."""
-    torch = _torch()
+    _check_u16(x)
     if ks > 1 and part is None:
-        part = torch.empty(ks * N, dtype=torch.float32, device=y.device)
-    _check(encode_lib().glint_apply_corr_km(_p(hole_k), _p(plug_k), _p(scales_k), _p(_as_u16(x)), _p(idx), _p(cnt),
-                                            _p(y), N, K, ks, _p(part) if part is not None else None,
-                                            _stream(stream)), "glint_apply_corr_km")
+        part = y.new_empty(ks * N, dtype=_TORCH.float32)
+    _check(encode_lib().glint_apply_corr_km(hole_k.data_ptr(), plug_k.data_ptr(), scales_k.data_ptr(), x.data_ptr(),
+                                            idx.data_ptr(), cnt.data_ptr(), y.data_ptr(), N, K, ks,
+                                            part.data_ptr() if part is not None else None, _sh(stream)),
+           "glint_apply_corr_km")
     return y
+
+
+def _quant_out(x, m: int, k_in: int, xq=None, sx=None):
+    """The activation scratch of m rows: int8 values and one f32 per 64 of them."""
+    xq = x.new_empty(m * k_in, dtype=_TORCH.int8) if xq is None else xq
+    sx = x.new_empty(m * (k_in // 64), dtype=_TORCH.float32) if sx is None else sx
+    return xq, sx
 
 
 def int8_mma_gemm(x, q, scale, n_out: int, k_in: int, xq=None, sx=None, stream=None):
     """The attach ABI's W8A8 GEMM: x bf16 [m, k_in] -> y f32 [m, n_out] (also returns xq, sx)."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     m = x.numel() // k_in
-    y = torch.empty((m, n_out), dtype=torch.float32, device=x.device)
-    xq = torch.empty(m * k_in, dtype=torch.int8, device=x.device) if xq is None else xq
-    sx = torch.empty(m * (k_in // 64), dtype=torch.float32, device=x.device) if sx is None else sx
+    y = x.new_empty((m, n_out), dtype=_TORCH.float32)
+    xq, sx = _quant_out(x, m, k_in, xq, sx)
     lin = Int8MmaLinear(q.data_ptr(), scale.data_ptr(), n_out, k_in)
-    _check(p7_lib().int8_mma_gemm(_p(x), lin, _p(y), m, _p(xq), _p(sx), _stream(stream)), "int8_mma_gemm")
+    _check(p7_lib().int8_mma_gemm(x.data_ptr(), lin, y.data_ptr(), m, xq.data_ptr(), sx.data_ptr(), _sh(stream)),
+           "int8_mma_gemm")
     return y, xq, sx
 
 
 def int8_tile_gemm(x, q, scale, n_out: int, k_in: int, m: Optional[int] = None, y=None, stream=None):
     """W8A16 over an INT8 pin linear: x bf16 [m, k_in] -> y f32 [m, n_out] (int8_tile_gemm_bf16).
     x, q and scale may be views at any offset; the call takes their data pointers as they are."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     m = x.numel() // k_in if m is None else m
     if y is None:
-        y = torch.empty((m, n_out), dtype=torch.float32, device=x.device)
+        y = x.new_empty((m, n_out), dtype=_TORCH.float32)
     lin = Int8PinLinear(q.data_ptr(), scale.data_ptr(), n_out, k_in)
-    _check(p7_lib().int8_tile_gemm_bf16(_p(x), lin, _p(y), m, _stream(stream)), "int8_tile_gemm_bf16")
+    _check(p7_lib().int8_tile_gemm_bf16(x.data_ptr(), lin, y.data_ptr(), m, _sh(stream)), "int8_tile_gemm_bf16")
     return y
 
 
 def int8_mma_gemm_plug(x, q, scale, plug_q4, plug_scale, n_out: int, k_in: int, fused: bool = False, stream=None):
     """The late-plug forms: two passes through int8 scratch (int8_mma_gemm_plug) or one fused
     kernel (int8_mma_gemm_plug_fused). Returns y f32 [m, n_out]."""
-    torch = _torch()
-    x = _as_u16(x)
+    _check_u16(x)
     m = x.numel() // k_in
-    y = torch.empty((m, n_out), dtype=torch.float32, device=x.device)
-    xq = torch.empty(m * k_in, dtype=torch.int8, device=x.device)
-    sx = torch.empty(m * (k_in // 64), dtype=torch.float32, device=x.device)
+    y = x.new_empty((m, n_out), dtype=_TORCH.float32)
+    xq, sx = _quant_out(x, m, k_in)
     lin = Int8MmaLinear(q.data_ptr(), scale.data_ptr(), n_out, k_in)
     lib = p7_lib()
     if fused:
-        _check(lib.int8_mma_gemm_plug_fused(_p(x), lin, _p(plug_q4), _p(plug_scale), _p(y), m, _p(xq), _p(sx),
-                                            _stream(stream)), "int8_mma_gemm_plug_fused")
+        _check(lib.int8_mma_gemm_plug_fused(x.data_ptr(), lin, plug_q4.data_ptr(), plug_scale.data_ptr(), y.data_ptr(),
+                                            m, xq.data_ptr(), sx.data_ptr(), _sh(stream)), "int8_mma_gemm_plug_fused")
     else:
-        pi8 = torch.empty(n_out * k_in, dtype=torch.int8, device=x.device)
-        _check(lib.int8_mma_gemm_plug(_p(x), lin, _p(plug_q4), _p(plug_scale), _p(y), m, _p(xq), _p(sx), _p(pi8),
-                                      _stream(stream)), "int8_mma_gemm_plug")
+        pi8 = x.new_empty(n_out * k_in, dtype=_TORCH.int8)
+        _check(lib.int8_mma_gemm_plug(x.data_ptr(), lin, plug_q4.data_ptr(), plug_scale.data_ptr(), y.data_ptr(), m,
+                                      xq.data_ptr(), sx.data_ptr(), pi8.data_ptr(), _sh(stream)), "int8_mma_gemm_plug")
     return y
 
 
 def int8_mma_gemm_resolve(x, q, scale, n_out: int, k_in: int, plug_q4=None, plug_scale=None, stream=None):
     """int8_mma_gemm_resolve: base (+ plug) plus the re-quantized activation residual.
     Returns (y, xq, sx, rq, sr)."""
+    _check_u16(x)
     torch = _torch()
-    x = _as_u16(x)
     m = x.numel() // k_in
-    dev = x.device
-    y = torch.empty((m, n_out), dtype=torch.float32, device=dev)
-    xq = torch.empty(m * k_in, dtype=torch.int8, device=dev)
-    sx = torch.empty(m * (k_in // 64), dtype=torch.float32, device=dev)
+    y = x.new_empty((m, n_out), dtype=torch.float32)
+    xq, sx = _quant_out(x, m, k_in)
     rq = torch.empty_like(xq)
     sr = torch.empty_like(sx)
-    pi8 = torch.empty(n_out * k_in, dtype=torch.int8, device=dev) if plug_q4 is not None else None
+    pi8 = x.new_empty(n_out * k_in, dtype=torch.int8) if plug_q4 is not None else None
     lin = Int8MmaLinear(q.data_ptr(), scale.data_ptr(), n_out, k_in)
-    opt = lambda t: VP(t.data_ptr()) if t is not None else VP(None)
-    _check(p7_lib().int8_mma_gemm_resolve(_p(x), lin, opt(plug_q4), opt(plug_scale), _p(y), m, _p(xq), _p(sx),
-                                          _p(rq), _p(sr), opt(pi8), _stream(stream)), "int8_mma_gemm_resolve")
+    opt = lambda t: t.data_ptr() if t is not None else None
+    _check(p7_lib().int8_mma_gemm_resolve(x.data_ptr(), lin, opt(plug_q4), opt(plug_scale), y.data_ptr(), m,
+                                          xq.data_ptr(), sx.data_ptr(), rq.data_ptr(), sr.data_ptr(), opt(pi8),
+                                          _sh(stream)), "int8_mma_gemm_resolve")
     return y, xq, sx, rq, sr
 
 
@@ -430,21 +459,20 @@ def p7_selftest():
 
 
 def int8_gemm_i32(A, B, stream=None):
-    torch = _torch()
     M, K = A.shape
     N = B.shape[0]
-    C = torch.empty((M, N), dtype=torch.int32, device=A.device)
-    _check(p7_lib().glint_int8_gemm_i32(_p(A), _p(B), _p(C), M, N, K, _stream(stream)), "glint_int8_gemm_i32")
+    C = A.new_empty((M, N), dtype=_torch().int32)
+    _check(p7_lib().glint_int8_gemm_i32(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, _sh(stream)),
+           "glint_int8_gemm_i32")
     return C
 
 
 def int8_gemm_scaled_bf16(A, B, sa, sb, out=None, stream=None):
-    torch = _torch()
     M, K = A.shape
     N = B.shape[0]
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=A.device) if out is None else out
-    _check(p7_lib().glint_int8_gemm_scaled_bf16(_p(A), _p(B), _p(sa), _p(sb), _p(out), M, N, K, _stream(stream)),
-           "glint_int8_gemm_scaled_bf16")
+    out = A.new_empty((M, N), dtype=_torch().bfloat16) if out is None else out
+    _check(p7_lib().glint_int8_gemm_scaled_bf16(A.data_ptr(), B.data_ptr(), sa.data_ptr(), sb.data_ptr(),
+                                                out.data_ptr(), M, N, K, _sh(stream)), "glint_int8_gemm_scaled_bf16")
     return out
 
 
