@@ -5,7 +5,8 @@
  *
  * k_kmajor_pack_planes — 64 rows x 64 channels per workgroup through LDS: 8-byte loads of
  *   the row-major planes, 4-byte stores of the K-major rows.
- * k_gemv_km_fold — a lane owns KM_FOLD_RPL = 8 output rows (4 B of a K-major hole row), so
+ * k_gemv_km_fold_part — the fold at 8 to 64 channels per wave, every load in flight at once.
+ * k_gemv_km_fold — longer parts: a lane owns KM_FOLD_RPL = 8 output rows (4 B of a K-major hole row), so
  *   a wave reads 256 B contiguous per channel; the 8 waves of a workgroup take 8 parts of the
  *   workgroup's channel slice (grid.y) and meet in LDS; the slices of a row block meet in
  *   the last of its workgroups to finish (arrival counters), in slice order. Per element:
@@ -15,7 +16,7 @@
  * k_select_topk — one workgroup: keys in LDS, rank thresholds by a two-level radix select
  *   (LDS histograms of the top 8 and low 7 key bits), the price / relational / floor rules,
  *   then a block scan that writes the kept channels in ascending order.
- * k_apply_corr_km — the fold kernel's mapping (KM_CORR_RPL = 8 rows per lane) over the
+ * k_apply_corr_km — the fold kernel's mapping (8 rows per lane) over the
  *   selected list (count read on the device), with the 256-entry delta table
  *   (CELLS - PARENT) in 64 lane copies.
  */
@@ -98,9 +99,6 @@ __global__ __launch_bounds__(KM_T) void k_kmajor_scales(const float *__restrict_
 static_assert(KM_U % 4 == 0 && 64 % KM_U == 0, "fold batch");
 #ifndef KM_FOLD_RPL
 #define KM_FOLD_RPL 8 /* fold: output rows per lane (8, 16 or 32) */
-#endif
-#ifndef KM_CORR_RPL
-#define KM_CORR_RPL 8 /* correction: output rows per lane (8, 16 or 32) */
 #endif
 
 __device__ __forceinline__ float km_bf16(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
@@ -301,6 +299,96 @@ __global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint8_t *__restric
     km_finish<false, RPL>(lds, tot, r0, N, y, part, ctr, gridDim.y, blockIdx.y);
 }
 
+/* The fold where a wave's part is SUB <= 64 channels (8, 16, .. 64), the split a caller takes to
+ * fill the device: the same sums in the same order as k_gemv_km_fold, which walks a part in
+ * batches of 4 channels, each waiting for its own loads (33 MB in 12 us). Here every load of the
+ * part (SUB words of the hole, SUB x values in scalar registers, the two blocks' scales it can
+ * touch) is in flight at once, before the table is filled.
+ * The table holds PARENT pairs: a byte of a hole word is the codes of two adjacent rows, so one
+ * 8-byte lookup (256 entries, 32 lane copies) and one v_perm serve two weights, and the words
+ * need no masks; one lookup per weight kept the LDS busy for 4.5 us of 14336 x 4096.
+ * A 64-block's boundary falls inside a part only where SUB does not divide 64.
+ * Bound: about 5 us of launch, first loads and the meeting of the slices, and the planes' bytes.
+ * Measured (16 slices, rotated pins): 14336 x 4096 12.2 -> 11.3 us, 1024 x 3072 7.2 -> 6.3,
+ * 8192 x 5120 12.4 -> 11.6, 5120 x 2048 7.7 -> 7.1. */
+template <int SUB>
+__global__ __launch_bounds__(KM_WG) void k_gemv_km_fold_part(const uint32_t *__restrict__ hole_k,
+                                                             const float *__restrict__ scales_k,
+                                                             const uint16_t *__restrict__ x, float *__restrict__ y,
+                                                             float *__restrict__ part, unsigned *ctr, int N) {
+    constexpr int RPL = 8, ROWS = 64 * RPL;
+    constexpr bool SPLIT = 64 % SUB != 0;
+    static_assert(SUB % 8 == 0 && SUB <= 64, "a part");
+    __shared__ __attribute__((aligned(16))) float lds[256 * 32 * 2]; /* PARENT pairs, then parts */
+    const int lane = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane8 = (uint32_t)(lane & 31) * 8u;
+    const int r0 = blockIdx.x * ROWS;
+    const int rc = min(r0 + RPL * lane, N - RPL); /* this lane's first row, clamped */
+    const int rowv = N / RPL;
+    const int c0 = (int)blockIdx.y * (SUB * KM_SUB) + q * SUB;
+    const int left = SPLIT ? 64 - (c0 & 63) : SUB; /* channels of the first block */
+    uint32_t w[SUB];
+    const uint32_t *hp = hole_k + (int64_t)c0 * rowv + rc / RPL;
+#pragma unroll
+    for (int u = 0; u < SUB; ++u)
+        w[u] = __builtin_nontemporal_load(hp + (int64_t)u * rowv);
+    float sc[SPLIT ? 2 : 1][RPL];
+    km_load<RPL>(scales_k + (int64_t)(c0 >> 6) * N + rc, sc[0]);
+    if constexpr (SPLIT) /* the block of the part's last channel */
+        km_load<RPL>(scales_k + (int64_t)((c0 + SUB - 1) >> 6) * N + rc, sc[1]);
+    uint32_t xs[SUB / 2]; /* wave-uniform */
+#pragma unroll
+    for (int k = 0; k < SUB / 8; ++k) {
+        const glint_u32x4 v = *(const glint_u32x4 *)(x + c0 + 8 * k);
+        xs[4 * k] = v.x; xs[4 * k + 1] = v.y; xs[4 * k + 2] = v.z; xs[4 * k + 3] = v.w;
+    }
+    /* 16-byte runs of two copies: entry i >> 4, codes (low nibble, high nibble) */
+    {
+        const int l4 = lane >> 4;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int e0 = 4 * q + 32 * k; /* the wave's four entries share their high nibble */
+            const float hi = kParent[e0 >> 4];
+            const glint_f32x4 lo = *(const glint_f32x4 *)(kParent + (e0 & 15));
+            const float a = l4 & 1 ? lo.y : lo.x, b = l4 & 1 ? lo.w : lo.z;
+            const float v = l4 & 2 ? b : a;
+            ((glint_f32x4 *)lds)[threadIdx.x + k * KM_WG] = glint_f32x4{v, hi, v, hi};
+        }
+    }
+    __syncthreads();
+    float tot[RPL], acc[RPL];
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+        tot[j] = acc[j] = 0.f;
+#pragma unroll
+    for (int u = 0; u < SUB; ++u) {
+        if constexpr (SPLIT)
+            if (u % 8 == 0 && u > 0 && u == left) { /* c0 is a multiple of 8 */
+#pragma unroll
+                for (int j = 0; j < RPL; ++j) {
+                    tot[j] = fmaf(acc[j], sc[0][j], tot[j]);
+                    acc[j] = 0.f;
+                    sc[0][j] = sc[1][j];
+                }
+            }
+        const float xv = (u & 1) ? glint_bf16hi(xs[u >> 1]) : glint_bf16lo(xs[u >> 1]);
+        glint_u32x2 t[4];
+        t[0] = *(const glint_u32x2 *)((const char *)lds + glint_cell_addr<0>(w[u], lane8));
+        t[1] = *(const glint_u32x2 *)((const char *)lds + glint_cell_addr<1>(w[u], lane8));
+        t[2] = *(const glint_u32x2 *)((const char *)lds + glint_cell_addr<2>(w[u], lane8));
+        t[3] = *(const glint_u32x2 *)((const char *)lds + glint_cell_addr<3>(w[u], lane8));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            acc[2 * j] = fmaf(__uint_as_float(t[j].x), xv, acc[2 * j]);
+            acc[2 * j + 1] = fmaf(__uint_as_float(t[j].y), xv, acc[2 * j + 1]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < RPL; ++j)
+        tot[j] = fmaf(acc[j], sc[0][j], tot[j]);
+    km_finish<false, RPL>(lds, tot, r0, N, y, part, ctr, gridDim.y, blockIdx.y);
+}
+
 /* y[r] = ((part[r] + part[N + r]) + ...) + part[(ks - 1) N + r], plus y[r] first when ADD. */
 template <bool ADD>
 __global__ __launch_bounds__(KM_T) void k_km_combine(const float *__restrict__ part, float *__restrict__ y, int N, int ks) {
@@ -497,70 +585,115 @@ __global__ __launch_bounds__(SEL_T) void k_select_topk(const uint16_t *__restric
  * part q as runs of consecutive list entries inside one 64-block (the list is ascending,
  * so a block's channels are adjacent). Delta = CELLS - PARENT sits in LDS as 64 lane
  * copies, addressed by the code byte (h << 4 | p). One chunk adds into y; several write
- * part[by N + r] for k_km_combine<true>. */
-template <int RPL>
-__global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint8_t *__restrict__ hole_bytes,
-                                                         const uint8_t *__restrict__ plug_bytes,
+ * part[by N + r] for k_km_combine<true>.
+ * A part is a handful of entries (6 or 7 at 411 channels in 8 chunks), each behind a chain of
+ * list entry, x and rows: taken one entry at a time that chain was the kernel. A wave takes
+ * KM_CB entries at a time: lane l loads entry l of the batch and its x, and the rows and the
+ * block scales of all of them are in flight before the first is looked up (the first batch's
+ * before the table is filled). The table comes through scalar loads. 14336 x 4096, 411 entries
+ * in 8 chunks: 9.0 -> 7.7 us; 4096 x 14336, 1433 entries: 15.6 -> 9.9; 4096 x 1024, 100 entries
+ * (two per wave): 5.0 -> 5.4. Scalar loads of the list took 9.4 us (129 registers: one workgroup
+ * per CU), batches of 4 8.0. */
+#define KM_CB 8 /* list entries in flight per wave */
+__global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restrict__ hole_k,
+                                                         const uint32_t *__restrict__ plug_k,
                                                          const float *__restrict__ scales_k,
                                                          const uint16_t *__restrict__ x, const int32_t *__restrict__ idx,
                                                          const int32_t *__restrict__ cnt, float *__restrict__ y,
                                                          float *__restrict__ part, unsigned *ctr, int N, int ks) {
-    constexpr int ROWS = 64 * RPL, NW = RPL / 8; /* rows per workgroup, code words per lane */
-    using HV = typename std::conditional<RPL == 32, glint_u32x4,
-                                         typename std::conditional<RPL == 16, glint_u32x2, uint32_t>::type>::type;
-    static_assert(RPL == 8 || RPL == 16 || RPL == 32, "rows per lane");
-    const HV *__restrict__ hole_k = (const HV *)hole_bytes, *__restrict__ plug_k = (const HV *)plug_bytes;
-    constexpr int LDSW = KM_SUB * ROWS > GLINT_LDS_CELLS64_WORDS ? KM_SUB * ROWS : GLINT_LDS_CELLS64_WORDS;
-    __shared__ __attribute__((aligned(16))) float lds[LDSW]; /* delta table, then parts */
-    /* 4 adjacent copies of an entry per 16-B store: entry hp = word / 64 */
-    for (int i = threadIdx.x; i < GLINT_LDS_CELLS64_WORDS / 4; i += KM_WG) {
-        const int hp = i >> 4;
-        const float d = (&kCells[0][0])[hp] - kParent[hp >> 4];
-        *(glint_f32x4 *)(lds + 4 * i) = glint_f32x4{d, d, d, d};
-    }
-    __syncthreads();
+    constexpr int RPL = 8, ROWS = 64 * RPL;
+    static_assert(KM_SUB * ROWS <= GLINT_LDS_CELLS64_WORDS, "parts fit the table's LDS");
+    __shared__ __attribute__((aligned(16))) float lds[GLINT_LDS_CELLS64_WORDS]; /* delta table, then parts */
     const int lane = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane4 = (uint32_t)lane * 4u;
     const int r0 = blockIdx.x * ROWS;
     const int rc = min(r0 + RPL * lane, N - RPL);
-    const int64_t rowv = N / RPL;
+    const int rowv = N / RPL;
+    /* the table's 16-byte runs of four copies, 4096 of them: a wave's 64 runs of step k hold the
+     * four entries from 4 q + 32 k on, which share their hole */
+    glint_f32x4 ce[8];
+    float pe[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        ce[k] = *(const glint_f32x4 *)(&kCells[0][0] + 4 * q + 32 * k);
+        pe[k] = kParent[(4 * q + 32 * k) >> 4];
+    }
     const int cn = cnt[0];
+    __builtin_amdgcn_sched_barrier(0);
     const int chunk = (cn + ks - 1) / ks, sub = (chunk + KM_SUB - 1) / KM_SUB;
     const int lo = blockIdx.y * chunk, hi = min(lo + chunk, cn);
     const int i0 = min(lo + q * sub, hi), i1 = min(i0 + sub, hi);
-    float tot[RPL], acc[RPL];
+    float tot[RPL], acc[RPL], scur[RPL];
 #pragma unroll
     for (int j = 0; j < RPL; ++j)
-        tot[j] = acc[j] = 0.f;
-    int cur = -1;
+        tot[j] = acc[j] = scur[j] = 0.f;
+    int cur = -1; /* block of the run in acc, whose scales are scur */
+    struct Batch {
+        uint32_t h[KM_CB], p[KM_CB];
+        float sc[KM_CB][RPL];
+        int c[KM_CB]; /* wave-uniform */
+        float xv[KM_CB];
+    } bt;
+    /* the batch from entry i on: past the part's end its last entry again (loaded, not added) */
+    auto load = [&](int i) {
+        const int cl = idx[min(i + min(lane, KM_CB - 1), i1 - 1)];
+        const float xl = km_bf16(x[cl]);
+        int prev = cur;
+#pragma unroll
+        for (int u = 0; u < KM_CB; ++u) {
+            const int c = __builtin_amdgcn_readlane(cl, u);
+            bt.c[u] = c;
+            bt.h[u] = hole_k[(int64_t)c * rowv + rc / RPL];
+            /* (past the end the plug's row comes from the hole: the plug may lie across the bus) */
+            bt.p[u] = (i + u < i1 ? plug_k : hole_k)[(int64_t)c * rowv + rc / RPL];
+            if ((c >> 6) != prev) /* a run starts: its block's scales */
+                km_load<RPL>(scales_k + (int64_t)(c >> 6) * N + rc, bt.sc[u]);
+            prev = c >> 6;
+        }
+#pragma unroll
+        for (int u = 0; u < KM_CB; ++u)
+            bt.xv[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xl), u));
+    };
     auto flush = [&]() {
-        float sc[RPL];
-        km_load<RPL>(scales_k + (int64_t)cur * N + rc, sc);
 #pragma unroll
         for (int j = 0; j < RPL; ++j) {
-            tot[j] = fmaf(acc[j], sc[j], tot[j]);
+            tot[j] = fmaf(acc[j], scur[j], tot[j]);
             acc[j] = 0.f;
         }
     };
-    for (int i = i0; i < i1; ++i) {
-        const int c = idx[i];
-        const HV hv = hole_k[(int64_t)c * rowv + rc / RPL], pv = plug_k[(int64_t)c * rowv + rc / RPL];
-        if ((c >> 6) != cur) {
-            if (cur >= 0)
-                flush();
-            cur = c >> 6;
-        }
-        const float xv = km_bf16(x[c]);
-        uint32_t Hs[NW], Ps[NW];
-        __builtin_memcpy(Hs, &hv, sizeof(Hs));
-        __builtin_memcpy(Ps, &pv, sizeof(Ps));
-        uint32_t E[NW], O[NW];
+    auto add = [&](int n) {
 #pragma unroll
-        for (int q = 0; q < NW; ++q) {
-            E[q] = glint_codes_even(Hs[q], Ps[q]);
-            O[q] = glint_codes_odd(Hs[q], Ps[q]);
+        for (int u = 0; u < KM_CB; ++u) {
+            if (u >= n)
+                break;
+            if ((bt.c[u] >> 6) != cur) {
+                if (cur >= 0)
+                    flush();
+                cur = bt.c[u] >> 6;
+#pragma unroll
+                for (int j = 0; j < RPL; ++j)
+                    scur[j] = bt.sc[u][j];
+            }
+            const uint32_t E[1] = {glint_codes_even(bt.h[u], bt.p[u])}, O[1] = {glint_codes_odd(bt.h[u], bt.p[u])};
+            km_lookup_fma<RPL>(lds, E, O, lane4, bt.xv[u], acc);
         }
-        km_lookup_fma<RPL>(lds, E, O, lane4, xv, acc);
+    };
+    if (i0 < i1)
+        load(i0);
+    {
+        const int l4 = lane >> 4;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float a = l4 & 1 ? ce[k].y : ce[k].x, b = l4 & 1 ? ce[k].w : ce[k].z;
+            const float d = (l4 & 2 ? b : a) - pe[k];
+            ((glint_f32x4 *)lds)[threadIdx.x + k * KM_WG] = glint_f32x4{d, d, d, d};
+        }
+    }
+    __syncthreads();
+    for (int i = i0; i < i1; i += KM_CB) {
+        if (i > i0)
+            load(i);
+        add(i1 - i);
     }
     if (cur >= 0)
         flush();
@@ -605,9 +738,25 @@ GLINT_API int glint_gemv_km_fold(const uint8_t *hole_k, const float *scales_k, c
     if (N < 32 || (N % 32) != 0 || ksg < 1 || K < 64 || (K % (64 * ksg)) != 0 || !glint_aligned(hole_k, 16) ||
         !glint_aligned(scales_k, 16) || !glint_aligned(x, 16))
         return -2;
-    const dim3 grid((N + 64 * KM_FOLD_RPL - 1) / (64 * KM_FOLD_RPL), ksg);
+    static_assert(KM_FOLD_RPL == 8, "both folds take 512 rows per workgroup");
+    const dim3 grid((N + 511) / 512, ksg);
     unsigned *ctr = ksg > 1 ? km_counters(stream, grid.x) : nullptr;
-    k_gemv_km_fold<KM_FOLD_RPL><<<grid, KM_WG, 0, stream>>>(hole_k, scales_k, x, y, part, ctr, N, K / ksg);
+    auto parts = [&](auto sub_c) {
+        k_gemv_km_fold_part<decltype(sub_c)::value>
+            <<<grid, KM_WG, 0, stream>>>((const uint32_t *)hole_k, scales_k, x, y, part, ctr, N);
+    };
+    switch (K / ksg / KM_SUB) { /* channels per wave */
+    case 8: parts(std::integral_constant<int, 8>{}); break;
+    case 16: parts(std::integral_constant<int, 16>{}); break;
+    case 24: parts(std::integral_constant<int, 24>{}); break;
+    case 32: parts(std::integral_constant<int, 32>{}); break;
+    case 40: parts(std::integral_constant<int, 40>{}); break;
+    case 48: parts(std::integral_constant<int, 48>{}); break;
+    case 56: parts(std::integral_constant<int, 56>{}); break;
+    case 64: parts(std::integral_constant<int, 64>{}); break;
+    default:
+        k_gemv_km_fold<KM_FOLD_RPL><<<grid, KM_WG, 0, stream>>>(hole_k, scales_k, x, y, part, ctr, N, K / ksg);
+    }
     if (ksg > 1 && !ctr)
         k_km_combine<false><<<(N + KM_T - 1) / KM_T, KM_T, 0, stream>>>(part, y, N, ksg);
     return km_launched();
@@ -635,10 +784,10 @@ GLINT_API int glint_apply_corr_km(const uint8_t *hole_k, const uint8_t *plug_k, 
     if (N < 32 || (N % 32) != 0 || K < 64 || (K % 64) != 0 || ks < 1 || !glint_aligned(hole_k, 16) ||
         !glint_aligned(plug_k, 16) || !glint_aligned(scales_k, 16))
         return -2;
-    const dim3 grid((N + 64 * KM_CORR_RPL - 1) / (64 * KM_CORR_RPL), ks);
+    const dim3 grid((N + 511) / 512, ks);
     unsigned *ctr = ks > 1 ? km_counters(stream, grid.x) : nullptr;
-    k_apply_corr_km<KM_CORR_RPL><<<grid, KM_WG, 0, stream>>>(hole_k, plug_k, scales_k, x, idx, cnt, y, part, ctr, N,
-                                                             ks);
+    k_apply_corr_km<<<grid, KM_WG, 0, stream>>>((const uint32_t *)hole_k, (const uint32_t *)plug_k, scales_k, x, idx, cnt,
+                                                y, part, ctr, N, ks);
     if (ks > 1 && !ctr)
         k_km_combine<true><<<(N + KM_T - 1) / KM_T, KM_T, 0, stream>>>(part, y, N, ks);
     return km_launched();
