@@ -1830,8 +1830,9 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
             }
 }
 
-/* k_htile_f3: f32 out at M > 64 (the reference ABI's prefill), bs = 64, K % 128 == 0, aligned:
- * k_htile_rl3's exact cell planes and block scaling on 16 MB x 128 output tiles.
+/* k_htile_f3: f32 out at M > 64 (the reference ABI's prefill), and above the small-M launches
+ * where K % 128 == 64; bs = 64, K % 64 == 0, aligned: k_htile_rl3's exact cell planes and block
+ * scaling on 16 MB x 128 output tiles.
  *   - Wave w of 8 owns W rows [16 w, +16) of the tile and all its 16 MB rows of x, so the three
  *     planes of a weight are made once per workgroup in the registers of the wave that multiplies
  *     them, never pass through LDS, and every x fragment read from LDS feeds three MFMAs. (Tiles
@@ -1843,14 +1844,17 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
  *   - Block sums start from zero; a block's FMAs by its scale are issued among the next block's
  *     MFMAs (two sets of sums).
  *   - K is split over gridDim.z workgroups where the tiles alone leave CUs idle.
- * Special scales as in k_htile_rl3.
+ * Special scales as in k_htile_rl3. HALF: K % 128 == 64, the last chunk has one block: nothing of
+ * its second half is loaded, neither of W nor of x.
  * Bound: the matrix cores, three planes of every product (2048 x 14336 x 4096: 1.21 PFLOP/s of
  * BF16 MFMA; a dense BF16 product of that shape by the vendor's library runs at 1.14). Measured
  * against the three-plane LDS tiles (128 x 128; rotated pins): 2048 x 14336 x 4096 762 -> 597 us,
  * 2047 x 8192 x 3072 333 -> 261, 512 x 14336 x 4096 215 -> 164, 512 x 4096 x 14336 196 -> 158,
- * 128 x 14336 x 4096 64 -> 50, 96 x 4096 x 4096 28.8 -> 18.6; relative error against 64 bits
- * 7.1e-7 -> 1.6e-7 at 2048 x 14336 x 4096. */
-template <int MB>
+ * 128 x 14336 x 4096 64 -> 50, 96 x 4096 x 4096 28.8 -> 18.6; at K % 128 == 64 (HALF)
+ * 300 x 2000 x 2112 24.9 -> 15.7, 1000 x 4096 x 4160 111 -> 90, 16 x 4096 x 4160 22.8 -> 19.0,
+ * 64 x 14336 x 4160 52 -> 40; relative error against 64 bits 7.1e-7 -> 1.6e-7 at
+ * 2048 x 14336 x 4096. */
+template <int MB, bool HALF>
 __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
                                                      const float *__restrict__ absmax, const uint16_t *__restrict__ x,
                                                      float *__restrict__ y, int M, int N, int K, int cps,
@@ -1868,7 +1872,8 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
     const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
     const int nrows = min(BN, N - n0); /* >= 1 */
     const int c0 = blockIdx.z * cps;
-    const int nj = min(K >> 7, c0 + cps) - c0; /* chunks of the split, >= 1 */
+    const int nj = min((K + 127) >> 7, c0 + cps) - c0; /* chunks of the split, >= 1 */
+    const int nb = (K >> 6) - 2 * c0;                  /* 64-blocks from the split's first chunk to the row's end */
     const uint32_t rowb = (uint32_t)K >> 1;
     const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(hole + (int64_t)n0 * rowb), (short)0, (int)((uint32_t)nrows * rowb), GLINT_BUF_DWORD3);
@@ -1889,6 +1894,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         xgo[i] = (uint32_t)r * (uint32_t)K * 2u + (uint32_t)(pc << 4);
         xlo[i] = (uint32_t)(r * 256 + ((pc ^ (r & 15)) << 4));
     }
+    const int xblk = (int)(threadIdx.x & 15) >> 3; /* the block of the thread's x pieces (T % 16 == 0) */
     struct WBlk {
         glint_u32x2 h[2], p[2]; /* [block]: the words of MFMA steps 2 b and 2 b + 1 */
         glint_f32x2 a;          /* the blocks' scales */
@@ -1900,16 +1906,24 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         const uint32_t o = j < nj ? wofs + c * 64u : RD_OOR, oa = j < nj ? aofs + c * 8u : RD_OOR;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            s.h[b] = __builtin_bit_cast(glint_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rh, o + 32u * b, 0, 0));
-            s.p[b] = __builtin_bit_cast(glint_u32x2, __builtin_amdgcn_raw_buffer_load_b64(rp, o + 32u * b, 0, 0));
+            const bool in = !HALF || 2 * j + b < nb;
+            s.h[b] = __builtin_bit_cast(glint_u32x2,
+                                        __builtin_amdgcn_raw_buffer_load_b64(rh, in ? o + 32u * b : RD_OOR, 0, 0));
+            s.p[b] = __builtin_bit_cast(glint_u32x2,
+                                        __builtin_amdgcn_raw_buffer_load_b64(rp, in ? o + 32u * b : RD_OOR, 0, 0));
+            if constexpr (HALF) /* the scale behind a row's last block is another row's */
+                s.a[b] = __uint_as_float(
+                    __builtin_amdgcn_raw_buffer_load_b32(ra, in ? oa + 4u * b : RD_OOR, 0, 0));
         }
-        s.a = __builtin_bit_cast(glint_f32x2, __builtin_amdgcn_raw_buffer_load_b64(ra, oa, 0, 0));
+        if constexpr (!HALF)
+            s.a = __builtin_bit_cast(glint_f32x2, __builtin_amdgcn_raw_buffer_load_b64(ra, oa, 0, 0));
     };
     auto xload = [&](int j) {
         const uint32_t c = (uint32_t)(c0 + j) * 256u;
 #pragma unroll
         for (int i = 0; i < NX; ++i)
-            xr[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, j < nj ? xgo[i] + c : RD_OOR, 0, 0);
+            xr[i] = __builtin_amdgcn_raw_buffer_load_b128(
+                rx, j < nj && (!HALF || 2 * j + xblk < nb) ? xgo[i] + c : RD_OOR, 0, 0);
     };
     auto xstore = [&](uint8_t *buf) {
 #pragma unroll
@@ -2079,7 +2093,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
  * and 200 x 4096 x 14336 (79.2, 91.1): it picks the faster one at each. */
 static inline int64_t f3_cost(int mb, int M, int N, int K) {
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 16 * mb - 1) / (16 * mb)), cus = glint_cu_count();
-    const int nc = K >> 7, cps = glint_split_kps(tiles, cus, nc, F3_MIN_CHUNKS);
+    const int nc = (K + 127) >> 7, cps = glint_split_kps(tiles, cus, nc, F3_MIN_CHUNKS);
     const int64_t ks = (nc + cps - 1) / cps, rounds = (tiles * ks + cus - 1) / cus;
     return rounds * cps * (mb == 8 ? 266 : 155) + (ks > 1 ? (mb == 8 ? 600 : 400) : 0);
 }
@@ -2091,17 +2105,17 @@ template <int MB>
 static int htile_launch_f3(const uint8_t *hole, const uint8_t *plug, const float *absmax, const void *x, float *y, int M,
                            int N, int K, hipStream_t st, const GlintSplitWs *fixed) {
     constexpr int BM = 16 * MB;
-    if (!F3_ON || K % 128 != 0 || (int64_t)BM * K * 2 >= (int64_t)RD_OOR || (int64_t)128 * (K / 2) >= (int64_t)RD_OOR)
+    if (!F3_ON || K % 64 != 0 || (int64_t)BM * K * 2 >= (int64_t)RD_OOR || (int64_t)128 * (K / 2) >= (int64_t)RD_OOR)
         return 1;
     const unsigned gx = (unsigned)((N + 127) / 128), gy = (unsigned)((M + BM - 1) / BM);
     if (gy > 65535u)
         return 1;
     int cps, ks;
     GlintSplitWs ws;
-    if (!tile_split_plan(st, gx, gy, K >> 7, (size_t)BM * 128, cps, ks, ws, 1, fixed, F3_MIN_CHUNKS))
+    if (!tile_split_plan(st, gx, gy, (K + 127) >> 7, (size_t)BM * 128, cps, ks, ws, 1, fixed, F3_MIN_CHUNKS))
         return -5;
-    k_htile_f3<MB><<<dim3(gx, gy, (unsigned)ks), 512, 0, st>>>(hole, plug, absmax, (const uint16_t *)x, y, M, N, K, cps,
-                                                             ws.part, ws.ctr);
+    (K % 128 ? k_htile_f3<MB, true> : k_htile_f3<MB, false>)<<<dim3(gx, gy, (unsigned)ks), 512, 0, st>>>(
+        hole, plug, absmax, (const uint16_t *)x, y, M, N, K, cps, ws.part, ws.ctr);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -2163,8 +2177,8 @@ static int htile_launch_rd(const uint8_t *hole, const uint8_t *plug, const float
     return htile_launch_rd_mb<4, F32>(hole, plug, absmax, xb, y, M, N, K, st, fixed);
 }
 
-/* f32 output at M > 1 where K % 128 == 64 (else k_htile_rl3 and k_htile_f3 take it): 3-plane
- * k_tile_mfma, whose products are exact and whose sums are f32. 128 x 128 tiles over 8 waves (2 x 4, wave tile
+/* f32 output at M > 1 where k_htile_f3's 31-bit offsets do not reach: 3-plane k_tile_mfma, whose
+ * products are exact and whose sums are f32. 128 x 128 tiles over 8 waves (2 x 4, wave tile
  * 64 x 32) fill the 160 KiB of LDS: x 32 KiB, three W planes 96 KiB, cell table 32 KiB;
  * below 128 rows 64 x 128 tiles (8 waves in a row, wave tile 64 x 16), or 64 x 64 over 4
  * waves where those would leave CUs idle (4096 x 14336 at M = 64: 78.5 -> 61.6 us). */
@@ -2243,7 +2257,7 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
         const int rc = htile_launch_gemv_cu<OUT_BF16>(hole, plug, absmax, x, y, N, K, st);
         return rc != 1 ? rc : htile_launch_gemv_xreg<OUT_BF16>(hole, plug, absmax, x, y, N, K, st);
     }
-    int f3 = 1; /* f32 out above 64 rows: k_htile_f3's code, 1 where it does not take the shape */
+    int f3 = 1; /* f32 out: k_htile_f3's code, 1 where it does not take the shape */
     if (mfma_ok && OUT_BF16) {
         const GlintTileProducer p{(const glint_u32x2 *)hole, (const glint_u32x2 *)plug, absmax, N, K, nullptr};
         const uint16_t *xb = (const uint16_t *)x;
@@ -2275,7 +2289,7 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
                                                                                                        K, st, fixed);
         if (!planned)
             return -5;
-    } else if (mfma_ok && M > 64 &&
+    } else if (mfma_ok && M > 1 &&
                (f3 = f3_cost(8, M, N, K) <= f3_cost(4, M, N, K)
                          ? htile_launch_f3<8>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)
                          : htile_launch_f3<4>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)) != 1) {

@@ -5,7 +5,7 @@ Against the oracle's float64 sum within (K + 2) 2^-23 sum |w x| (each block's f3
 rounded scaling and one addition per block stay below one rounding per weight). Shapes: one,
 two and four 16-row blocks of x, a single W chunk, odd chunk counts (the last line half used),
 strips partly filled, K split over workgroups; above 64 rows both tile heights (64 and 128 rows
-of x), one chunk, odd chunk counts, row and column tails, split and unsplit K."""
+of x), one chunk, odd chunk counts, a last chunk of one 64-block, row and column tails, split and unsplit K."""
 import numpy as np
 import pytest
 
@@ -26,7 +26,9 @@ def _inputs(M, N, K):
 SHAPES = [(5, 13, 128), (6, 1000, 384), (8, 4097, 4096), (16, 56, 2048), (17, 777, 640), (32, 300, 14464), (33, 130, 256),
           (64, 64, 14464), (64, 1000, 2304),
           (65, 13, 128), (66, 1000, 384), (96, 4096, 1152), (128, 130, 256), (129, 5000, 640), (200, 257, 14464),
-          (300, 5000, 1024), (513, 4100, 256), (700, 2049, 896)]
+          (300, 5000, 1024), (513, 4100, 256), (700, 2049, 896),
+          # K % 128 == 64: half a last chunk (one block in all at K = 64), split and not
+          (9, 300, 64), (16, 4096, 1088), (33, 130, 4160), (65, 13, 192), (130, 257, 14400), (300, 5000, 320)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -39,7 +41,7 @@ def test_vs_float64(oracle, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(5, 13, 384), (20, 100, 1152), (64, 64, 14464), (70, 40, 384), (130, 64, 14464),
-                                   (300, 5000, 256)])
+                                   (300, 5000, 256), (70, 40, 448)])
 def test_special_scales(oracle, M, N, K):
     """Infinite, NaN and huge scales: NaN and infinities where the f32 restatement has them (a
     workgroup that met one goes over its K range again with weights as products), finite
