@@ -1484,9 +1484,11 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
  *     W row, so a block's sums (4 per lane and 16 rows of x) take one FMA by the lane's scale.
  *     x times a plane is exact; the f32 sums of a block, one rounded product with the scale and
  *     one addition per block are all the roundings there are.
- *   - A workgroup that met a scale that is infinite, NaN or at least 2^126 goes over its split
- *     again with the products w = cell * absmax split as GlintTileProducer::finish_split does,
- *     so infinities of both signs meet as they do in a sum of weights.
+ *   - A workgroup that met a scale that is infinite, NaN or at least 2^126, or whose sums came out
+ *     infinite or NaN (an infinite or NaN x, or x so large that a block's unscaled sum overflows),
+ *     goes over its split again with the products w = cell * absmax split as
+ *     GlintTileProducer::finish_split does, so infinities of both signs meet as they do in a sum
+ *     of weights; there only the hi plane meets infinities and NaNs of x.
  * Bound: a step's chain of LDS reads, lookups and MFMAs at two waves per SIMD, as k_htile_rl.
  * Measured against the per-weight split (rotated pins):
  * 14336 x 4096 M = 5 30.6 (as two small-M launches) -> 21.0 us, 8 30.0 -> 21.0, 32 33.9 -> 26.1,
@@ -1514,6 +1516,28 @@ __device__ __forceinline__ glint_u32x2 rl_entry(float cell) {
     uint32_t o[3];
     rl_split3(cell, false, o);
     return glint_u32x2{(o[0] >> 16) | o[1], o[2] >> 16};
+}
+/* x with its infinities and NaNs as zeros: what the planes below hi meet, since infinity times a
+ * plane that is 0 is not the product's value (hi is 0 only where the weight is) */
+__device__ __forceinline__ glint_bf16x8 rl_finite(glint_bf16x8 x) {
+    glint_u32x4 v = __builtin_bit_cast(glint_u32x4, x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t e = v[i] & 0x7F807F80u;
+        v[i] &= (e >> 16 == 0x7F80u ? 0u : 0xFFFF0000u) | ((e & 0xFFFFu) == 0x7F80u ? 0u : 0xFFFFu);
+    }
+    return __builtin_bit_cast(glint_bf16x8, v);
+}
+/* any output of the lane infinite or NaN */
+template <int MB>
+__device__ __forceinline__ bool rl_nonfinite(const glint_f32x4 (&acc)[MB][1]) {
+    bool bad = false;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            bad |= !(__builtin_fabsf(acc[mb][0][i]) < __builtin_inff());
+    return bad;
 }
 template <int MB>
 __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
@@ -1695,7 +1719,8 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
                     t[b][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        af[mb], bp[pl], i < 2 && pl == NP - 1 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb], 0, 0, 0);
+                        scaled && pl > 0 ? rl_finite(af[mb]) : af[mb], bp[pl],
+                        i < 2 && pl == NP - 1 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb], 0, 0, 0);
         }
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -1785,12 +1810,12 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
             step(X + u, u);
     __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0); /* the trailing dropped loads */
     /* the strip's two partials meet in xb0 (the x buffers are free); the waves' largest scales
-     * in xb1 tell whether the workgroup has to run again */
+     * and their sums, in xb1, tell whether the workgroup has to run again */
     float *red = (float *)xb0;
     uint32_t *wmax = (uint32_t *)xb1;
     static_assert(STRIPS * 64 * MB * 4 * 4 <= XCH, "partials fit an x buffer");
     auto meet = [&]() -> bool {
-        const bool big = __any(amax >= 0x7E800000u); /* 2^126, infinite or NaN */
+        const bool big = __any(amax >= 0x7E800000u || rl_nonfinite<MB>(acc)); /* 2^126, infinite or NaN */
         __syncthreads();
         if (lane == 0)
             wmax[w] = big;
@@ -1844,7 +1869,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
  *   - Block sums start from zero; a block's FMAs by its scale are issued among the next block's
  *     MFMAs (two sets of sums).
  *   - K is split over gridDim.z workgroups where the tiles alone leave CUs idle.
- * Special scales as in k_htile_rl3. HALF: K % 128 == 64, the last chunk has one block: nothing of
+ * Special scales and x as in k_htile_rl3. HALF: K % 128 == 64, the last chunk has one block: nothing of
  * its second half is loaded, neither of W nor of x.
  * Bound: the matrix cores, three planes of every product (2048 x 14336 x 4096: 1.21 PFLOP/s of
  * BF16 MFMA; a dense BF16 product of that shape by the vendor's library runs at 1.14). Measured
@@ -1980,11 +2005,26 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
             else
                 planes(k.h[b][s], k.p[b][s], bp);
             const int pc = 8 * b + 2 * g + s;
+            auto aread = [&](int mb) {
+                return __builtin_bit_cast(glint_bf16x8,
+                                          *(const glint_u32x4 *)(xs + (16 * mb + m16) * 256 + ((pc ^ m16) << 4)));
+            };
+            if (scaled) { /* one fragment of x at a time: few registers */
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) {
+                    const glint_bf16x8 a = aread(mb), fin = rl_finite(a);
+                    glint_f32x4 v = s == 0 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb];
+                    v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fin, bp[2], v, 0, 0, 0);
+                    v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fin, bp[1], v, 0, 0, 0);
+                    t[b][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bp[0], v, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                continue;
+            }
             glint_bf16x8 af[MB];
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
-                af[mb] = __builtin_bit_cast(glint_bf16x8,
-                                            *(const glint_u32x4 *)(xs + (16 * mb + m16) * 256 + ((pc ^ m16) << 4)));
+                af[mb] = aread(mb);
 #pragma unroll
             for (int pl = 2; pl >= 0; --pl) /* the smallest plane first */
 #pragma unroll
@@ -2040,9 +2080,9 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         step(j, 0);
     add(1, ap);
 
-    /* a special scale anywhere in the workgroup: the split once more, unpipelined, with every
+    /* a special scale or sum anywhere in the workgroup: the split once more, unpipelined, with every
      * weight multiplied by its scale */
-    const bool big = __any(amax >= 0x7E800000u); /* 2^126, infinite or NaN */
+    const bool big = __any(amax >= 0x7E800000u || rl_nonfinite<MB>(acc)); /* 2^126, infinite or NaN */
     uint32_t *flag = (uint32_t *)xb0;
     __syncthreads();
     if (lane == 0)

@@ -59,3 +59,26 @@ def test_special_scales(oracle, M, N, K):
     assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isinf(y), np.isinf(want))
     fin = np.isfinite(want)
     assert (np.abs(y - ref)[fin] <= ((K + 2) * 2.0 ** -23 * asum)[fin]).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 1024, 8192), (7, 13, 384), (20, 100, 1152), (64, 64, 14464), (9, 40, 192),
+                                   (70, 40, 384), (130, 64, 14464), (70, 40, 448)])
+def test_special_x(oracle, M, N, K):
+    """Infinities and NaN in x, and rows whose block sums overflow before the scale is applied:
+    as the f32 restatement has them, and finite outputs within the bound."""
+    print(f"htile planes special x M={M} N={N} K={K}", flush=True)
+    hole, plug, am, x = _inputs(M, N, K)
+    am = np.where(am > 0, np.float32(2.0 ** -12) * am, np.float32(2.0 ** -12))
+    x = x.reshape(M, K).copy()
+    x[0, 3], x[1, K - 1], x[2, K // 2] = 0x7F80, 0xFF80, 0x7FC0
+    x[3] = 0x7F00  # 2^127
+    x = x.reshape(-1)
+    y = host(H.htile_f32(dev(hole), dev(plug), dev(am), dev(x).reshape(M, K), N, K, 64)).reshape(M, N)
+    with np.errstate(all="ignore"):
+        want = oracle.htile_f32(hole, plug, am, x, M, N, K, 64).reshape(M, N)
+        ref, asum = (a.reshape(M, N) for a in oracle.htile_f64(hole, plug, am, x, M, N, K, 64))
+    assert np.isinf(want[:2]).any() and np.isnan(want[2]).all()
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(y[np.isinf(want)], want[np.isinf(want)])
+    assert np.array_equal(np.isinf(y), np.isinf(want))
+    fin = np.isfinite(want)
+    assert (np.abs(y[fin] - ref[fin]) <= (K + 2) * 2.0 ** -23 * asum[fin]).all()
