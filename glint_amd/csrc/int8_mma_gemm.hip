@@ -772,26 +772,32 @@ __global__ __launch_bounds__(512) void k_int8_gemm_dma5(const int8_t *__restrict
  *
  * Two VALU ops per output and slice, with no convert. The MFMAs start from C = 2^20, so the
  * int32 result is ic + 2^20, in [0, 2^21] (|ic| <= 64 * 128 * 127 < 2^20): read as f32 bits it
- * is the subnormal (ic + 2^20) 2^-149, exactly. With S = sx 2^120 and P = -2^20 2^-149 S (both
- * exact), fma(that, S, P) rounds ic sx 2^-29 once: RN((float)ic * sx) times 2^-29. The
- * accumulators carry the 2^-29 (undone at the store), and every step is the plain form's scaled
- * by it, exactly, as long as nothing leaves the f32 range or loses bits to subnormals. That
- * holds for sx in [2^-36, 2^7) and |sw| zero or in the same range: then S < 2^127; a nonzero
- * ic sx 2^-29 is at least 2^-65; acc is a multiple of ulp(2^-36)^2 = 2^-118, so acc 2^-29 is a
- * multiple of 2^-147, which f32 holds at any magnitude. A workgroup that met another scale goes
- * over its tile again with the convert, the multiply and the fused multiply-add.
+ * is the subnormal (ic + 2^20) 2^-149, exactly. With S = sx 2^116 and P = -2^20 2^-149 S (both
+ * exact), fma(that, S, P) rounds ic sx 2^-33 once: RN((float)ic * sx) times 2^-33. The
+ * accumulators carry the 2^-33, and every step is the plain form's scaled by it, exactly, as
+ * long as nothing leaves the f32 range or loses bits to subnormals. That holds for sx in
+ * [2^-30, 2^11) and |sw| zero or in [2^-40, 2^60): then S < 2^127, a nonzero ic sx 2^-33 is at
+ * least 2^-63, and a slice adds multiples of ulp(2^-30) ulp(2^-40) = 2^-116 to acc, which times
+ * 2^-33 f32 holds at any magnitude. The workgroup looks over its tile's scales while the first
+ * operands are under way, in place of looking at each slice's in its turn (2048 x 8192 x 8192
+ * 236.4 -> 235.5 us, 2047 x 8192 x 3072 101.0 -> 101.5), and a tile with another scale takes the
+ * ring with the convert, the multiply and the FMA: with one in every tile 270 and 114 us (a check
+ * in the ring and the tile walked once more: 1640 and 615; without the fast form 270 and 108).
  * W rows are the MFMA's rows and x rows its columns, so a lane's S and P are four pairs per
  * slice (against 32 the other way around), its 4 results are consecutive outputs of one x row
  * and leave in 16-byte stores.
  * Bound: a slice's chain of barrier, fragment reads, MFMAs and FMAs at two waves per SIMD, on
  * matrix and vector instructions that do not overlap there (per slice and SIMD 64 MFMAs and 512
  * FMAs). Against the form with the convert (whole call, one box): 2048 x 8192 x 8192 269 -> 256 us,
- * 4096 x 14336 x 4096 502 -> 475, 2047 x 8192 x 3072 109.6 -> 104.0. Two 256 x 128 workgroups of
- * four waves per CU in place of one of eight were slower (288 us at 2048 x 8192 x 8192).
+ * 4096 x 14336 x 4096 502 -> 475, 2047 x 8192 x 3072 109.6 -> 104.0 (another box 257.9 -> 235.5 and
+ * 104.7 -> 101.5). Two 256 x 128 workgroups of four waves per CU in place of one of eight were
+ * slower (288 us at 2048 x 8192 x 8192).
  * ACCUM stores y + acc (the second pass of the two-pass forms). Offsets are 32-bit:
  * M K, N K, M K / 16 and N K / 16 < 2^31 (the host checks). */
-#define Q_SC_LO 0x2D800000u /* f32 bits of 2^-36 */
-#define Q_SC_HI 0x43000000u /* 2^7 */
+#define Q_SX_LO 0x30800000u /* f32 bits of 2^-30 */
+#define Q_SX_HI 0x45000000u /* 2^11 */
+#define Q_SW_LO 0x2B800000u /* 2^-40 */
+#define Q_SW_HI 0x5D800000u /* 2^60 */
 template <bool ACCUM>
 __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
                                                       const float *__restrict__ sw, const float *__restrict__ sx,
@@ -803,6 +809,7 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
         sB2[G2_BN * G2_LDS_ROW], sB3[G2_BN * G2_LDS_ROW];
     /* scales of a slice: [0, 256) sw of the tile's W rows, [256, 512) sx of its x rows */
     __shared__ __attribute__((aligned(16))) float sS0[512], sS1[512], sS2[512], sS3[512];
+    __shared__ __attribute__((aligned(16))) uint32_t sF[8]; /* per wave: met a scale out of range */
     auto bufA = [&](int i) { return i == 0 ? sA0 : (i == 1 ? sA1 : (i == 2 ? sA2 : sA3)); };
     auto bufB = [&](int i) { return i == 0 ? sB0 : (i == 1 ? sB1 : (i == 2 ? sB2 : sB3)); };
     auto bufS = [&](int i) { return i == 0 ? sS0 : (i == 1 ? sS1 : (i == 2 ? sS2 : sS3)); };
@@ -848,8 +855,8 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
     const int fr_ofs = g2_lds_ofs(lane & 15, lane >> 4);
     glint_i32x4 c20 = glint_i32x4{1 << 20, 1 << 20, 1 << 20, 1 << 20};
     asm volatile("" : "+v"(c20)); /* in registers once, not set again before every MFMA */
-    uint32_t far = 0; /* how far the scales met lie above 2^-36, in f32 bits */
-    auto step = [&](int kb, int u) {
+    /* slice kb's data landed and the next load out */
+    auto turn = [&](int kb, int u) {
         /* own loads of step kb landed (later steps' 2 QN + 1 each remain), own reads of step
          * kb - 1 done; then the barrier with global-only fences (see k_int8_gemm_dma) */
         __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT_LGKM0((2 * QN + 1) * (G3_NBUF - 2)));
@@ -858,24 +865,22 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "global");
         dma(kb + G3_NBUF - 1, (u + G3_NBUF - 1) % G3_NBUF);
         __builtin_amdgcn_sched_barrier(0);
+    };
+    /* slice kb from slot u, scales in range */
+    auto step = [&](int kb, int u) {
+        turn(kb, u);
         const int8_t *ta = bufA(u), *tb = bufB(u);
         const float *ts = bufS(u);
         glint_i32x4 bf[TN];
         float S[TN], P[TN];
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            bf[b] = *(const glint_i32x4 *)(tb + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
             S[b] = ts[256 + wn * TN * 16 + b * 16 + (lane & 15)];
+            bf[b] = *(const glint_i32x4 *)(tb + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
         }
-        /* the wave's scales, each looked at once: 128 sw as pairs, 64 sx */
-        const glint_u32x2 cw = *(const glint_u32x2 *)(ts + wm * 128 + 2 * lane);
-        const uint32_t cx = __float_as_uint(ts[256 + wn * 64 + lane]);
-        const uint32_t c0 = cw.x & 0x7FFFFFFFu, c1 = cw.y & 0x7FFFFFFFu;
-        /* below 2^-36 the difference wraps to the top; a zero sw is taken as 2^-36 */
-        far = max(far, max(cx - Q_SC_LO, max((c0 ? c0 : Q_SC_LO) - Q_SC_LO, (c1 ? c1 : Q_SC_LO) - Q_SC_LO)));
 #pragma unroll
         for (int b = 0; b < TN; ++b) {
-            S[b] *= 0x1p120f;
+            S[b] *= 0x1p116f;
             P[b] = S[b] * -0x1p-129f;
         }
         /* A tile a's MFMAs go out before tile a - 2's epilogue, which then runs while they
@@ -907,28 +912,63 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
         for (int a = TM - PD; a < TM; ++a)
             epi(a, ic[a % (PD + 1)], swv[a % (PD + 1)]);
     };
+    /* the same into plain accumulators, any scales */
+    auto step_plain = [&](int kb, int u) {
+        turn(kb, u);
+        const int8_t *ta = bufA(u), *tb = bufB(u);
+        const float *ts = bufS(u);
+        glint_i32x4 bf[TN];
+        float S[TN];
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+        for (int b = 0; b < TN; ++b) {
+            bf[b] = *(const glint_i32x4 *)(tb + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
+            S[b] = ts[256 + wn * TN * 16 + b * 16 + (lane & 15)];
+        }
+        constexpr int PD = 2;
+        glint_i32x4 ic[PD + 1][TN];
+        glint_f32x4 swv[PD + 1];
+        auto epi = [&](int a, const glint_i32x4 (&c)[TN], const glint_f32x4 &sv) {
 #pragma unroll
-        for (int b = 0; b < TN; ++b)
+            for (int b = 0; b < TN; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[a][b][i] = 0.0f;
+                for (int i = 0; i < 4; ++i)
+                    acc[a][b][i] = __builtin_fmaf((float)c[b][i] * S[b], sv[i], acc[a][b][i]);
+        };
 #pragma unroll
-    for (int i = 0; i < G3_NBUF - 1; ++i)
-        dma(i, i);
-    int kb = 0;
-    for (; kb + G3_NBUF <= nkb; kb += G3_NBUF) {
+        for (int a = 0; a < TM; ++a) {
+            const glint_i32x4 af = *(const glint_i32x4 *)(ta + (wm * 128 + a * 16) * G2_LDS_ROW + fr_ofs);
+            swv[a % (PD + 1)] = *(const glint_f32x4 *)(ts + wm * 128 + a * 16 + (lane >> 4) * 4);
 #pragma unroll
-        for (int u = 0; u < G3_NBUF; ++u)
-            step(kb + u, u);
-    }
+            for (int b = 0; b < TN; ++b)
+                ic[a % (PD + 1)][b] = glint_mfma_i8(af, bf[b], glint_i32x4{0, 0, 0, 0});
+            if (a >= PD)
+                epi(a - PD, ic[(a - PD) % (PD + 1)], swv[(a - PD) % (PD + 1)]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
-    for (int u = 0; u + 1 < G3_NBUF; ++u)
-        if (kb + u < nkb)
-            step(kb + u, u);
-    __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT_LGKM0(0)); /* the ring's last (clamped) loads land first */
-
+        for (int a = TM - PD; a < TM; ++a)
+            epi(a, ic[a % (PD + 1)], swv[a % (PD + 1)]);
+    };
+    auto ring = [&](auto one) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[a][b][i] = 0.0f;
+        int kb = 0;
+        for (; kb + G3_NBUF <= nkb; kb += G3_NBUF) {
+#pragma unroll
+            for (int u = 0; u < G3_NBUF; ++u)
+                one(kb + u, u);
+        }
+#pragma unroll
+        for (int u = 0; u + 1 < G3_NBUF; ++u)
+            if (kb + u < nkb)
+                one(kb + u, u);
+        __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT_LGKM0(0)); /* the ring's last (clamped) loads land first */
+    };
     /* the tile's 16-row block a: W rows r .. r + 3 of x row c */
     auto store = [&](int a, const float (&o)[TN][4], float unscale) {
 #pragma unroll
@@ -951,48 +991,51 @@ __global__ __launch_bounds__(512) void k_int8_mma_dma(const int8_t *__restrict__
             }
         }
     };
-    uint32_t *flag = (uint32_t *)sS0;
-    __syncthreads();
-    const bool wbad = __any(far >= Q_SC_HI - Q_SC_LO);
-    if (lane == 0)
-        flag[wave] = wbad;
-    __syncthreads();
-    const glint_u32x4 f0 = ((const glint_u32x4 *)flag)[0], f1 = ((const glint_u32x4 *)flag)[1];
-    if (__builtin_expect((f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) == 0u, 1)) {
+#pragma unroll
+    for (int i = 0; i < G3_NBUF - 1; ++i)
+        dma(i, i);
+    /* the tile's scales, each looked at once while the first operands are under way: those of the
+     * wave's 64 rows are adjacent in memory */
+    {
+        const uint32_t lo = wave < 4 ? Q_SW_LO : Q_SX_LO, span = wave < 4 ? Q_SW_HI - Q_SW_LO : Q_SX_HI - Q_SX_LO;
+        const int row0 = wave < 4 ? m0 + 64 * wave : n0 + 64 * (wave - 4);
+        const uint32_t first = (uint32_t)row0 * (uint32_t)nkb;
+        const uint32_t n = (uint32_t)max(min((wave < 4 ? M : N) - row0, 64), 0) * (uint32_t)nkb;
+        uint32_t far = 0;
+        auto see = [&](uint32_t v) {
+            const uint32_t c = v & 0x7FFFFFFFu;
+            far = max(far, (c ? c : lo) - lo); /* below the range it wraps to the top; zero counts as in it */
+        };
+        const int rounds = (int)(n >> 8); /* of 256, eight in flight (the last one again past the end) */
+        for (int r = 0; r < rounds; r += 8) {
+            glint_u32x4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                v[i] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rs, (first + 256u * (uint32_t)min(r + i, rounds - 1) + 4u * (uint32_t)lane) * 4u, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                see(v[i].x), see(v[i].y), see(v[i].z), see(v[i].w);
+        }
+        for (uint32_t e = ((uint32_t)rounds << 8) + (uint32_t)lane; e < n; e += 64u)
+            see(__builtin_amdgcn_raw_buffer_load_b32(rs, (first + e) * 4u, 0, 0));
+        sF[wave] = __any(far >= span);
+    }
+    __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT_LGKM0(63));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "global");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "global");
+    const glint_u32x4 f0 = ((const glint_u32x4 *)sF)[0], f1 = ((const glint_u32x4 *)sF)[1];
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) == 0u, 1)) {
+        ring(step);
 #pragma unroll
         for (int a = 0; a < TM; ++a)
-            store(a, acc[a], 0x1p29f);
-        return;
-    }
-    /* the tile once more with the convert, one 16-row block of W at a time (a second set of 128
-     * accumulators made the compiler spill in the ring) */
-#pragma unroll 1
-    for (int a = 0; a < TM; ++a) {
-        float ax[TN][4];
+            store(a, acc[a], 0x1p33f);
+    } else {
+        ring(step_plain);
 #pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                ax[b][i] = 0.0f;
-#pragma unroll 1
-        for (int k = 0; k < nkb; ++k) {
-            __syncthreads(); /* the flags, then the last slice, have been read */
-            dma(k, 0);
-            __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0);
-            __syncthreads();
-            const glint_i32x4 af = *(const glint_i32x4 *)(sA0 + (wm * 128 + a * 16) * G2_LDS_ROW + fr_ofs);
-            const glint_f32x4 sv = *(const glint_f32x4 *)(sS0 + wm * 128 + a * 16 + (lane >> 4) * 4);
-#pragma unroll
-            for (int b = 0; b < TN; ++b) {
-                const glint_i32x4 bf = *(const glint_i32x4 *)(sB0 + (wn * TN * 16 + b * 16) * G2_LDS_ROW + fr_ofs);
-                const float S = sS0[256 + wn * TN * 16 + b * 16 + (lane & 15)];
-                const glint_i32x4 ic = glint_mfma_i8(af, bf, glint_i32x4{0, 0, 0, 0});
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    ax[b][i] = __builtin_fmaf((float)ic[i] * S, sv[i], ax[b][i]);
-            }
-        }
-        store(a, ax, 1.0f);
+        for (int a = 0; a < TM; ++a)
+            store(a, acc[a], 1.0f);
     }
 }
 

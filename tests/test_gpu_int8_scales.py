@@ -1,7 +1,9 @@
-"""int8_mma_gemm on the 256 x 256 DMA tiles: its convert-free epilogue and the walk that scales
-outside [2^-36, 2^7) take. Both are the emulation's f32 operations, so every output is compared
-bit for bit: scales at the ends of the range, zero, negative, below, above, infinite and NaN, in
-some tiles only; columns not a multiple of 4 and y at an odd address (no 16-byte stores)."""
+"""int8_mma_gemm on the 256 x 256 DMA tiles: its convert-free epilogue and the plain one that a
+tile with sx outside [2^-30, 2^11) or sw outside 0 and [2^-40, 2^60) takes. Both are the
+emulation's f32 operations, so every output is compared bit for bit: scales at the ends of the
+range, zero, negative, below, above, infinite and NaN, in some tiles only; columns not a multiple
+of 4 and y at an odd address (no 16-byte stores); one scale anywhere in a tile, at every part of
+the look over it; and the time with such scales beside the time without."""
 import numpy as np
 import pytest
 
@@ -64,3 +66,57 @@ def test_scales_out_of_range(oracle, what):
     else:
         sw[300, 1] = {"sw tiny": 1e-20, "sw huge": 1e20, "sw inf": np.inf, "sw nan": np.nan}[what]
     _check(oracle, x.reshape(-1), wq, sw.reshape(-1), m, n, k, (0, 256))
+
+
+@pytest.mark.parametrize("k", [64, 256, 320, 2112])
+def test_one_scale_anywhere_in_a_tile(oracle, k):
+    """A lone tiny scale whose outputs the scaled accumulators could not hold, at another row and
+    slice in each tile: whole rounds of the look, the last round, the rest behind it."""
+    m, n, nkb = 2047, 6143, k // 64
+    print(f"int8 scales one anywhere k={k}", flush=True)
+    rng = np.random.default_rng(k)
+    x = bf16_bits(rng.normal(0, 1, m * k).astype(np.float32)).reshape(m, nkb, 64)
+    wq = rng.integers(-127, 128, n * k, dtype=np.int8)
+    sw = rng.uniform(1e-3, 2e-2, (n, nkb)).astype(np.float32)
+    for t in range(24):  # column tiles: the first and the last row of a wave's 64, slices from both ends
+        r, c = 256 * t + min((64 * t + (63 if t & 4 else 0)) % 256, n - 1 - 256 * t), (t // 8 * nkb // 2 + t % 2 * (nkb - 1)) % nkb
+        sw[r] = 0.0
+        sw[r, c] = np.float32(1.2345e-35) * (t + 1)
+    rows = []
+    for t in range(8):  # row tiles
+        r, c = min(256 * t + 64 * (t % 4) + (63 if t & 4 else 0), m - 1), (t * 5) % nkb
+        x[r] = 0
+        x[r, c] = bf16_bits((rng.normal(0, 1, 64) * 1e-33).astype(np.float32))
+        rows.append(min(r, m - 16))
+    _check(oracle, x.reshape(-1), wq, sw.reshape(-1), m, n, k, rows)
+
+
+@pytest.mark.parametrize("what", ["x tiny", "x huge", "sw tiny"])
+def test_scales_out_of_range_cost_no_second_walk(what):
+    """One such scale in every tile takes less than half as long again as none (the plain epilogue
+    measured 1.0 to 1.15 times the other; a tile walked twice is at least 2)."""
+    torch = torch_cuda()
+    m, n, k = 2048, 8192, 2048
+    print(f"int8 scales time {what}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    q = torch.randint(-127, 128, (n * k,), device="cuda", generator=g, dtype=torch.int8)
+    sw = torch.rand(n, k // 64, device="cuda", generator=g) * 0.019 + 1e-3
+    x2, sw2 = x.clone(), sw.clone()
+    if what == "sw tiny":
+        sw2[9::256, 3] = 1e-20
+    else:
+        x2[9::256, 64:128] = 1e-12 if what == "x tiny" else 1e9
+    xq, sx = torch.empty(m * k, dtype=torch.int8, device="cuda"), torch.empty(m * k // 64, device="cuda")
+
+    def us(xx, ss):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        for _ in range(20):
+            H.int8_mma_gemm(xx, q, ss, n, k, xq, sx)
+        e[1].record()
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1]) * 50
+    us(x, sw)
+    t = sorted(us(x2, sw2) / us(x, sw) for _ in range(7))
+    assert t[3] < 1.5, t
