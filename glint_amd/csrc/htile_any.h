@@ -19,7 +19,7 @@
  * additions, for BF16 out as for f32 out. Where a scale is nonzero and below 2^-90 (lo may
  * then have bits BF16 cannot hold) or an output comes out infinite or NaN (an infinite or NaN
  * scale or x, where inf * 0 of a plane is not the product's value, or an overflow), the
- * workgroup forms its outputs again with one f32 FMA per weight in k order.
+ * workgroup forms its outputs again with one f32 FMA per weight in k order (htile_any_again).
  *
  * Bound: the dequantization (about 9 VALU instructions and one LDS read per weight, once per
  * 16 MB rows of x) and the latency of a wave's 4 or 5 dependent chunks; the planes' bytes
@@ -45,21 +45,127 @@ __device__ __forceinline__ uint32_t glint_nibble(const uint8_t *pk, int64_t i) {
     return (pk[i >> 1] >> ((uint32_t)(i & 1) * 4)) & 15u;
 }
 
-/* one output by f32 FMAs in k order, w = CELLS * absmax per weight */
-__device__ __noinline__ float htile_any_scalar(const uint8_t *hole, const uint8_t *plug, const float *absmax,
-                                               const uint16_t *x, int m, int n, int K, int bs) {
-    float acc = 0.0f;
-    int64_t i = (int64_t)n * K, q = i / bs;
-    int r = (int)(i - q * bs);
-    for (int k = 0; k < K; ++k, ++i) {
-        const float w = kCells[glint_nibble(hole, i)][glint_nibble(plug, i)] * absmax[q];
-        acc = fmaf(w, __uint_as_float((uint32_t)x[(int64_t)m * K + k] << 16), acc);
-        if (++r == bs) {
-            r = 0;
+/* A workgroup's outputs v[j] (threadIdx.x + j T of the 16 NB x 16 MB tile) once more, by one f32
+ * FMA per weight in k order, w = CELLS * absmax: 128 elements of K at a time, the tile's weights
+ * and x as f32 through LDS (rows of 132 words: 16 rows' 16-byte reads lie in different banks), the
+ * next 128 loaded meanwhile. A thread brings 8 elements of a row of W and of 16 MB / 32 rows of x,
+ * read element by element where the row ends. Every thread of the workgroup calls it.
+ * Bound: the f32 FMAs and their LDS reads (3 or 4 of 16 bytes for 4 NB NA FMAs). One NaN in x, all
+ * scales 1e-35, against one thread per output walking K in global memory, and a kernel of scalar
+ * f32 FMAs on 64 x 32 LDS tiles: 17 x 3001 x 4104 98, 98 us (1349, 1352; 630, 633),
+ * 130 x 5000 x 5000 BF16 208, 410 (10420, 20700; 1070, 1070), 512 x 14336 x 4104 BF16 650, 2300
+ * (16650, 113000; 2240, 2260). */
+template <int MB, int NB>
+__device__ __forceinline__ void htile_any_again(float *lds, const uint8_t *hole, const uint8_t *plug,
+                                                const float *absmax, const uint16_t *x, int m0, int n0, int M, int N,
+                                                int K, int bs,
+                                                float (&v)[(NB * MB * 256 + 64 * ANY_KW - 1) / (64 * ANY_KW)]) {
+    constexpr int T = 64 * ANY_KW, KC = 128, ROW = KC + 4, XJ = (16 * MB + 31) / 32, NA = MB > 1 ? MB / 2 : 1;
+    static_assert(T == 512 && (MB == 1 || MB % 2 == 0), "the outputs of a thread are NB x NA of the tile's 16 x 16");
+    static_assert((16 * NB + 16 * MB) * ROW + 256 <= GLINT_LDS_CELLS64_WORDS, "the tiles fit the table's LDS");
+    float *ws = lds, *xs = ws + 16 * NB * ROW, *cells = xs + 16 * MB * ROW;
+    const int tid = (int)threadIdx.x, row = tid >> 4, k8 = 8 * (tid & 15);
+    const bool wact = row < 16 * NB;
+    int64_t e = (int64_t)min(n0 + row, N - 1) * K + k8, q = e / bs; /* the thread's next weight, its block */
+    uint32_t r = (uint32_t)(e - q * bs);                            /* and its place there */
+    const int dq = KC / bs;
+    const uint32_t dr = (uint32_t)(KC % bs);
+    uint32_t h = 0, p = 0;
+    float a[8];
+    glint_u32x4 xw[XJ];
+    auto load = [&](int k0) {
+        const int kin = min(max(K - k0 - k8, 0), 8);
+        const int nb = wact && kin > 0 ? (int)(((e + kin - 1) >> 1) - (e >> 1)) + 1 : 0; /* bytes: at most 5 */
+        uint64_t hb = 0, pb = 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+            if (i < nb) {
+                hb |= (uint64_t)hole[(e >> 1) + i] << (8 * i);
+                pb |= (uint64_t)plug[(e >> 1) + i] << (8 * i);
+            }
+        h = (uint32_t)(hb >> (4 * (e & 1)));
+        p = (uint32_t)(pb >> (4 * (e & 1)));
+        int64_t qi = q;
+        uint32_t ri = r;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            a[i] = wact && i < kin ? absmax[qi] : 0.0f;
+            if (++ri == (uint32_t)bs) {
+                ri = 0;
+                ++qi;
+            }
+        }
+        e += KC;
+        q += dq;
+        r += dr;
+        if (r >= (uint32_t)bs) {
+            r -= (uint32_t)bs;
             ++q;
         }
+#pragma unroll
+        for (int j = 0; j < XJ; ++j) {
+            const uint16_t *xp = x + (int64_t)min(m0 + row + 32 * j, M - 1) * K + k0 + k8;
+            xw[j] = glint_u32x4{0u, 0u, 0u, 0u};
+            if (row + 32 * j < 16 * MB && kin == 8)
+                xw[j] = *(const glint_u32x4_b2 *)xp;
+            else if (row + 32 * j < 16 * MB)
+                for (int i = 0; i < kin; ++i)
+                    xw[j][i >> 1] |= (uint32_t)xp[i] << (16 * (i & 1));
+        }
+    };
+    auto put = [&](int k0) {
+        const int kin = min(max(K - k0 - k8, 0), 8);
+        float w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) /* past K zeros, also under an infinite x: they change no sum */
+            w[i] = i < kin ? cells[((h >> (4 * i)) & 15u) << 4 | ((p >> (4 * i)) & 15u)] * a[i] : 0.0f;
+        if (wact) {
+            *(glint_f32x4 *)(ws + row * ROW + k8) = glint_f32x4{w[0], w[1], w[2], w[3]};
+            *(glint_f32x4 *)(ws + row * ROW + k8 + 4) = glint_f32x4{w[4], w[5], w[6], w[7]};
+        }
+#pragma unroll
+        for (int j = 0; j < XJ; ++j)
+            if (row + 32 * j < 16 * MB)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    *(glint_f32x4 *)(xs + (row + 32 * j) * ROW + k8 + 4 * i) =
+                        glint_f32x4{glint_bf16lo(xw[j][2 * i]), glint_bf16hi(xw[j][2 * i]),
+                                    glint_bf16lo(xw[j][2 * i + 1]), glint_bf16hi(xw[j][2 * i + 1])};
+    };
+    /* output j = jb NA + ja: W row 16 jb + tid % 16 and x row 16 (tid / 256 + 2 ja) + .. of the tile */
+    const float *wr = ws + (tid & 15) * ROW, *xr = xs + (16 * (tid >> 8) + 4 * ((tid & 63) >> 4) + ((tid >> 6) & 3)) * ROW;
+    const bool out = MB > 1 || tid < 256;
+#pragma unroll
+    for (int j = 0; j < NB * NA; ++j)
+        v[j] = 0.0f;
+    load(0);
+    __syncthreads(); /* the outputs of the first way have been read */
+    if (tid < 256)
+        cells[tid] = (&kCells[0][0])[tid];
+    __syncthreads();
+    for (int k0 = 0; k0 < K; k0 += KC) {
+        put(k0);
+        __syncthreads();
+        if (k0 + KC < K)
+            load(k0 + KC);
+        if (out)
+#pragma unroll 4
+            for (int k = 0; k < min(KC, K - k0); k += 4) {
+                glint_f32x4 wv[NB], xv[NA];
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    wv[j] = *(const glint_f32x4 *)(wr + 16 * j * ROW + k);
+#pragma unroll
+                for (int j = 0; j < NA; ++j)
+                    xv[j] = *(const glint_f32x4 *)(xr + 32 * j * ROW + k);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int j = 0; j < NB * NA; ++j)
+                        v[j] = fmaf(wv[j / NA][c], xv[j % NA][c], v[j]);
+            }
+        __syncthreads();
     }
-    return acc;
 }
 
 /* ODD: K is odd, so odd rows start in the middle of a byte. SB: bs < 32, more than two
@@ -385,7 +491,8 @@ __global__ __launch_bounds__(64 * ANY_KW) void k_htile_any(const uint8_t *__rest
     if (again)
         s_again = 1;
     __syncthreads();
-    again = s_again != 0;
+    if (s_again)
+        htile_any_again<MB, NB>(ltab, hole, plug, absmax, x, m0, n0, M, N, K, bs, v);
 #pragma unroll
     for (int j = 0; j < (OUTS + T - 1) / T; ++j) {
         const int o = (int)threadIdx.x + j * T;
@@ -393,11 +500,8 @@ __global__ __launch_bounds__(64 * ANY_KW) void k_htile_any(const uint8_t *__rest
             break;
         const int l = o & 63, i = (o >> 6) & 3, a = (o >> 8) % MB, b = (o >> 8) / MB;
         const int m = m0 + 16 * a + 4 * (l >> 4) + i, n = n0 + 16 * b + (l & 15);
-        if (m < M && n < N) {
-            if (again)
-                v[j] = htile_any_scalar(hole, plug, absmax, x, m, n, K, bs);
+        if (m < M && n < N)
             Out::store(y, (int64_t)m * N + n, v[j]);
-        }
     }
 }
 

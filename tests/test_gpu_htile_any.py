@@ -12,7 +12,7 @@ import pytest
 
 from glint_amd import glint_hip as H
 from oracle import glint_oracle as G
-from tests.gpu_util import bf16_bits, dev, host
+from tests.gpu_util import bf16_bits, dev, host, torch_cuda
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +91,52 @@ def test_special_values_as_the_scalar_sum(oracle, M, N, K, bs, what):
         assert (np.abs(f - ref)[fin] <= bound[fin]).all()
         assert np.array_equal(np.isnan(b), np.isnan(want))
         assert (np.abs(b - ref)[fin] <= (np.abs(ref) * 2.0 ** -8 + bound * 1.01 + 2.0 ** -133)[fin]).all()
+
+
+@pytest.mark.parametrize("M,N,K,bs", [(16, 17, 5, 2), (17, 16, 128, 32), (33, 40, 129, 32), (64, 30, 263, 48),
+                                      (65, 4111, 393, 64), (130, 4111, 264, 33), (2, 50, 777, 5), (20, 100, 999, 1 << 20)])
+def test_second_way_in_k_order(oracle, M, N, K, bs):
+    """An infinite x in the last element, and a scale below 2^-90: every workgroup forms its outputs
+    by one f32 FMA per weight in k order, bit for bit the emulation's, at the edges of its 128-wide
+    steps of K, of a thread's 8 elements and of the tiles (one and two strips of W)."""
+    print(f"htile_any second way M={M} N={N} K={K} bs={bs}", flush=True)
+    hole, plug, am, x = _inputs(M, N, K, bs, seed=2)
+    am = (am * np.float32(1e-33)).astype(np.float32)
+    am[0] = 1e-30
+    x[-1] = 0x7F80
+    f, _ = _run(M, N, K, bs, hole, plug, am, x)
+    with np.errstate(all="ignore"):
+        want = _fma_sum(oracle, hole, plug, am, x, M, N, K, bs)
+    assert np.array_equal(np.isnan(f), np.isnan(want))
+    met = ~np.isnan(want)
+    rows = np.arange(N) * K  # strips of W that met a nonzero scale: all outputs of these are the second way's
+    first, last = rows // bs, (rows + K - 1) // bs
+    tiny = np.array([(am[a:b + 1] != 0).any() for a, b in zip(first, last)])
+    met &= tiny[None, :]
+    assert met.any() and np.array_equal(f[met] + 0.0, want[met] + 0.0)
+
+
+def test_special_values_time():
+    """NaN in every row of x, and every scale below 2^-90: the second way takes less than 12 times
+    the common one (one thread per output over global memory took 150 to 300 times)."""
+    torch = torch_cuda()
+    M, N, K, bs = 130, 5000, 5000, 64
+    print("htile_any time of the second way", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    pin = H.encode_bf16((torch.randn(N * K, device="cuda", generator=g) * 0.02).to(torch.bfloat16), bs)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    xn = x.clone()
+    xn[:, 7] = float("nan")
+
+    def us(pin, x):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        for _ in range(5):
+            H.htile_bf16(*pin, x, N, K, bs)
+        e[1].record()
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1]) * 200
+    us(pin, x)
+    for other in ((pin, xn), ((pin[0], pin[1], pin[2] * 1e-33), x)):
+        t = sorted(us(*other) / us(pin, x) for _ in range(5))
+        assert t[2] < 12, t
