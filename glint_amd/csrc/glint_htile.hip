@@ -1474,7 +1474,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
 
 /* k_htile_rl3: f32 out (the reference ABI) at M <= 64: k_htile_rl's loads and x path with exact
  * f32 weights, and the block scale applied to block sums instead of to weights.
- *   - The cell table holds the cells as three BF16 planes, hi + mid + lo == cell exactly (8-byte
+ *   - The cell table holds cell 2^24 as three BF16 planes, hi + mid + lo == cell 2^24 exactly (8-byte
  *     entries, 32 copies: all 256 B of a row, so the W lines have LDS rows of their own). A
  *     weight costs half a VALU op for its code byte, one v_perm for the address, one LDS read
  *     and half a v_perm per plane; splitting w = cell * absmax per weight cost a multiply, the
@@ -1482,11 +1482,14 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
  *   - A lane takes 8 B of each 64-block of its row (16 weights), so MFMA steps 2 b and 2 b + 1 of
  *     a chunk hold block b alone. Their MFMAs start from zero, and D's column is the lane's own
  *     W row, so a block's sums (4 per lane and 16 rows of x) take one FMA by the lane's scale.
- *     x times a plane is exact; the f32 sums of a block, one rounded product with the scale and
- *     one addition per block are all the roundings there are.
+ *     x times a plane is exact, for the smallest x too (f3_entry; without the 2^24 an x of 2^-126
+ *     under a scale of 2^100 lost up to 13 bits); the f32 sums of a block, one rounded product with
+ *     the scale and one addition per block are all the roundings there are. Only a subnormal x is
+ *     added less exactly: the matrix core aligns its products as if x were 2^-126, so a product of
+ *     2^-133 may lose 7 bits (per-weight planes of w are no different there).
  *   - A workgroup that met a scale that is infinite, NaN or at least 2^126, or whose sums came out
- *     infinite or NaN (an infinite or NaN x, or x so large that a block's unscaled sum overflows),
- *     goes over its split again with the products w = cell * absmax split as
+ *     infinite or NaN (an infinite or NaN x, or x so large, from 2^97 on, that a block's unscaled
+ *     sum overflows), goes over its split again with the products w = cell * absmax split as
  *     GlintTileProducer::finish_split does, so infinities of both signs meet as they do in a sum
  *     of weights; there only the hi plane meets infinities and NaNs of x.
  * Bound: a step's chain of LDS reads, lookups and MFMAs at two waves per SIMD, as k_htile_rl.
@@ -1511,11 +1514,78 @@ __device__ __forceinline__ void rl_split3(float v, bool big, uint32_t (&o)[3]) {
     o[1] = __float_as_uint(md);
     o[2] = __float_as_uint(r1 - md);
 }
-/* a cell's table entry for f32 out: hi | mid << 16, lo */
-__device__ __forceinline__ glint_u32x2 rl_entry(float cell) {
+/* The cell table of the f32-out kernels: cell 2^24 as three planes, hi | mid << 16 and lo, in 32
+ * copies. The 2^24 makes x times a plane exact for every finite x: a cell is a multiple of 2^-36
+ * and a BF16 x of 2^-133, so the products are multiples of 2^-145, which f32 holds. */
+#define F3_UP 0x1p24f
+#define F3_DOWN 0x1p-24f
+__device__ __forceinline__ glint_u32x2 f3_entry(float cell) {
     uint32_t o[3];
-    rl_split3(cell, false, o);
+    rl_split3(cell * F3_UP, false, o);
     return glint_u32x2{(o[0] >> 16) | o[1], o[2] >> 16};
+}
+/* Its fill by 512 threads: 16-B runs of two copies; run r is cell r / 16 (a wave's 64 runs hold 4
+ * cells: scalar loads), 4096 runs in 8 steps. */
+__device__ __forceinline__ void f3_fill_load(int w, glint_f32x4 (&c4)[8]) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        c4[k] = *(const glint_f32x4 *)(&kCells[0][0] + ((64 * w + k * 512) >> 4));
+}
+__device__ __forceinline__ void f3_fill_store(uint8_t *lt, int g, const glint_f32x4 (&c4)[8]) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float lo = g & 1 ? c4[k].y : c4[k].x, hi = g & 1 ? c4[k].w : c4[k].z;
+        const glint_u32x2 e = f3_entry(g & 2 ? hi : lo);
+        ((glint_u32x4 *)lt)[threadIdx.x + k * 512] = glint_u32x4{e.x, e.y, e.x, e.y};
+    }
+}
+/* The 8 weights of an MFMA step (H, P: their code words; lane8: copy lane % 32) as planes of
+ * their cells */
+__device__ __forceinline__ void f3_lookup(const uint8_t *lt, uint32_t H, uint32_t P, uint32_t lane8, glint_u32x2 (&e)[8]) {
+    const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
+    const uint32_t ad[8] = {glint_cell_addr<0>(E, lane8), glint_cell_addr<0>(O, lane8), glint_cell_addr<1>(E, lane8),
+                            glint_cell_addr<1>(O, lane8), glint_cell_addr<2>(E, lane8), glint_cell_addr<2>(O, lane8),
+                            glint_cell_addr<3>(E, lane8), glint_cell_addr<3>(O, lane8)};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        e[i] = *(const glint_u32x2 *)(lt + ad[i]);
+}
+__device__ __forceinline__ void f3_planes(const uint8_t *lt, uint32_t H, uint32_t P, uint32_t lane8, glint_bf16x8 (&bp)[3]) {
+    glint_u32x2 e[8];
+    f3_lookup(lt, H, P, lane8, e);
+    uint32_t pk[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        pk[0][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x05040100u);
+        pk[1][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x07060302u);
+        pk[2][j] = __builtin_amdgcn_perm(e[2 * j + 1].y, e[2 * j].y, 0x05040100u);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+}
+/* the same of the weights, cell * a (without the 2^24) */
+__device__ __forceinline__ void f3_planes_scaled(const uint8_t *lt, uint32_t H, uint32_t P, uint32_t lane8, float a,
+                                                 glint_bf16x8 (&bp)[3]) {
+    glint_u32x2 e[8];
+    f3_lookup(lt, H, P, lane8, e);
+    uint32_t pk[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t o[2][3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const glint_u32x2 c = e[2 * j + h];
+            const float cell = (__uint_as_float(c.x << 16) + __uint_as_float(c.x & 0xFFFF0000u)) + __uint_as_float(c.y << 16);
+            rl_split3(cell * F3_DOWN * a, true, o[h]);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            pk[i][j] = __builtin_amdgcn_perm(o[1][i], o[0][i], 0x07060302u);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
 }
 /* x with its infinities and NaNs as zeros: what the planes below hi meet, since infinity times a
  * plane that is 0 is not the product's value (hi is 0 only where the weight is) */
@@ -1645,50 +1715,6 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
             s.p[b] = *(const glint_u32x2 *)(wln + a + PLANE);
         }
     };
-    /* the 8 weights of MFMA step st as planes of their cells */
-    auto planes = [&](const WBlk &s, int st, glint_bf16x8 (&bp)[NP]) {
-        const uint32_t H = s.h[st >> 1][st & 1], P = s.p[st >> 1][st & 1];
-        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
-        const uint32_t ad[8] = {glint_cell_addr<0>(E, lane4), glint_cell_addr<0>(O, lane4), glint_cell_addr<1>(E, lane4),
-                                glint_cell_addr<1>(O, lane4), glint_cell_addr<2>(E, lane4), glint_cell_addr<2>(O, lane4),
-                                glint_cell_addr<3>(E, lane4), glint_cell_addr<3>(O, lane4)};
-        uint32_t pk[NP][4];
-        glint_u32x2 e[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            e[i] = *(const glint_u32x2 *)(lt + ad[i]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            pk[0][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x05040100u);
-            pk[1][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x07060302u);
-            pk[2][j] = __builtin_amdgcn_perm(e[2 * j + 1].y, e[2 * j].y, 0x05040100u);
-        }
-#pragma unroll
-        for (int i = 0; i < NP; ++i)
-            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
-    };
-    /* the same with the weights of the lane's row multiplied by `a` */
-    auto planes_scaled = [&](const WBlk &s, int st, float a, glint_bf16x8 (&bp)[NP]) {
-        const uint32_t H = s.h[st >> 1][st & 1], P = s.p[st >> 1][st & 1];
-        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            v[i] = (&kCells[0][0])[((i & 1 ? O : E) >> (8 * (i >> 1))) & 255u] * a;
-        uint32_t pk[NP][4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t l[3], h[3];
-            rl_split3(v[2 * j], true, l);
-            rl_split3(v[2 * j + 1], true, h);
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                pk[i][j] = __builtin_amdgcn_perm(h[i], l[i], 0x07060302u);
-        }
-#pragma unroll
-        for (int i = 0; i < NP; ++i)
-            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
-    };
     glint_f32x4 acc[MB][1];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -1711,9 +1737,9 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
             glint_bf16x8 af[MB], bp[NP];
             aread(xs, st, af);
             if (scaled)
-                planes_scaled(s, st, b ? a.y : a.x, bp);
+                f3_planes_scaled(lt, s.h[b][st & 1], s.p[b][st & 1], lane4, b ? a.y : a.x, bp);
             else
-                planes(s, st, bp);
+                f3_planes(lt, s.h[b][st & 1], s.p[b][st & 1], lane4, bp);
 #pragma unroll
             for (int pl = NP - 1; pl >= 0; --pl)
 #pragma unroll
@@ -1768,12 +1794,8 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
         }
     };
 
-    /* 16-B runs of two copies; run r is cell r / 16 (a wave's 64 runs hold 4 cells: scalar
-     * loads), 4096 runs in 8 steps */
     glint_f32x4 c4[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        c4[k] = *(const glint_f32x4 *)(&kCells[0][0] + ((64 * w + k * T) >> 4));
+    f3_fill_load(w, c4);
     __builtin_amdgcn_sched_barrier(0);
     xload(0, xr[0]);
     __builtin_amdgcn_sched_barrier(0);
@@ -1786,12 +1808,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
     for (int s = 0; s < U; ++s)
         wline(s, wl[s]);
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const float lo = g & 1 ? c4[k].y : c4[k].x, hi = g & 1 ? c4[k].w : c4[k].z;
-        const glint_u32x2 e = rl_entry(g & 2 ? hi : lo);
-        ((glint_u32x4 *)lt)[threadIdx.x + k * T] = glint_u32x4{e.x, e.y, e.x, e.y};
-    }
+    f3_fill_store(lt, g, c4);
     xstore(xb0, xr[0]);
     xload(2, xr[0]);
     wput(0, wl[0]);
@@ -1829,16 +1846,18 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
         const glint_u32x4 f0 = ((const glint_u32x4 *)wmax)[0], f1 = ((const glint_u32x4 *)wmax)[1];
         return (f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) != 0u;
     };
+    float down = F3_DOWN; /* the cells' 2^24 goes */
     if (meet()) {
         rerun();
         meet();
+        down = 1.0f;
     }
     if (kw == 0) /* added in kw order */
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                acc[mb][0][i] += red[((strip * MB + mb) * 4 + i) * 64 + lane];
+                acc[mb][0][i] = acc[mb][0][i] * down + red[((strip * MB + mb) * 4 + i) * 64 + lane] * down;
     __syncthreads(); /* the split-K epilogue's flag word lives in xb0 */
     if (gridDim.z > 1 && !tile_splitk_epilogue<MB, 1, 64 * STRIPS>(acc, part, ctr, *(unsigned *)xb1,
                                                                     (int)threadIdx.x, kw == 0))
@@ -1955,42 +1974,6 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         for (int i = 0; i < NX; ++i)
             *(glint_u32x4 *)(buf + xlo[i]) = xr[i];
     };
-    auto planes = [&](uint32_t H, uint32_t P, glint_bf16x8 (&bp)[3]) {
-        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
-        const uint32_t ad[8] = {glint_cell_addr<0>(E, lane8), glint_cell_addr<0>(O, lane8), glint_cell_addr<1>(E, lane8),
-                                glint_cell_addr<1>(O, lane8), glint_cell_addr<2>(E, lane8), glint_cell_addr<2>(O, lane8),
-                                glint_cell_addr<3>(E, lane8), glint_cell_addr<3>(O, lane8)};
-        glint_u32x2 e[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            e[i] = *(const glint_u32x2 *)(lt + ad[i]);
-        uint32_t pk[3][4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            pk[0][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x05040100u);
-            pk[1][j] = __builtin_amdgcn_perm(e[2 * j + 1].x, e[2 * j].x, 0x07060302u);
-            pk[2][j] = __builtin_amdgcn_perm(e[2 * j + 1].y, e[2 * j].y, 0x05040100u);
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
-    };
-    auto planes_scaled = [&](uint32_t H, uint32_t P, float a, glint_bf16x8 (&bp)[3]) {
-        const uint32_t E = glint_codes_even(H, P), O = glint_codes_odd(H, P);
-        uint32_t pk[3][4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint32_t l[3], h[3];
-            rl_split3((&kCells[0][0])[(E >> (8 * j)) & 255u] * a, true, l);
-            rl_split3((&kCells[0][0])[(O >> (8 * j)) & 255u] * a, true, h);
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                pk[i][j] = __builtin_amdgcn_perm(h[i], l[i], 0x07060302u);
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            bp[i] = __builtin_bit_cast(glint_bf16x8, glint_u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
-    };
     glint_f32x4 acc[MB][1], t[2][MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -2001,9 +1984,9 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         for (int s = 0; s < 2; ++s) {
             glint_bf16x8 bp[3];
             if (scaled)
-                planes_scaled(k.h[b][s], k.p[b][s], b ? k.a.y : k.a.x, bp);
+                f3_planes_scaled(lt, k.h[b][s], k.p[b][s], lane8, b ? k.a.y : k.a.x, bp);
             else
-                planes(k.h[b][s], k.p[b][s], bp);
+                f3_planes(lt, k.h[b][s], k.p[b][s], lane8, bp);
             const int pc = 8 * b + 2 * g + s;
             auto aread = [&](int mb) {
                 return __builtin_bit_cast(glint_bf16x8,
@@ -2057,18 +2040,11 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         ap = k.a.y;
     };
 
-    glint_f32x4 c4[8]; /* the table: as k_htile_rl3's */
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-        c4[i] = *(const glint_f32x4 *)(&kCells[0][0] + ((64 * w + i * T) >> 4));
+    glint_f32x4 c4[8];
+    f3_fill_load(w, c4);
     xload(0);
     wload(0, wb[0]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float lo = g & 1 ? c4[i].y : c4[i].x, hi = g & 1 ? c4[i].w : c4[i].z;
-        const glint_u32x2 e = rl_entry(g & 2 ? hi : lo);
-        ((glint_u32x4 *)lt)[threadIdx.x + i * T] = glint_u32x4{e.x, e.y, e.x, e.y};
-    }
+    f3_fill_store(lt, g, c4);
     xstore(xb0);
     xload(1);
     int j = 0;
@@ -2105,6 +2081,10 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
             block(xb1, wb[0], 1, true);
             add(1, 1.f);
         }
+    } else {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            acc[mb][0] *= F3_DOWN; /* the cells' 2^24 goes */
     }
     if (gridDim.z > 1) {
         __syncthreads(); /* the flags have been read: their words are the epilogue's */

@@ -16,10 +16,12 @@
  * Arithmetic: the f32 weight w = CELLS * absmax as three exact BF16 planes (hi, mid, lo;
  * GlintTileProducer::finish_split's rule), each multiplied with x in the MFMA, f32 sums. The
  * products are exact, so y differs from the scalar sum of w x only by the order of its f32
- * additions, for BF16 out as for f32 out. Where a scale is nonzero and below 2^-90 (lo may
- * then have bits BF16 cannot hold) or an output comes out infinite or NaN (an infinite or NaN
- * scale or x, where inf * 0 of a plane is not the product's value, or an overflow), the
- * workgroup forms its outputs again with one f32 FMA per weight in k order (htile_any_again).
+ * additions, for BF16 out as for f32 out (a subnormal x is aligned by the matrix core as if it were
+ * 2^-126: the sums are then exact to 2^-23 of sum |w| 2^-126). Where a scale is nonzero and below
+ * 2^-90 (lo may then have bits BF16 cannot hold) or an output comes out infinite or NaN (an
+ * infinite or NaN scale or x, where inf * 0 of a plane is not the product's value, or an
+ * overflow), the workgroup forms its outputs again with one f32 FMA per weight in k order
+ * (htile_any_again).
  *
  * Bound: the dequantization (about 9 VALU instructions and one LDS read per weight, once per
  * 16 MB rows of x) and the latency of a wave's 4 or 5 dependent chunks; the planes' bytes

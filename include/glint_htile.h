@@ -14,10 +14,13 @@ extern "C" {
 struct ihipStream_t;
 
 /* f32 output, f32 products and f32 sums (within 1e-5 * (1 + |ref|) of a float64 reference).
- * At M > 1 with blocksize 64, K % 64 == 0 and aligned pointers the products run on BF16
- * MFMA with each f32 weight split exactly into three BF16 planes (the sum differs from a
- * sequential f32 sum only in order); M = 1 is the f32 GEMV (K <= 32768; larger K takes
- * the MFMA route), other shapes the same three planes from unaligned rows. Enqueued on `stream`; y is overwritten
+ * With blocksize 64, K % 64 == 0 and aligned pointers, M = 1 (K <= 32768) and M = 2 .. 4 (5 and 6
+ * on small matrices, 5 .. 8 where K % 128 != 0) are f32 FMAs per weight. Above, the products run on
+ * BF16 MFMA with each cell split exactly into three BF16 planes, and a block's f32 sum is
+ * multiplied by its absmax; M = 1 at K > 32768 and every other shape split the f32 weight
+ * cell * absmax in the same way. x times a plane is exact, so against a sequential f32 sum only
+ * the order of the additions and the place of the scaling differ (a subnormal x is added as
+ * coarsely as 2^-126 would be). Enqueued on `stream`; y is overwritten
  * (with zeros when K <= 0: the empty sum, as in the reference). Returns 0, -1 for a null
  * pointer, -2 for blocksize <= 0, -3 for a launch error; M <= 0 or N <= 0 launches nothing
  * and returns 0. The MFMA route uses the stream's split-K workspace as
