@@ -1214,7 +1214,7 @@ __global__ __launch_bounds__(64 * RD_STRIPS * KW, 1) void k_htile_rd(const uint8
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         acc[mb][0][i] += red[((((k - 1) * RD_STRIPS + strip) * MB + mb) * 4 + i) * 64 + lane];
-        __syncthreads(); /* the split-K epilogue's flag word lives in xb0 */
+        __syncthreads(); /* the split-K epilogue's flag word lives in xb1 */
     }
     if (gridDim.z > 1 && !tile_splitk_epilogue<MB, 1, 64 * RD_STRIPS>(acc, part, ctr, *(unsigned *)xb1,
                                                                        (int)threadIdx.x, kw == 0))
@@ -1456,7 +1456,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 acc[mb][0][i] += red[((strip * MB + mb) * 4 + i) * 64 + lane];
-    __syncthreads(); /* the split-K epilogue's flag word lives in xb0 */
+    __syncthreads(); /* the split-K epilogue's flag word lives in xb1 */
     if (gridDim.z > 1 && !tile_splitk_epilogue<MB, 1, 64 * STRIPS>(acc, part, ctr, *(unsigned *)xb1,
                                                                     (int)threadIdx.x, kw == 0))
         return;
@@ -1487,11 +1487,14 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl(const uint8_t *__restrict__
  *     the scale and one addition per block are all the roundings there are. Only a subnormal x is
  *     added less exactly: the matrix core aligns its products as if x were 2^-126, so a product of
  *     2^-133 may lose 7 bits (per-weight planes of w are no different there).
- *   - A workgroup that met a scale that is infinite, NaN or at least 2^126, or whose sums came out
- *     infinite or NaN (an infinite or NaN x, or x so large, from 2^97 on, that a block's unscaled
- *     sum overflows), goes over its split again with the products w = cell * absmax split as
- *     GlintTileProducer::finish_split does, so infinities of both signs meet as they do in a sum
- *     of weights; there only the hi plane meets infinities and NaNs of x.
+ *   - A workgroup that met an infinite scale, or an infinite or NaN sum that neither a NaN scale of
+ *     its row of W nor a NaN in its row of x explains (an infinite x, or x so large, from 2^97 on,
+ *     that a block's unscaled sum overflows; x is looked through for NaN only then), goes over its
+ *     split again with the products w = cell * absmax split as GlintTileProducer::finish_split
+ *     does, so infinities of both signs meet as they do in a sum of weights; there only the hi
+ *     plane meets infinities and NaNs of x. 14336 x 4096 M = 8 19.8 us: with NaN in every row of x
+ *     21.8 (the second pass for it, unpipelined and on cells from global memory, 79.6), with an
+ *     infinite x 57.9; 4096 x 14336 M = 64 32.1, 36.2 (99.2), 90.3.
  * Bound: a step's chain of LDS reads, lookups and MFMAs at two waves per SIMD, as k_htile_rl.
  * Measured against the per-weight split (rotated pins):
  * 14336 x 4096 M = 5 30.6 (as two small-M launches) -> 21.0 us, 8 30.0 -> 21.0, 32 33.9 -> 26.1,
@@ -1598,16 +1601,59 @@ __device__ __forceinline__ glint_bf16x8 rl_finite(glint_bf16x8 x) {
     }
     return __builtin_bit_cast(glint_bf16x8, v);
 }
-/* any output of the lane infinite or NaN */
+/* any output of the lane infinite or NaN, but for those in rows of x that rows[] names */
 template <int MB>
-__device__ __forceinline__ bool rl_nonfinite(const glint_f32x4 (&acc)[MB][1]) {
+__device__ __forceinline__ bool f3_nonfinite(const glint_f32x4 (&acc)[MB][1], const uint32_t *rows, int g) {
     bool bad = false;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            bad |= !(__builtin_fabsf(acc[mb][0][i]) < __builtin_inff());
+            bad |= !(__builtin_fabsf(acc[mb][0][i]) < __builtin_inff()) & (!rows || rows[16 * mb + 4 * g + i] == 0u);
     return bad;
+}
+/* What a lane's scales and sums ask for: 2 the second pass (an infinite scale), 1 a look at x (a
+ * sum infinite or NaN), 0 nothing. amax: the largest |scale| bits of the lane's row of W; where
+ * that is NaN the row's outputs are, and nothing has to be formed again. */
+template <int MB>
+__device__ __forceinline__ uint32_t f3_word(uint32_t amax, const glint_f32x4 (&acc)[MB][1]) {
+    const bool fin = amax <= 0x7F800000u;
+    return __any(amax == 0x7F800000u) ? 2u : (__any(fin && f3_nonfinite<MB>(acc, nullptr, 0)) ? 1u : 0u);
+}
+/* the OR of the 8 waves' words, through LDS words[0 .. 8) that all have finished with */
+__device__ __forceinline__ uint32_t f3_all(uint32_t *words, int w, uint32_t word) {
+    words[w] = word;
+    __syncthreads();
+    const glint_u32x4 a = ((const glint_u32x4 *)words)[0], b = ((const glint_u32x4 *)words)[1];
+    return a.x | a.y | a.z | a.w | b.x | b.y | b.z | b.w;
+}
+/* rows[r] = whether row r of x has a NaN in the n elements (a multiple of 64) from k0 on: its
+ * outputs are NaN in the first pass as they have to be */
+template <int BM>
+__device__ __forceinline__ void f3_nan_rows(const __amdgpu_buffer_rsrc_t rx, int K, int k0, int n, uint32_t *rows) {
+    constexpr int TPR = 512 / BM; /* threads per row */
+    const int r = (int)threadIdx.x / TPR, np = n / 8, rounds = (np + TPR - 1) / TPR;
+    const uint32_t o = ((uint32_t)r * (uint32_t)K + (uint32_t)k0) * 2u;
+    if (threadIdx.x < BM)
+        rows[threadIdx.x] = 0;
+    using u16x2 = uint16_t __attribute__((ext_vector_type(2)));
+    u16x2 most = {0, 0};
+    for (int i = 0; i < rounds; i += 8) { /* the last piece again past the end */
+        glint_u32x4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = __builtin_amdgcn_raw_buffer_load_b128(
+                rx, o + 16u * (uint32_t)min((i + u) * TPR + (int)threadIdx.x % TPR, np - 1), 0, 0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, v[u][j] & 0x7FFF7FFFu));
+    }
+    __syncthreads();
+    if (most.x > 0x7F80 || most.y > 0x7F80)
+        rows[r] = 1u;
+    __syncthreads();
 }
 template <int MB>
 __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict__ hole, const uint8_t *__restrict__ plug,
@@ -1775,22 +1821,26 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
         }
         mma((u & 1) ? xb1 : xb0, wb[u & 1], a, false);
     };
-    /* the split once more, unpipelined, with every weight multiplied by its scale */
+    /* the split once more, a line ahead, with every weight multiplied by its scale */
     auto rerun = [&]() {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
             acc[mb][0] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+        xload(0, xr[0]);
+        wline(0, wl[0]);
+        aload(0, am[0]);
 #pragma unroll 1
         for (int X = 0; X < nxc; ++X) {
             __syncthreads();
-            xload(X, xr[0]);
-            wline(X, wl[0]);
-            aload(X, am[0]);
             xstore(xb0, xr[0]);
             wput(0, wl[0]);
+            const glint_f32x2 a = am[0];
             __syncthreads();
+            xload(X + 1, xr[0]);
+            wline(X + 1, wl[0]);
+            aload(X + 1, am[0]);
             wget(0, wb[0]);
-            mma(xb0, wb[0], am[0], true);
+            mma(xb0, wb[0], a, true);
         }
     };
 
@@ -1815,6 +1865,10 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
     wput(1, wl[1]);
     __syncthreads();
     wget(0, wb[0]);
+    /* The loop's place modulo 8 bytes decides 5% of it: 14336 x 4096 M = 8 19.8 us where it starts
+     * on a multiple of 8, 18.8 four bytes further on (nothing but this moved; one, two and eight
+     * instructions tried at either place). */
+    asm volatile(".p2align 3\n\ts_nop 0");
     int X = 0;
     for (; X + U <= nxc; X += U) {
 #pragma unroll
@@ -1826,31 +1880,34 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
         if (X + u < nxc)
             step(X + u, u);
     __builtin_amdgcn_s_waitcnt(GLINT_WAIT_VMCNT0); /* the trailing dropped loads */
-    /* the strip's two partials meet in xb0 (the x buffers are free); the waves' largest scales
-     * and their sums, in xb1, tell whether the workgroup has to run again */
+    /* the strip's two partials meet in xb0 (the x buffers are free); the waves' words in xb1 tell
+     * whether the workgroup has to look further */
     float *red = (float *)xb0;
-    uint32_t *wmax = (uint32_t *)xb1;
+    uint32_t *words = (uint32_t *)xb1, *rows = words + 16;
     static_assert(STRIPS * 64 * MB * 4 * 4 <= XCH, "partials fit an x buffer");
-    auto meet = [&]() -> bool {
-        const bool big = __any(amax >= 0x7E800000u || rl_nonfinite<MB>(acc)); /* 2^126, infinite or NaN */
+    auto meet = [&](uint32_t word) -> uint32_t {
         __syncthreads();
-        if (lane == 0)
-            wmax[w] = big;
         if (kw > 0)
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     red[((strip * MB + mb) * 4 + i) * 64 + lane] = acc[mb][0][i];
-        __syncthreads();
-        const glint_u32x4 f0 = ((const glint_u32x4 *)wmax)[0], f1 = ((const glint_u32x4 *)wmax)[1];
-        return (f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) != 0u;
+        return f3_all(words, w, word);
     };
     float down = F3_DOWN; /* the cells' 2^24 goes */
-    if (meet()) {
-        rerun();
-        meet();
-        down = 1.0f;
+    const uint32_t met = meet(f3_word<MB>(amax, acc));
+    if (__builtin_expect(met != 0u, 0)) {
+        bool again = met & 2u;
+        if (!again) {
+            f3_nan_rows<16 * MB>(rx, K, c0 * 128, nj * 128, rows);
+            again = f3_all(words, w, __any(amax <= 0x7F800000u && f3_nonfinite<MB>(acc, rows, g))) != 0u;
+        }
+        if (again) {
+            rerun();
+            meet(0);
+            down = 1.0f;
+        }
     }
     if (kw == 0) /* added in kw order */
 #pragma unroll
@@ -1858,7 +1915,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 acc[mb][0][i] = acc[mb][0][i] * down + red[((strip * MB + mb) * 4 + i) * 64 + lane] * down;
-    __syncthreads(); /* the split-K epilogue's flag word lives in xb0 */
+    __syncthreads(); /* the split-K epilogue's flag word lives in xb1 */
     if (gridDim.z > 1 && !tile_splitk_epilogue<MB, 1, 64 * STRIPS>(acc, part, ctr, *(unsigned *)xb1,
                                                                     (int)threadIdx.x, kw == 0))
         return;
@@ -1888,8 +1945,9 @@ __global__ __launch_bounds__(512, 1) void k_htile_rl3(const uint8_t *__restrict_
  *   - Block sums start from zero; a block's FMAs by its scale are issued among the next block's
  *     MFMAs (two sets of sums).
  *   - K is split over gridDim.z workgroups where the tiles alone leave CUs idle.
- * Special scales and x as in k_htile_rl3. HALF: K % 128 == 64, the last chunk has one block: nothing of
- * its second half is loaded, neither of W nor of x.
+ * Special scales and x as in k_htile_rl3 (512 x 14336 x 4096 161 us: with NaN in every row of x 181,
+ * after a second pass 576; with an infinity in every row 557). HALF: K % 128 == 64, the last
+ * chunk has one block: nothing of its second half is loaded, neither of W nor of x.
  * Bound: the matrix cores, three planes of every product (2048 x 14336 x 4096: 1.21 PFLOP/s of
  * BF16 MFMA; a dense BF16 product of that shape by the vendor's library runs at 1.14). Measured
  * against the three-plane LDS tiles (128 x 128; rotated pins): 2048 x 14336 x 4096 762 -> 597 us,
@@ -1992,14 +2050,25 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
                 return __builtin_bit_cast(glint_bf16x8,
                                           *(const glint_u32x4 *)(xs + (16 * mb + m16) * 256 + ((pc ^ m16) << 4)));
             };
-            if (scaled) { /* one fragment of x at a time: few registers */
+            if (scaled) { /* two fragments of x at a time: few registers */
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) {
-                    const glint_bf16x8 a = aread(mb), fin = rl_finite(a);
-                    glint_f32x4 v = s == 0 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb];
-                    v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fin, bp[2], v, 0, 0, 0);
-                    v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fin, bp[1], v, 0, 0, 0);
-                    t[b][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bp[0], v, 0, 0, 0);
+                for (int mb = 0; mb < MB; mb += 2) {
+                    glint_bf16x8 a[2], fin[2];
+                    glint_f32x4 v[2];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        a[i] = aread(mb + i);
+                        fin[i] = rl_finite(a[i]);
+                        v[i] = s == 0 ? glint_f32x4{0.f, 0.f, 0.f, 0.f} : t[b][mb + i];
+                    }
+#pragma unroll
+                    for (int pl = 2; pl >= 0; --pl)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            v[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl ? fin[i] : a[i], bp[pl], v[i], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        t[b][mb + i] = v[i];
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 continue;
@@ -2047,6 +2116,7 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
     f3_fill_store(lt, g, c4);
     xstore(xb0);
     xload(1);
+    asm volatile(".p2align 3"); /* the loop's place: 512 x 14336 x 4096 161.8 us, four bytes further on 163.3 */
     int j = 0;
     for (; j + 2 <= nj; j += 2) {
         step(j, 0);
@@ -2056,29 +2126,33 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
         step(j, 0);
     add(1, ap);
 
-    /* a special scale or sum anywhere in the workgroup: the split once more, unpipelined, with every
-     * weight multiplied by its scale */
-    const bool big = __any(amax >= 0x7E800000u || rl_nonfinite<MB>(acc)); /* 2^126, infinite or NaN */
-    uint32_t *flag = (uint32_t *)xb0;
+    /* an infinite scale or an unexplained sum anywhere in the workgroup: the split once more, a
+     * chunk ahead, with every weight multiplied by its scale */
+    uint32_t *words = (uint32_t *)xb0, *rows = words + 16;
     __syncthreads();
-    if (lane == 0)
-        flag[w] = big;
-    __syncthreads();
-    const glint_u32x4 f0 = ((const glint_u32x4 *)flag)[0], f1 = ((const glint_u32x4 *)flag)[1];
-    if ((f0.x | f0.y | f0.z | f0.w | f1.x | f1.y | f1.z | f1.w) != 0u) {
+    const uint32_t met = f3_all(words, w, f3_word<MB>(amax, acc));
+    bool again = met & 2u;
+    if (met == 1u) {
+        f3_nan_rows<BM>(rx, K, c0 * 128, 64 * min(2 * nj, nb), rows);
+        again = f3_all(words, w, __any(amax <= 0x7F800000u && f3_nonfinite<MB>(acc, rows, g))) != 0u;
+    }
+    if (__builtin_expect(again, 0)) {
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
             acc[mb][0] = glint_f32x4{0.f, 0.f, 0.f, 0.f};
+        xload(0);
+        wload(0, wb[0]);
 #pragma unroll 1
         for (int i = 0; i < nj; ++i) {
-            xload(i);
-            wload(i, wb[0]);
             __syncthreads();
             xstore(xb1);
+            const WBlk k = wb[0];
             __syncthreads();
-            block(xb1, wb[0], 0, true);
+            xload(i + 1);
+            wload(i + 1, wb[0]);
+            block(xb1, k, 0, true);
             add(0, 1.f);
-            block(xb1, wb[0], 1, true);
+            block(xb1, k, 1, true);
             add(1, 1.f);
         }
     } else {

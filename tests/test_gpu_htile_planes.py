@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from glint_amd import glint_hip as H
-from tests.gpu_util import bf16_bits, dev, host
+from tests.gpu_util import bf16_bits, dev, host, torch_cuda
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +82,57 @@ def test_special_x(oracle, M, N, K):
     assert np.array_equal(np.isinf(y), np.isinf(want))
     fin = np.isfinite(want)
     assert (np.abs(y[fin] - ref[fin]) <= (K + 2) * 2.0 ** -23 * asum[fin]).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(7, 13, 384), (20, 100, 1152), (64, 64, 14464), (9, 40, 192), (70, 40, 384),
+                                   (128, 24576, 192), (130, 64, 14464), (70, 40, 448)])
+@pytest.mark.parametrize("inf", [False, True])
+def test_nan_rows_and_columns(oracle, M, N, K, inf):
+    """NaN in some rows of x and some scales, which need no second pass, alone and beside an infinity
+    that does: in a row with a NaN, in one without; every place of a row at one shape or another."""
+    print(f"htile planes NaN M={M} N={N} K={K} inf={inf}", flush=True)
+    hole, plug, am, x = _inputs(M, N, K)
+    x = x.reshape(M, K).copy()
+    rng = np.random.default_rng(M + K)
+    for r in range(0, M, 3):
+        x[r, rng.integers(0, K)] = rng.choice([0x7FC0, 0x7F81, 0xFFFF])
+    x[M - 1, K - 1] = 0xFF81
+    if inf:
+        x[1, K // 3], x[3, 5] = 0x7F80, 0xFF80
+    am = np.where(am > 0, am, np.float32(0.5)).astype(np.float32)
+    am[(K // 64) * 5 + 1] = am[-1] = np.nan
+    y = host(H.htile_f32(dev(hole), dev(plug), dev(am), dev(x).reshape(M, K), N, K, 64)).reshape(M, N)
+    nan = (((x & 0x7FFF) > 0x7F80).any(1)[:, None]) | np.isnan(am).reshape(N, -1).any(1)[None, :]
+    ref, asum = (a.reshape(M, N) for a in oracle.htile_f64(hole, plug, np.nan_to_num(am), np.where(((x & 0x7F80) == 0x7F80), 0, x).astype(np.uint16).reshape(-1), M, N, K, 64))
+    if inf:
+        assert np.isinf(y[1][~nan[1]]).all()
+        nan[1], nan[3] = True, True
+        y[1] = np.nan
+    assert np.array_equal(np.isnan(y), nan)
+    assert (np.abs(y - ref) <= (K + 2) * 2.0 ** -23 * asum)[~nan].all()
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 14336, 4096), (64, 4096, 14336), (512, 14336, 4096)])
+def test_special_values_time(M, N, K):
+    """NaN in x costs a look at x (measured 1.1 to 1.2 times a call without), an infinity one more
+    pass over the tiles that met it."""
+    torch = torch_cuda()
+    print(f"htile planes time M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    pin = H.encode_bf16((torch.randn(N * K, device="cuda", generator=g) * 0.02).to(torch.bfloat16), 64)
+    x = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+
+    def us(x):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record()
+        for _ in range(20):
+            H.htile_f32(*pin, x, N, K, 64)
+        e[1].record()
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1]) * 50
+    us(x)
+    for value, limit in ((float("nan"), 1.5), (float("inf"), 3.5)):
+        xs = x.clone()
+        xs[:, 7] = value
+        t = sorted(us(xs) / us(x) for _ in range(7))
+        assert t[3] < limit, (value, t)
