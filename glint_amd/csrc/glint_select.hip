@@ -590,11 +590,13 @@ __global__ __launch_bounds__(SEL_T) void k_select_topk(const uint16_t *__restric
  * list entry, x and rows: taken one entry at a time that chain was the kernel. A wave takes
  * KM_CB entries at a time: lane l loads entry l of the batch and its x, and the rows and the
  * block scales of all of them are in flight before the first is looked up (the first batch's
- * before the table is filled). The table comes through scalar loads. 14336 x 4096, 411 entries
- * in 8 chunks: 9.0 -> 7.7 us; 4096 x 14336, 1433 entries: 15.6 -> 9.9; 4096 x 1024, 100 entries
- * (two per wave): 5.0 -> 5.4. Scalar loads of the list took 9.4 us (129 registers: one workgroup
- * per CU), batches of 4 8.0. */
-#define KM_CB 8 /* list entries in flight per wave */
+ * before the table is filled). A part of at most 4 or 2 entries loads no more: eight for two cost
+ * 8% (4096 x 1024, 100 entries: 5.1 us, eight at a time 5.6, one at a time 5.2; 1024 x 4096, 64
+ * entries 5.0, 5.5, 5.2). The table comes through scalar loads. Against one entry at a time
+ * 14336 x 4096, 411 entries in 8 chunks: 9.0 -> 7.7 us; 4096 x 14336, 1433 entries: 15.4 -> 10.0.
+ * Scalar loads of the list took 9.4 us (129 registers: one workgroup per CU), batches of 4 8.0,
+ * smaller batches behind the first one too 10.9 (1433 entries; 194 registers). */
+#define KM_CB 8 /* most list entries in flight per wave */
 __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restrict__ hole_k,
                                                          const uint32_t *__restrict__ plug_k,
                                                          const float *__restrict__ scales_k,
@@ -634,13 +636,14 @@ __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restr
         int c[KM_CB]; /* wave-uniform */
         float xv[KM_CB];
     } bt;
-    /* the batch from entry i on: past the part's end its last entry again (loaded, not added) */
-    auto load = [&](int i) {
-        const int cl = idx[min(i + min(lane, KM_CB - 1), i1 - 1)];
+    /* CB entries from entry i on: past the part's end its last entry again (loaded, not added) */
+    auto load = [&](int i, auto count) __attribute__((always_inline)) {
+        constexpr int CB = decltype(count)::value;
+        const int cl = idx[min(i + min(lane, CB - 1), i1 - 1)];
         const float xl = km_bf16(x[cl]);
         int prev = cur;
 #pragma unroll
-        for (int u = 0; u < KM_CB; ++u) {
+        for (int u = 0; u < CB; ++u) {
             const int c = __builtin_amdgcn_readlane(cl, u);
             bt.c[u] = c;
             bt.h[u] = hole_k[(int64_t)c * rowv + rc / RPL];
@@ -651,19 +654,19 @@ __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restr
             prev = c >> 6;
         }
 #pragma unroll
-        for (int u = 0; u < KM_CB; ++u)
+        for (int u = 0; u < CB; ++u)
             bt.xv[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(xl), u));
     };
-    auto flush = [&]() {
+    auto flush = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < RPL; ++j) {
             tot[j] = fmaf(acc[j], scur[j], tot[j]);
             acc[j] = 0.f;
         }
     };
-    auto add = [&](int n) {
+    auto add = [&](int n, auto count) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < KM_CB; ++u) {
+        for (int u = 0; u < decltype(count)::value; ++u) {
             if (u >= n)
                 break;
             if ((bt.c[u] >> 6) != cur) {
@@ -678,9 +681,7 @@ __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restr
             km_lookup_fma<RPL>(lds, E, O, lane4, bt.xv[u], acc);
         }
     };
-    if (i0 < i1)
-        load(i0);
-    {
+    auto fill = [&]() __attribute__((always_inline)) {
         const int l4 = lane >> 4;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
@@ -688,12 +689,30 @@ __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restr
             const float d = (l4 & 2 ? b : a) - pe[k];
             ((glint_f32x4 *)lds)[threadIdx.x + k * KM_WG] = glint_f32x4{d, d, d, d};
         }
-    }
-    __syncthreads();
-    for (int i = i0; i < i1; i += KM_CB) {
-        if (i > i0)
-            load(i);
-        add(i1 - i);
+        __syncthreads();
+    };
+    /* ways of their own up to the sums: where they met behind the loads, the waits before the first
+     * entry were those of the shortest part (1000 entries 9.7 -> 10.0 us) */
+    using B2 = std::integral_constant<int, 2>;
+    using B4 = std::integral_constant<int, 4>;
+    using B8 = std::integral_constant<int, KM_CB>;
+    if (i1 - i0 > 4) {
+        load(i0, B8{});
+        fill();
+        for (int i = i0; i < i1; i += KM_CB) {
+            if (i > i0)
+                load(i, B8{});
+            add(i1 - i, B8{});
+        }
+    } else if (i1 - i0 > 2) {
+        load(i0, B4{});
+        fill();
+        add(i1 - i0, B4{});
+    } else {
+        if (i1 > i0)
+            load(i0, B2{});
+        fill();
+        add(i1 - i0, B2{});
     }
     if (cur >= 0)
         flush();

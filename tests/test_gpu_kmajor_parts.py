@@ -57,3 +57,24 @@ def test_correction_batches(oracle, count, ks):
     got = host(H.apply_corr_km(dev(hk), dev(pk), dev(sk), dev(x), dev(pad), dev(np.array([count], np.int32)), dev(y0), N, K, ks))
     want = oracle.apply_corr_km(hk, pk, sk, x, idx, N, K, y0, ks)
     assert got.tobytes() == want.tobytes(), first_diff(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("ks", [1, 8])
+@pytest.mark.parametrize("per_wave", [1, 2, 3, 4, 5])
+def test_correction_short_parts(oracle, per_wave, ks):
+    """Parts of one to five entries per wave (loaded two, four or eight at once), the last wave's
+    shorter, with and without neighbours in a block."""
+    torch_cuda()
+    N, K = 544, 640
+    (hk, pk, sk), x = _km(oracle, N, K)
+    y0 = np.random.default_rng(ks).normal(0, 1, N).astype(np.float32)
+    for short in (0, 1):
+        count = per_wave * 8 * ks - short * (per_wave * 4 - 1)
+        for idx in (np.arange(count), np.sort(np.random.default_rng(count).choice(K, count, replace=False))):
+            print(f"correction parts of {per_wave} count={count} ks={ks}", flush=True)
+            pad = np.zeros(K, np.int32)
+            pad[:count] = idx
+            got = host(H.apply_corr_km(dev(hk), dev(pk), dev(sk), dev(x), dev(pad), dev(np.array([count], np.int32)),
+                                       dev(y0), N, K, ks))
+            want = oracle.apply_corr_km(hk, pk, sk, x, idx.astype(np.int32), N, K, y0, ks)
+            assert got.tobytes() == want.tobytes(), first_diff(got.view(np.uint32), want.view(np.uint32))
