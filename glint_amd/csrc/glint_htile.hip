@@ -2235,13 +2235,17 @@ static int htile_launch_rd_mb(const uint8_t *hole, const uint8_t *plug, const fl
     int ks = plan(std::max(1, std::min(std::min(TILE_SPLIT_MAX, nc), (int)((int64_t)cus * RMAX / N))), cps, R, gx);
     GlintSplitWs ws{nullptr, nullptr, 0, 0};
     if (ks > 1) {
-        const bool got = fixed ? (ws = *fixed, true) : glint_split_ws_stream(st, ws);
+        /* M = 5 and 6 have the two small-M launches, which need no workspace: a graph takes those, so
+         * that it is bound to none that a release or another graph's replay could touch */
+        const bool two = F32 && M <= 2 * GEMV_MR_MAX_F32 - 2;
+        const bool got = fixed ? (ws = *fixed, true)
+                               : !(two && glint_stream_captures(st)) && glint_split_ws_stream(st, ws);
         const bool fits = got && (size_t)ks * gx * TILE_FLOATS <= ws.part_floats && (size_t)gx <= ws.nctr;
         if (!fits) {
             if (fixed)
                 return -5;
-            if (F32 && M <= 2 * GEMV_MR_MAX_F32 - 2)
-                return 1; /* no workspace (a capture without one): the two small-M launches need none */
+            if (two)
+                return 1; /* a capture, or no workspace */
             ks = plan(1, cps, R, gx); /* no workspace (a capture without one): unsplit */
             ws = GlintSplitWs{nullptr, nullptr, 0, 0};
         }

@@ -1076,6 +1076,10 @@ static inline size_t glint_split_ws_bytes(size_t &cb, size_t &nctr, size_t &part
     cb = glint_split_ctr_bytes(nctr);
     return cb + part_floats * sizeof(float);
 }
+static inline bool glint_stream_captures(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+}
 static inline bool glint_split_ws_stream(hipStream_t st, GlintSplitWs &ws, bool may_alloc = true) {
     uint64_t key = 0;
     if (!glint_split_ws_key(st, key))

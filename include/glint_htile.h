@@ -49,7 +49,8 @@ int launch_glint_htile_s3_f32(const uint8_t *d_hole, const uint8_t *d_plug, cons
  * a fresh eager one. So replays and eager calls never share counters, replays of graphs
  * captured on one stream share theirs and must not overlap one another, and capture ->
  * eager cycles allocate nothing after the first. hipStreamPerThread gets its own per host
- * thread. A capture on a stream with no workspace yet runs unsplit. Same return codes. */
+ * thread. A capture on a stream with no workspace yet runs unsplit. f32 out at M = 5 and 6
+ * binds no workspace under capture. Same return codes. */
 int launch_glint_htile_bf16_stream(const uint8_t *d_hole, const uint8_t *d_plug, const float *d_absmax,
                                    const void *d_x_bf16, uint16_t *d_y_bf16,
                                    int M, int N, int K, int blocksize, struct ihipStream_t *stream);
