@@ -16,7 +16,12 @@
  *   tiles alone would leave CUs idle (fixed-order reduction). k_tile_mfma: 256 x 128 tiles
  *   over 8 waves for M >= 256; k_tile_ss: 64 x 64 / 128 x 64 over 4 waves below, with the
  *   weights loaded a whole 128-B line per 8 lanes. Both are shared with the INT8-pin
- *   W8A16 GEMM.
+ *   W8A16 GEMM. M <= 64 with K % 128 == 0 takes k_htile_rl first.
+ * k_htile_gemv_mr — 2 <= M <= 4, and 5 .. 8 in two launches where k_htile_rl / k_htile_rl3 do
+ *   not go first.
+ * f32 out above that: k_htile_rl3 (M <= 64, K % 128 == 0) and k_htile_f3 (the rest, any
+ *   K % 64 == 0): exact cells as three BF16 planes, block scales on f32 block sums. M = 1 with
+ *   K > 32768: k_tile_mfma with three planes of the weights.
  * k_htile_any (htile_any.h) — every other shape (any M, K, bs, alignment): unaligned rows
  *   read from their own byte address, exact f32 weights as three BF16 planes on MFMA.
  */
@@ -2191,7 +2196,7 @@ static inline int64_t f3_cost(int mb, int M, int N, int K) {
     const int64_t ks = (nc + cps - 1) / cps, rounds = (tiles * ks + cus - 1) / cus;
     return rounds * cps * (mb == 8 ? 266 : 155) + (ks > 1 ? (mb == 8 ? 600 : 400) : 0);
 }
-/* Returns 1 where the shape does not fit (the caller takes the f32 LDS tiles), else 0 or -3. */
+/* Returns 1 where its 31-bit offsets or grid do not reach (the caller takes the f32 LDS tiles), else 0 or -3. */
 #ifndef F3_ON
 #define F3_ON 1
 #endif
@@ -2213,9 +2218,10 @@ static int htile_launch_f3(const uint8_t *hole, const uint8_t *plug, const float
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-/* k_htile_rl (k_htile_rd) over an M <= 64 prefill, BF16 out, or f32 out (F32: k_htile_rl3). Returns 1 where the shape does not fit (K % 128 != 0, offsets beyond 31 bits; the
- * caller takes the LDS tiles), -5 where a `fixed` workspace is too small for the split plan,
- * else 0 or -3. */
+/* k_htile_rl (k_htile_rd) over an M <= 64 prefill, BF16 out, or f32 out (F32: k_htile_rl3).
+ * Returns 1 where the shape does not fit (K % 128 != 0, offsets beyond 31 bits; the caller takes
+ * the LDS tiles, f32 out k_htile_f3), -5 where a `fixed` workspace is too small for the split
+ * plan, else 0 or -3. */
 template <int MB, bool F32>
 static int htile_launch_rd_mb(const uint8_t *hole, const uint8_t *plug, const float *absmax, const uint16_t *x,
                               void *y, int M, int N, int K, hipStream_t st, const GlintSplitWs *fixed) {
@@ -2275,15 +2281,11 @@ static int htile_launch_rd(const uint8_t *hole, const uint8_t *plug, const float
     return htile_launch_rd_mb<4, F32>(hole, plug, absmax, xb, y, M, N, K, st, fixed);
 }
 
-/* f32 output at M > 1 where k_htile_f3's 31-bit offsets do not reach: 3-plane k_tile_mfma, whose
- * products are exact and whose sums are f32. 128 x 128 tiles over 8 waves (2 x 4, wave tile
- * 64 x 32) fill the 160 KiB of LDS: x 32 KiB, three W planes 96 KiB, cell table 32 KiB;
- * below 128 rows 64 x 128 tiles (8 waves in a row, wave tile 64 x 16), or 64 x 64 over 4
- * waves where those would leave CUs idle (4096 x 14336 at M = 64: 78.5 -> 61.6 us). */
-#define F32_TILE_MIN_M 128
-#ifndef F32_BN64
-#define F32_BN64 1
-#endif
+/* f32 output at M = 1 and K > 32768, beyond the GEMV's K (and at M > 1 beyond k_htile_f3's 31-bit
+ * offsets, K of 8 million and more): 3-plane k_tile_mfma, whose products are exact and whose sums
+ * are f32. 64 x 128 tiles (8 waves in a row, wave tile 64 x 16), or 64 x 64 over 4 waves where
+ * those, split K ways at most TILE_SPLIT_MAX, would leave CUs idle (4096 x 14336 at M = 64:
+ * 78.5 -> 61.6 us). */
 
 /* `fixed`: the caller's split-K workspace (the no-allocation entry point); null for the
  * stream's own. Returns 0, -1 null pointer, -2 bs <= 0, -3 launch error, -5 the split plan
@@ -2388,7 +2390,7 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
         if (!planned)
             return -5;
     } else if (mfma_ok && M > 1 &&
-               (f3 = f3_cost(8, M, N, K) <= f3_cost(4, M, N, K)
+               (f3 = (M + 63) / 64 > 65535 /* the 64-row tiles' grid */ || f3_cost(8, M, N, K) <= f3_cost(4, M, N, K)
                          ? htile_launch_f3<8>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)
                          : htile_launch_f3<4>(hole, plug, absmax, x, (float *)y, M, N, K, st, fixed)) != 1) {
         return f3;
@@ -2396,16 +2398,11 @@ static int htile_launch(const uint8_t *hole, const uint8_t *plug, const float *a
         const GlintTileProducer p{(const glint_u32x2 *)hole, (const glint_u32x2 *)plug, absmax, N, K, nullptr};
         const uint16_t *xb = (const uint16_t *)x;
         float *yf = (float *)y;
-        /* below 128 rows, 64 x 64 tiles (4 waves) where the 64 x 128 ones, split K ways at most
-         * TILE_SPLIT_MAX, would leave CUs idle (the 4096-row down projection) */
         const int64_t tiles128 = (int64_t)((N + 127) / 128) * ((M + 63) / 64);
-        const bool narrow = F32_BN64 && tiles128 * TILE_SPLIT_MAX < glint_cu_count();
         const bool planned =
-            M < F32_TILE_MIN_M
-                ? (narrow ? tile_mfma_launch<64, 64, 1, 4, 2, GlintTileProducer, TileOutF32, 3>(p, xb, yf, M, N, K, st, fixed)
-                          : tile_mfma_launch<64, 128, 1, 8, 2, GlintTileProducer, TileOutF32, 3>(p, xb, yf, M, N, K, st,
-                                                                                                  fixed))
-                : tile_mfma_launch<128, 128, 2, 4, 2, GlintTileProducer, TileOutF32, 3>(p, xb, yf, M, N, K, st, fixed);
+            tiles128 * TILE_SPLIT_MAX < glint_cu_count()
+                ? tile_mfma_launch<64, 64, 1, 4, 2, GlintTileProducer, TileOutF32, 3>(p, xb, yf, M, N, K, st, fixed)
+                : tile_mfma_launch<64, 128, 1, 8, 2, GlintTileProducer, TileOutF32, 3>(p, xb, yf, M, N, K, st, fixed);
         if (!planned)
             return -5;
     } else {

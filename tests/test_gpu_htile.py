@@ -420,8 +420,8 @@ def test_f32_prefill_mfma_vs_float64(oracle, M, N, K):
     summation bound (K + 2) 2^-23 sum|t| and within the reference's 1e-5 (1 + |ref|);
     ragged M and N: M <= 64 with K % 128 == 0 on the register-dequantized kernel (one, two or
     four MFMA row blocks; K split 4 ways on the 4096 x 14336 down shape; half-used last W
-    lines at K = 1152 and 640), 64 x 128 tiles below M = 128 otherwise, 128 x 128 above;
-    split K, odd K steps."""
+    lines at K = 1152 and 640), k_htile_f3's 64- and 128-row tiles otherwise; split K, odd
+    K steps."""
     torch = torch_cuda()
     print(f"f32 prefill M={M} N={N} K={K}", flush=True)
     hole, plug, am = _encoded_weight(oracle, N, K, 3200 + M)

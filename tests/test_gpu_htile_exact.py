@@ -12,7 +12,7 @@ import pytest
 
 from glint_amd import glint_hip as H
 from oracle import glint_oracle as G
-from tests.gpu_util import dev, host
+from tests.gpu_util import dev, host, torch_cuda
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +61,22 @@ def test_subnormal_x_under_large_scales(oracle, M, N, K, bs):
     up = np.maximum(x & 0x7FFF, 0x0080).astype(np.uint16)
     _, asum = (a.reshape(M, N) for a in oracle.htile_f64(hole, plug, am, up, M, N, K, bs))
     assert (np.abs(y - ref) <= (K + 2) * 2.0 ** -23 * asum).all()
+
+
+@pytest.mark.parametrize("N", [70, 8200])
+def test_single_products_m1_tiles(N):
+    """M = 1 beyond the GEMV's K: 64 x 64 tiles, and 64 x 128 ones where those fill the CUs; k at the
+    ends of a 64-wide step, of a K split and between."""
+    torch = torch_cuda()
+    K = 32832
+    print(f"htile single products M=1 N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    hole, plug = (torch.randint(0, 256, (N * K // 2,), dtype=torch.uint8, device="cuda", generator=g) for _ in range(2))
+    am = torch.rand(N * K // 64, device="cuda", generator=g) + 0.01
+    for k in (0, 1, 31, 32, 63, 64, 8191, 8192, 8255, 8256, 16448, 20000, 24639, 32767, 32768, 32831):
+        x = torch.zeros(K, dtype=torch.bfloat16, device="cuda")
+        x[k] = 1.0
+        i = torch.arange(N, device="cuda") * K + k
+        h, p = (((t[i >> 1] >> (4 * (k & 1))) & 15).cpu().numpy() for t in (hole, plug))
+        want = G.CELLS_F32[h, p] * am[i // 64].cpu().numpy()
+        assert np.array_equal(host(H.htile_f32(hole, plug, am, x, N, K, 64)).reshape(-1), want), k
