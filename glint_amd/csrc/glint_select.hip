@@ -6,7 +6,7 @@
  * k_kmajor_pack_planes — 64 rows x 64 channels per workgroup through LDS: 8-byte loads of
  *   the row-major planes, 4-byte stores of the K-major rows.
  * k_gemv_km_fold_part — the fold at 8 to 64 channels per wave, every load in flight at once.
- * k_gemv_km_fold — longer parts: a lane owns KM_FOLD_RPL = 8 output rows (4 B of a K-major hole row), so
+ * k_gemv_km_fold — longer parts: a lane owns KM_RPL = 8 output rows (4 B of a K-major hole row), so
  *   a wave reads 256 B contiguous per channel; the 8 waves of a workgroup take 8 parts of the
  *   workgroup's channel slice (grid.y) and meet in LDS; the slices of a row block meet in
  *   the last of its workgroups to finish (arrival counters), in slice order. Per element:
@@ -97,9 +97,7 @@ __global__ __launch_bounds__(KM_T) void k_kmajor_scales(const float *__restrict_
 #define KM_U 4 /* channels per batch (two batches in flight per wave); a multiple of 4 dividing 64 */
 #endif
 static_assert(KM_U % 4 == 0 && 64 % KM_U == 0, "fold batch");
-#ifndef KM_FOLD_RPL
-#define KM_FOLD_RPL 8 /* fold: output rows per lane (8, 16 or 32) */
-#endif
+#define KM_RPL 8 /* output rows per lane of the folds and the correction: one word of a K-major row */
 
 __device__ __forceinline__ float km_bf16(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 
@@ -214,17 +212,12 @@ __device__ __forceinline__ void km_finish(float *lds, const float (&tot)[RPL], i
 /* Workgroup (row block bx, channel slice by): wave q walks part q of the slice as runs of
  * channels inside one 64-block; out[by N + r] (y when there is one slice) = the slice's
  * sum for row r. N % 32 == 0; rows of lanes past N are clamped and not stored. */
-template <int RPL>
-__global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint8_t *__restrict__ hole_bytes,
+__global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint32_t *__restrict__ hole_k,
                                                         const float *__restrict__ scales_k,
                                                         const uint16_t *__restrict__ x, float *__restrict__ y,
                                                         float *__restrict__ part, unsigned *ctr, int N, int ksl) {
-    constexpr int ROWS = 64 * RPL, NW = RPL / 8; /* rows per workgroup, code words per lane */
-    using HV = typename std::conditional<RPL == 32, glint_u32x4,
-                                         typename std::conditional<RPL == 16, glint_u32x2, uint32_t>::type>::type;
-    static_assert(RPL == 8 || RPL == 16 || RPL == 32, "rows per lane");
+    constexpr int RPL = KM_RPL, ROWS = 64 * RPL; /* rows per workgroup */
     static_assert(KM_SUB * ROWS >= 16 * 64, "PARENT table fits the part buffer");
-    const HV *__restrict__ hole_k = (const HV *)hole_bytes;
     __shared__ __attribute__((aligned(16))) float lds[KM_SUB * ROWS]; /* PARENT table at offset 0, then parts */
     for (int i = threadIdx.x; i < 16 * 64; i += KM_WG)
         lds[i] = kParent[i >> 6];
@@ -233,7 +226,7 @@ __global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint8_t *__restric
     const uint32_t lane4 = (uint32_t)lane * 4u;
     const int r0 = blockIdx.x * ROWS;
     const int rc = min(r0 + RPL * lane, N - RPL); /* this lane's first row, clamped */
-    const int64_t rowv = N / RPL;                 /* RPL / 2-byte vectors per K-major row */
+    const int64_t rowv = N / RPL;                 /* words per K-major row */
     const int sub = ksl / KM_SUB;
     const int c0 = blockIdx.y * ksl + q * sub, c1 = c0 + sub;
     float tot[RPL], acc[RPL], sc[RPL];
@@ -244,14 +237,14 @@ __global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint8_t *__restric
      * KM_U and blocks multiples of 64), the next batch's loads in flight while this one is
      * looked up. A run is the batches of one block: acc restarts at its first batch and is
      * folded into tot by the block scale after its last, in channel order. */
-    auto load_batch = [&](int c, HV (&wv)[KM_U]) {
+    auto load_batch = [&](int c, uint32_t (&wv)[KM_U]) {
         c = min(c, c1 - KM_U); /* past the part: a clamped reload nobody uses */
 #pragma unroll
         for (int u = 0; u < KM_U; ++u)
             wv[u] = __builtin_nontemporal_load(&hole_k[(int64_t)(c + u) * rowv + rc / RPL]);
     };
-    HV wa[KM_U], wb[KM_U];
-    auto batch = [&](int c, const HV (&wv)[KM_U]) {
+    uint32_t wa[KM_U], wb[KM_U];
+    auto batch = [&](int c, const uint32_t (&wv)[KM_U]) {
         if (c == c0 || (c & 63) == 0) { /* a run starts: its block scales, acc from zero */
             km_load<RPL>(scales_k + (int64_t)(c >> 6) * N + rc, sc);
 #pragma unroll
@@ -270,14 +263,7 @@ __global__ __launch_bounds__(KM_WG) void k_gemv_km_fold(const uint8_t *__restric
 #pragma unroll
         for (int u = 0; u < KM_U; ++u) {
             const float xv = (u & 1) ? glint_bf16hi(xs[u >> 1]) : glint_bf16lo(xs[u >> 1]);
-            uint32_t W[NW];
-            __builtin_memcpy(W, &wv[u], sizeof(W));
-            uint32_t E[NW], O[NW];
-#pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                E[q] = W[q] & 0x0F0F0F0Fu;
-                O[q] = (W[q] >> 4) & 0x0F0F0F0Fu;
-            }
+            const uint32_t E[1] = {wv[u] & 0x0F0F0F0Fu}, O[1] = {(wv[u] >> 4) & 0x0F0F0F0Fu};
             km_lookup_fma<RPL>(lds, E, O, lane4, xv, acc);
         }
         if (c + KM_U == c1 || ((c + KM_U) & 63) == 0) { /* the run ends */
@@ -316,7 +302,7 @@ __global__ __launch_bounds__(KM_WG) void k_gemv_km_fold_part(const uint32_t *__r
                                                              const float *__restrict__ scales_k,
                                                              const uint16_t *__restrict__ x, float *__restrict__ y,
                                                              float *__restrict__ part, unsigned *ctr, int N) {
-    constexpr int RPL = 8, ROWS = 64 * RPL;
+    constexpr int RPL = KM_RPL, ROWS = 64 * RPL;
     constexpr bool SPLIT = 64 % SUB != 0;
     static_assert(SUB % 8 == 0 && SUB <= 64, "a part");
     __shared__ __attribute__((aligned(16))) float lds[256 * 32 * 2]; /* PARENT pairs, then parts */
@@ -603,7 +589,7 @@ __global__ __launch_bounds__(KM_WG) void k_apply_corr_km(const uint32_t *__restr
                                                          const uint16_t *__restrict__ x, const int32_t *__restrict__ idx,
                                                          const int32_t *__restrict__ cnt, float *__restrict__ y,
                                                          float *__restrict__ part, unsigned *ctr, int N, int ks) {
-    constexpr int RPL = 8, ROWS = 64 * RPL;
+    constexpr int RPL = KM_RPL, ROWS = 64 * RPL;
     static_assert(KM_SUB * ROWS <= GLINT_LDS_CELLS64_WORDS, "parts fit the table's LDS");
     __shared__ __attribute__((aligned(16))) float lds[GLINT_LDS_CELLS64_WORDS]; /* delta table, then parts */
     const int lane = threadIdx.x & 63, q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -757,7 +743,7 @@ GLINT_API int glint_gemv_km_fold(const uint8_t *hole_k, const float *scales_k, c
     if (N < 32 || (N % 32) != 0 || ksg < 1 || K < 64 || (K % (64 * ksg)) != 0 || !glint_aligned(hole_k, 16) ||
         !glint_aligned(scales_k, 16) || !glint_aligned(x, 16))
         return -2;
-    static_assert(KM_FOLD_RPL == 8, "both folds take 512 rows per workgroup");
+    static_assert(KM_RPL == 8, "a workgroup takes 512 rows");
     const dim3 grid((N + 511) / 512, ksg);
     unsigned *ctr = ksg > 1 ? km_counters(stream, grid.x) : nullptr;
     auto parts = [&](auto sub_c) {
@@ -774,7 +760,7 @@ GLINT_API int glint_gemv_km_fold(const uint8_t *hole_k, const float *scales_k, c
     case 56: parts(std::integral_constant<int, 56>{}); break;
     case 64: parts(std::integral_constant<int, 64>{}); break;
     default:
-        k_gemv_km_fold<KM_FOLD_RPL><<<grid, KM_WG, 0, stream>>>(hole_k, scales_k, x, y, part, ctr, N, K / ksg);
+        k_gemv_km_fold<<<grid, KM_WG, 0, stream>>>((const uint32_t *)hole_k, scales_k, x, y, part, ctr, N, K / ksg);
     }
     if (ksg > 1 && !ctr)
         k_km_combine<false><<<(N + KM_T - 1) / KM_T, KM_T, 0, stream>>>(part, y, N, ksg);
