@@ -1059,7 +1059,36 @@ def counter_workload(torch, H, manifest_path):
         phase(name, key, 6, lambda: [c() for c in calls], ops=6 * 2.0 * M * N * K,
               nbytes=6 * (N * K * (1 + 4 / 64) + 2 * M * K + 2 * M * N))
         del xm, ym
-    del pins
+    # f32 out on the same shape: a batch of 8 and the prefill
+    for M, key, name in ((8, "k_htile_rl3<1>", "f32_m8_14336x4096"),
+                         (2048, "k_htile_f3<8,false>", "f32_m2048_14336x4096")):
+        xm = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+        ym = torch.empty(M, N, dtype=torch.float32, device="cuda")
+        calls = [bound(lib.launch_glint_htile_s3_f32_stream, p[0], p[1], p[2], xm, ym, M, N, K, 64, st) for p in pins]
+        phase(name, key, 6, lambda: [c() for c in calls], ops=6 * 2.0 * M * N * K,
+              nbytes=6 * (N * K * (1 + 4 / 64) + 2 * M * K + 4 * M * N), note="three BF16 planes per cell: 3x ops on MFMA")
+        del xm, ym
+    # the K-major step's fold and correction (16 slices of 32 channels per wave; a tenth of the channels)
+    kms = [H.kmajor_pack(*p, N, K) for p in pins]
+    xk = torch.randn(K, device="cuda", generator=g).to(torch.bfloat16)
+    yk, part = torch.empty(N, device="cuda"), torch.empty(16 * N, device="cuda")
+    idx, cnt = H.select_topk(xk, 409)
+    phase("kmajor_fold_14336x4096", "k_gemv_km_fold_part<32>", 6,
+          lambda: [H.gemv_km_fold(k[0], k[2], xk, N, K, 16, yk, part) for k in kms],
+          nbytes=6 * (N * K * (0.5 + 4 / 64) + 2 * K + 4 * N))
+    phase("kmajor_correction_14336x4096_409", "k_apply_corr_km", 6,
+          lambda: [H.apply_corr_km(*k, xk, idx, cnt, yk, N, K, 8, part) for k in kms],
+          nbytes=6 * (N * 409 * 1.0 + N * K * 4 / 64 + 8 * N), note="bytes: 409 rows of both planes and every block's scales")
+    del pins, kms
+    # a linear whose rows are no whole number of blocks
+    No, Ko, Mo = 3001, 4104, 17
+    podd = [encode_pin((torch.randn(No * Ko, device="cuda", generator=g) * 0.02).to(torch.bfloat16)) for _ in range(6)]
+    xo = torch.randn(Mo, Ko, device="cuda", generator=g).to(torch.bfloat16)
+    yo = torch.empty(Mo, No, dtype=torch.float32, device="cuda")
+    calls = [bound(lib.launch_glint_htile_s3_f32_stream, p[0], p[1], p[2], xo, yo, Mo, No, Ko, 64, st) for p in podd]
+    phase("f32_any_17x3001x4104", "k_htile_any<2,1,false,false,TileOutF32>", 6, lambda: [c() for c in calls],
+          ops=6 * 2.0 * Mo * No * Ko, nbytes=6 * (No * Ko * (1 + 4 / 64) + 2 * Mo * Ko + 4 * Mo * No))
+    del podd, xo, yo
     # INT8 GEMM at the INT8 config: the raw per-row / per-column GEMM and the attach ABI
     M, N8, K8 = 2048, 8192, 8192
     A = torch.randint(-127, 128, (M, K8), device="cuda", generator=g, dtype=torch.int8)
@@ -1080,7 +1109,7 @@ def counter_workload(torch, H, manifest_path):
     lin = H.Int8MmaLinear(q.data_ptr(), sc.data_ptr(), N8, K8)
     call = bound(p7.int8_mma_gemm, xb, lin, yf, M, xq, sx, st)
     phase("int8_mma_gemm_abi_2048x8192x8192", "k_int8_mma_dma", 4, lambda: [call() for _ in range(4)],
-          ops=4 * 2.0 * M * N8 * K8, note="per-64 scales, kb-ordered f32 epilogue, last step fused")
+          ops=4 * 2.0 * M * N8 * K8, note="per-64 scales, kb-ordered f32 epilogue without the convert")
     Path(manifest_path).write_text(json.dumps({"phases": phases, "cu_num": CU_NUM, "simd_num": SIMD_NUM}, indent=1) + "\n")
 
 
@@ -1184,6 +1213,8 @@ def load_counters():
             "gemv_m1_14336x4096": ("hbm_frac", "traffic_over_algorithmic", "VALUBusy"),
             "prefill_m2048_14336x4096": ("mfma_frac", "MfmaUtil", "LDSBankConflict", "lds_active_pct"),
             "prefill_m64_14336x4096": ("hbm_frac", "mfma_frac", "MfmaUtil", "LDSBankConflict", "lds_active_pct"),
+            "f32_m8_14336x4096": ("hbm_frac", "VALUBusy", "MfmaUtil", "lds_active_pct"),
+            "f32_m2048_14336x4096": ("mfma_frac", "VALUBusy", "MfmaUtil", "lds_active_pct"),
             "int8_gemm_2048x8192x8192": ("mfma_frac", "MfmaUtil"),
             "int8_mma_gemm_abi_2048x8192x8192": ("mfma_frac", "MfmaUtil", "VALUBusy")}
     return {k: {f: round(c[k][f], 4) for f in fs if f in c[k]} for k, fs in pick.items() if k in c}
