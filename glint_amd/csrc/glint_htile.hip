@@ -770,7 +770,9 @@ __global__ __launch_bounds__(MAXT) void k_htile_gemv_mr(const void *__restrict__
 #endif
 #ifndef GEMV_MR_RL_F32_WEIGHTS
 /* f32 out, M = 5 and 6: fewer weights than this take the two small-M launches (1024 x 4096 M = 5
- * 8.8 us against 9.2; 4096 x 4096 12.9 against 10.1). M = 7 and 8 always took k_htile_rl's form. */
+ * 8.8 us against 9.2; 4096 x 4096 12.9 against 10.1). M = 7 and 8 take k_htile_rl3 always. With
+ * that M = 4 .. 64 is nowhere slower than the per-weight form and the two launches before it were
+ * (9 M on 11 matrices from 512 x 512 to 14336 x 4096 and 512 x 14336, within 1%). */
 #define GEMV_MR_RL_F32_WEIGHTS (1 << 23)
 #endif
 #ifndef GEMV_MR_MAX_F32
@@ -2189,7 +2191,10 @@ __global__ __launch_bounds__(512, 1) void k_htile_f3(const uint8_t *__restrict__
  * and the meeting of a K split, 6 and 4 us. Fitted on both tiles measured at 300 x 5000 x 1024
  * (128 rows split twice 21.1 us, 64 rows unsplit 15.3), 512 x 2048 x 2048 (21.4, 20.1),
  * 96 x 4096 x 4096 (27.3, 18.6), 256 x 4096 x 4096 (31.2, 31.7), 128 x 14336 x 4096 (49.6, 53.1)
- * and 200 x 4096 x 14336 (79.2, 91.1): it picks the faster one at each. */
+ * and 200 x 4096 x 14336 (79.2, 91.1): it picks the faster one at each. Over 12 M from 65 to 2047
+ * on 13 matrices from 512 x 512 to 14336 x 4096, both tiles timed, it picks the faster one (within
+ * 1%) at 142 of 156, loses 0.3% on average and 7.6% at worst (160 x 4096 x 4096: 128 rows 30.7 us,
+ * 64 rows 28.5); 64 rows everywhere would lose 5% on average, 128 rows 21%. */
 static inline int64_t f3_cost(int mb, int M, int N, int K) {
     const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 16 * mb - 1) / (16 * mb)), cus = glint_cu_count();
     const int nc = (K + 127) >> 7, cps = glint_split_kps(tiles, cus, nc, F3_MIN_CHUNKS);
